@@ -3969,15 +3969,55 @@ __global__ void __launch_bounds__(kSvWaves * kWave)
 }
 
 // ---------------------------------------------------------------------------
+// A hybrid cache's buffered tokens for the merge launch: element j of token t
+// of (b, h) at buf[b*sb + h*sh + t*st + j], original basis, positions t_kv + t.
+// vec: every row is 16-byte aligned.
+struct MergeBuffer {
+    const void *k, *v;
+    int dtype, vec;
+    int64_t sb, sh, st, n;
+};
+
+// Eight consecutive elements at p (element index i) as float32.
+__device__ __forceinline__ void load8_f32(const void *p, int dtype, int vec, int64_t i, float (&x)[8]) {
+    if (vec && dtype != SS_F32) {
+        const uint4 u = *reinterpret_cast<const uint4 *>(static_cast<const char *>(p) + i * 2);
+        if (dtype == SS_F16)
+            unpack16<__half>(u, x);
+        else
+            unpack16<__hip_bfloat16>(u, x);
+    } else if (vec) {
+        const uint4 *u = reinterpret_cast<const uint4 *>(static_cast<const char *>(p) + i * 4);
+        unpack16<float>(u[0], x);
+        unpack16<float>(u[1], x + 4);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = load_as_f32(p, dtype, i + e);
+    }
+}
+
 // Merge of split-T partials: one workgroup per (group, row).  One wave turns
 // the splits' (m, l) into weights exp2(m_s - M) and the merged l; every thread
 // then streams float4 slices of the accumulators of a subset of splits (loads
 // issued back to back) and the slices are reduced in LDS.  Runs as its own
 // launch: a cross-workgroup hand-off inside one kernel needs an agent-scope L2
 // write-back per workgroup on multi-XCD CDNA parts.
-template <int D>
+//
+// BUF: a hybrid cache's buffered tokens (at positions t_kv ..) join here (the
+// reference runs its two-pass path instead, attention.py:307-350): the
+// workgroup attends them for its row with fp32 dot products against the
+// unpermuted scaled query, 128 tokens at a time, before it reads the splits'
+// partials, and their accumulator is added after the rotation, in the
+// original basis.  Latency bounds it: D/8 lanes share a token (16-byte loads
+// of 16-bit rows) and a chunk's key and value rows are requested together.
+// One slot of the partials stays reserved for the buffer and is not read.
+// As a launch of its own, one workgroup per column with a token per thread
+// and element loads, the buffer took 85 us at 32 columns (B = 4, 128 tokens)
+// and 105 us at 128; the merge with it takes 14.8 and 18.4 us (5.5 without).
+template <int D, bool BUF>
 __global__ void __launch_bounds__(kDecodeThreads)
-    decode_merge_kernel(DecodeCommon c, int R, const float *rot, void *rot_out, int rot_dtype) {
+    decode_merge_kernel(DecodeCommon c, int R, const float *rot, void *rot_out, int rot_dtype,
+                        MergeBuffer mb) {
     constexpr int CH = D / 4;                // float4 chunks of one output row
     constexpr int NP = kDecodeThreads / CH;  // split partitions
     __shared__ float wsh[kMaxSplits];
@@ -3988,12 +4028,78 @@ __global__ void __launch_bounds__(kDecodeThreads)
     const int col = blockIdx.x, r = blockIdx.y;
     const int64_t gr = (int64_t)(col % c.n_rg) * R + r;
     if (gr >= c.rows_total) return;  // uniform over the workgroup
-    const int S = c.n_splits;
+    const int S = c.n_splits - (BUF ? 1 : 0), SS = c.n_splits;
     const int kvh = (col / c.n_rg) % c.n_kv_heads;
     const int64_t bb = col / (c.n_rg * c.n_kv_heads);
-    const float *ml = c.part_ml + ((int64_t)col * S * R + r) * 2;
+    const int64_t rr = gr / c.t_q, tq = gr - rr * c.t_q;
+    const int64_t off = ((bb * c.n_q_heads + kvh * c.rep + rr) * c.t_q + tq) * D;
+    // buffered tokens: running maximum and sum (same in every thread), and
+    // the row's accumulator in LDS
+    constexpr int LPT = D / 8;                    // lanes per token
+    constexpr int TPG = kDecodeThreads / LPT;     // tokens per pass of the workgroup
+    constexpr int BT = 128, PASSES = BT / TPG;    // tokens of a chunk
+    __shared__ float bp[BUF ? BT : 1];
+    __shared__ float bacc[BUF ? kDecodeThreads / kWave : 1][BUF ? D : 1];
+    float bm = -1e30f, bl = 0.f;
+    if constexpr (BUF) {
+        const int dl = tid % LPT, tg = tid / LPT;  // dims 8*dl .. +7 of tokens tg + i*TPG
+        float qv[8], ba[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            qv[e] = round_to(c.q_dtype, load_as_f32(c.q, c.q_dtype, off + dl * 8 + e) * c.scale) * kLog2e;
+            ba[e] = 0.f;
+        }
+        // tokens of the buffer this row sees
+        const int64_t lim = c.causal ? c.q_offset + tq - c.t_kv + 1 : mb.n;
+        const int64_t n = min(mb.n, lim);
+        const int64_t base = bb * mb.sb + kvh * mb.sh + dl * 8;
+        for (int64_t j0 = 0; j0 < n; j0 += BT) {
+            float kx[PASSES][8], vx[PASSES][8];
+#pragma unroll
+            for (int i = 0; i < PASSES; ++i) {
+                const int64_t j = min(j0 + tg + i * TPG, n - 1);
+                load8_f32(mb.k, mb.dtype, mb.vec, base + j * mb.st, kx[i]);
+                load8_f32(mb.v, mb.dtype, mb.vec, base + j * mb.st, vx[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < PASSES; ++i) {
+                float a = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) a = fmaf(qv[e], kx[i][e], a);
+#pragma unroll
+                for (int o = LPT / 2; o > 0; o >>= 1) a += __shfl_xor(a, o);
+                const int tl = tg + i * TPG;
+                if (dl == 0) bp[tl] = j0 + tl < n ? a : -INFINITY;
+            }
+            __syncthreads();
+            float mx = wave_max(fmaxf(bp[lane], bp[lane + kWave]));
+            const float mn = fmaxf(bm, mx), corr = fast_exp2(bm - mn);
+            bm = mn;
+            bl = fmaf(bl, corr, wave_sum(fast_exp2(bp[lane] - mn) + fast_exp2(bp[lane + kWave] - mn)));
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ba[e] *= corr;
+#pragma unroll
+            for (int i = 0; i < PASSES; ++i) {
+                const float p = fast_exp2(bp[tg + i * TPG] - mn);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) ba[e] = fmaf(p, vx[i][e], ba[e]);
+            }
+            __syncthreads();  // bp is written again by the next chunk
+        }
+        // the wave's token groups, then (below) its row in LDS
+#pragma unroll
+        for (int o = LPT; o < kWave; o <<= 1)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ba[e] += __shfl_xor(ba[e], o);
+        if (lane < LPT)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) bacc[wv][dl * 8 + e] = ba[e];
+    }
+    const float *ml = c.part_ml + ((int64_t)col * SS * R + r) * 2;
+    float bw = 0.f;  // the buffer's weight (wave 0 sets it below)
+    __shared__ float bwsh;
     if (wv == 0) {
-        float M = -1e30f;
+        float M = bm;
         for (int s2 = lane; s2 < S; s2 += kWave) M = fmaxf(M, ml[(int64_t)s2 * R * 2]);
         M = wave_max(M);
         float L = 0.f;
@@ -4004,13 +4110,28 @@ __global__ void __launch_bounds__(kDecodeThreads)
             L = fmaf(v.y, w, L);
         }
         L = wave_sum(L);
+        if constexpr (BUF) {
+            bw = fast_exp2(bm - M);
+            L = fmaf(bl, bw, L);
+            if (lane == 0) bwsh = bw;
+        }
         if (lane == 0) lsh = L;
     }
     __syncthreads();
+    // the buffered tokens' part of output dim d
+    auto buffered = [&](int d) {
+        float a = 0.f;
+        if constexpr (BUF) {
+#pragma unroll
+            for (int w = 0; w < kDecodeThreads / kWave; ++w) a += bacc[w][d];
+            a = lsh > 0.f ? a * bwsh / lsh : 0.f;
+        }
+        return a;
+    };
     {
         const int chunk = tid % CH, part = tid / CH;
         const float4 *ap =
-            reinterpret_cast<const float4 *>(c.part_acc + ((int64_t)col * S * R + r) * D) + chunk;
+            reinterpret_cast<const float4 *>(c.part_acc + ((int64_t)col * SS * R + r) * D) + chunk;
         float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll 8
         for (int s2 = part; s2 < S; s2 += NP) {
@@ -4032,13 +4153,11 @@ __global__ void __launch_bounds__(kDecodeThreads)
             const float4 v = red[p * CH + chunk];
             A += (d & 3) == 0 ? v.x : (d & 3) == 1 ? v.y : (d & 3) == 2 ? v.z : v.w;
         }
-        const int64_t rr = gr / c.t_q, tq = gr - rr * c.t_q;
-        const int64_t off = ((bb * c.n_q_heads + kvh * c.rep + rr) * c.t_q + tq) * D;
         const float y = lsh > 0.f ? A / lsh : 0.f;
         if (rot)
             yrow[d] = y;
         else
-            store_from_f32(c.out, c.out_dtype, off + d, y);
+            store_from_f32(c.out, c.out_dtype, off + d, y + buffered(d));
     }
     if (rot) {
         // the merged row is in a transformed basis (TurboQuant rotation, a
@@ -4061,12 +4180,10 @@ __global__ void __launch_bounds__(kDecodeThreads)
         }
         __syncthreads();
         if (tid < D) {
-            const int64_t rr = gr / c.t_q, tq = gr - rr * c.t_q;
-            const int64_t off = ((bb * c.n_q_heads + kvh * c.rep + rr) * c.t_q + tq) * D;
             float a = 0.f;
 #pragma unroll
             for (int pp = 0; pp < PARTS; ++pp) a += rsum[pp][tid];
-            store_from_f32(rot_out, rot_dtype, off + tid, a);
+            store_from_f32(rot_out, rot_dtype, off + tid, a + buffered(tid));
         }
     }
 }
@@ -4102,145 +4219,6 @@ __global__ void __launch_bounds__(256)
     for (int j = 0; j < RPT; ++j) {
         const int64_t r = r0 + part * RPT + j;
         if (r < rows) store_from_f32(out, out_dtype, r * D + d, acc[j]);
-    }
-}
-
-// A hybrid cache's buffered tokens (original basis, element j of token t of
-// (b, h) at buf[b*sb + h*sh + t*st + j]) as split partial `slot` of the
-// TurboQuant decode, so they join the compressed tokens' softmax in the merge
-// (the reference runs its two-pass path instead, attention.py:307-350).  One
-// workgroup per column.  Scores are fp32 dot products with the unpermuted
-// scaled query, in log2 units, at positions t_kv + t; online softmax over
-// chunks of 256 tokens; P.V in the original basis.  The accumulators are then
-// taken into the rotated basis, acc @ R^T (R orthogonal), where the merge
-// adds them to the compressed splits' before the output rotation; with no
-// R (rot null: values in the original basis) they are stored as they are.
-template <int D, int R>
-__global__ void __launch_bounds__(256)
-    buffer_partial_kernel(DecodeCommon c, const void *kbuf, const void *vbuf, int buf_dtype,
-                          int64_t sb, int64_t sh, int64_t st, int64_t t_buf, const float *rot,
-                          int slot) {
-    constexpr int T = 256, NW = T / kWave;
-    __shared__ float qs[R][D];
-    __shared__ float pr[R][T];
-    __shared__ float red[NW][R];
-    __shared__ float acc_s[R][D];
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid >> 6;
-    const int col = blockIdx.x;
-    const int rg = col % c.n_rg;
-    const int kvh = (col / c.n_rg) % c.n_kv_heads;
-    const int64_t bb = col / (c.n_rg * c.n_kv_heads);
-    auto row_ok = [&](int r) { return (int64_t)rg * R + r < c.rows_total; };
-    auto row_off = [&](int r) -> int64_t {
-        const int64_t g = (int64_t)rg * R + r;
-        const int64_t rr = g / c.t_q, tq = g - rr * c.t_q;
-        return ((bb * c.n_q_heads + kvh * c.rep + rr) * c.t_q + tq) * D;
-    };
-    for (int i = tid; i < R * D; i += T) {
-        const int r = i / D, j = i - r * D;
-        qs[r][j] = row_ok(r) ? round_to(c.q_dtype, load_as_f32(c.q, c.q_dtype, row_off(r) + j) *
-                                                        c.scale)
-                             : 0.f;
-    }
-    int64_t lim[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int64_t g = (int64_t)rg * R + r;
-        lim[r] = !row_ok(r) ? -1 : c.causal ? c.q_offset + (g % c.t_q) : INT64_MAX;
-    }
-    const int64_t base = bb * sb + kvh * sh;
-    // thread (r, d) of the P.V: rows r = tid / D + k * (T / D)
-    constexpr int RPT = (R * D + T - 1) / T;
-    float m[R], l[R], acc[RPT];
-#pragma unroll
-    for (int r = 0; r < R; ++r) m[r] = -1e30f, l[r] = 0.f;
-#pragma unroll
-    for (int k = 0; k < RPT; ++k) acc[k] = 0.f;
-    __syncthreads();
-    for (int64_t j0 = 0; j0 < t_buf; j0 += T) {
-        const int64_t j = j0 + tid;
-        float s[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) s[r] = 0.f;
-        if (j < t_buf) {
-            for (int d = 0; d < D; ++d) {
-                const float kv = load_as_f32(kbuf, buf_dtype, base + j * st + d);
-#pragma unroll
-                for (int r = 0; r < R; ++r) s[r] = fmaf(qs[r][d], kv, s[r]);
-            }
-        }
-        float cm[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const bool ok = j < t_buf && c.t_kv + j <= lim[r];
-            s[r] = ok ? s[r] * kLog2e : -INFINITY;
-            cm[r] = wave_max(s[r]);
-        }
-        if (lane == 0)
-#pragma unroll
-            for (int r = 0; r < R; ++r) red[wv][r] = cm[r];
-        __syncthreads();
-        float corr[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            float mx = red[0][r];
-#pragma unroll
-            for (int w = 1; w < NW; ++w) mx = fmaxf(mx, red[w][r]);
-            const float mn = fmaxf(m[r], mx);
-            corr[r] = fast_exp2(m[r] - mn);
-            m[r] = mn;
-            pr[r][tid] = fast_exp2(s[r] - mn);
-        }
-        __syncthreads();  // probabilities staged; red free
-        float ps[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) ps[r] = wave_sum(pr[r][tid]);
-        if (lane == 0)
-#pragma unroll
-            for (int r = 0; r < R; ++r) red[wv][r] = ps[r];
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            float sum = 0.f;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) sum += red[w][r];
-            l[r] = fmaf(l[r], corr[r], sum);
-        }
-        const int n = (int)min((int64_t)T, t_buf - j0);
-#pragma unroll
-        for (int k = 0; k < RPT; ++k) {
-            const int e = tid + k * T;
-            if (e < R * D) {
-                const int r = e / D, d = e - r * D;
-                float a = acc[k] * corr[r];
-                for (int i = 0; i < n; ++i)
-                    a = fmaf(pr[r][i], load_as_f32(vbuf, buf_dtype, base + (j0 + i) * st + d), a);
-                acc[k] = a;
-            }
-        }
-        __syncthreads();  // pr and red reused by the next chunk
-    }
-#pragma unroll
-    for (int k = 0; k < RPT; ++k) {
-        const int e = tid + k * T;
-        if (e < R * D) acc_s[e / D][e % D] = acc[k];
-    }
-    __syncthreads();
-    const int64_t slot0 = ((int64_t)col * c.n_splits + slot) * R;
-#pragma unroll
-    for (int k = 0; k < RPT; ++k) {
-        const int e = tid + k * T;
-        if (e < R * D) {
-            const int r = e / D, kk = e - r * D;
-            float a = 0.f;
-            if (rot)
-                for (int d = 0; d < D; ++d) a = fmaf(acc_s[r][d], rot[kk * D + d], a);
-            else
-                a = acc_s[r][kk];
-            c.part_acc[(slot0 + r) * D + kk] = a;
-            if (kk == 0)
-                *reinterpret_cast<float2 *>(c.part_ml + (slot0 + r) * 2) = make_float2(m[r], l[r]);
-        }
     }
 }
 
@@ -4319,11 +4297,12 @@ static size_t decode_ws_bytes(const DecodeShape &s, int head_dim) {
 
 template <int D>
 static int launch_merge(const DecodeCommon &c, const DecodeShape &s, hipStream_t st,
-                        const float *rot = nullptr, void *rot_out = nullptr, int rot_dtype = 0) {
+                        const float *rot = nullptr, void *rot_out = nullptr, int rot_dtype = 0,
+                        const MergeBuffer &mb = MergeBuffer{}) {
     if (s.S <= 1) return SS_OK;
-    auto merge = decode_merge_kernel<D>;
+    auto merge = mb.n > 0 ? decode_merge_kernel<D, true> : decode_merge_kernel<D, false>;
     hipLaunchKernelGGL(merge, dim3(s.n_cols, s.R), dim3(kDecodeThreads), 0, st, c, s.R, rot,
-                       rot_out, rot_dtype);
+                       rot_out, rot_dtype, mb);
     SS_LAUNCH_CHECK("decode_merge_kernel launch");
     return SS_OK;
 }
@@ -4771,9 +4750,9 @@ extern "C" size_t ss_decode_turboquant_workspace_bytes(int64_t batch, int n_q_he
 // Shared host side of the decodes whose values accumulate in a transformed
 // basis (TurboQuant's rotation, a SunShape value codec's permutation or
 // rotation): the VALU decode writes y (fp32, that basis) or split partials;
-// buffered original-basis tokens become one more partial, taken into that
-// basis with transform^T (orthogonal); the merge launch, or rotate_rows_kernel
-// for a single split, writes out = y @ transform in out_dtype.  A null
+// the merge launch attends buffered original-basis tokens and adds them after
+// the transform; it, or rotate_rows_kernel for a single split without a
+// buffer, writes out = y @ transform in out_dtype.  A null
 // transform is the identity (values in the original basis: the grouped and
 // dense VALU decodes with a hybrid cache's buffer): the kernels and the merge
 // write out directly.
@@ -4816,23 +4795,18 @@ static int transformed_decode(const void *q, int q_dtype, int64_t batch, int hq,
     if (rc) return rc;
     c.tiles_per_split = s.tiles_per_split;  // the compressed tokens' splits: grid s.S
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    rc = launch_main(c, s, st);  // no merge: it follows the buffer's partial
+    rc = launch_main(c, s, st);  // no merge: it follows, with the buffer
     if (rc) return rc;
+    MergeBuffer mb{};
     if (t_buf > 0) {
-#define SS_BUFP(DD, RR)                                                                       \
-    hipLaunchKernelGGL((buffer_partial_kernel<DD, RR>), dim3(sw.n_cols), dim3(256), 0, st, c,   \
-                       k_buf, v_buf, buf_dtype, buf_sb, buf_sh, buf_st, t_buf, transform, s.S)
-        if (head_dim == 128) {
-            if (sw.R == 1) SS_BUFP(128, 1); else SS_BUFP(128, 4);
-        } else {
-            if (sw.R == 1) SS_BUFP(64, 1); else SS_BUFP(64, 4);
-        }
-#undef SS_BUFP
-        SS_LAUNCH_CHECK("buffer_partial_kernel launch");
+        const int64_t es = buf_dtype == SS_F32 ? 4 : 2;
+        const bool vec = (((uintptr_t)k_buf | (uintptr_t)v_buf) % 16) == 0 &&
+                         ((buf_sb | buf_sh | buf_st) * es) % 16 == 0;
+        mb = MergeBuffer{k_buf, v_buf, buf_dtype, vec ? 1 : 0, buf_sb, buf_sh, buf_st, t_buf};
     }
     if (sw.S > 1)
-        return head_dim == 128 ? launch_merge<128>(c, sw, st, transform, out, out_dtype)
-                               : launch_merge<64>(c, sw, st, transform, out, out_dtype);
+        return head_dim == 128 ? launch_merge<128>(c, sw, st, transform, out, out_dtype, mb)
+                               : launch_merge<64>(c, sw, st, transform, out, out_dtype, mb);
     if (ident) return SS_OK;  // the one split wrote out
     const unsigned blocks = (unsigned)((rows + kRotRows - 1) / kRotRows);
     if (head_dim == 128)
