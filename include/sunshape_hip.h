@@ -470,8 +470,8 @@ int ss_decode_attn_grouped(const void *q, int q_dtype, int64_t batch, int n_q_he
  * recent-token buffer (k_buf / v_buf, buf_dtype SS_F16 / SS_BF16 / SS_F32,
  * element j of token t of (b, h) at b*buf_sb + h*buf_sh + t*buf_st + j,
  * original basis) joins the same softmax as positions t_kv .. t_kv + t_buf - 1
- * (one more split partial: fp32 dot products with the unpermuted scaled
- * query, online softmax over 256-token chunks).  The reference runs its
+ * (attended by the split-merge launch: fp32 dot products with the unpermuted
+ * scaled query, online softmax over 128-token chunks).  The reference runs its
  * two-pass path whenever the buffer holds tokens (attention.py:238,
  * 307-350).  Workspace: ss_decode_turboquant_workspace_bytes(..., t_buf, ...)
  * bytes, the same layout.
@@ -490,6 +490,23 @@ int ss_decode_attn_dense_hybrid(
     int n_centroids, const uint8_t *idx, const void *values, int v_dtype, int64_t cap,
     int64_t t_kv, const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb,
     int64_t buf_sh, int64_t buf_st, int64_t t_buf, int causal, int64_t q_offset, void *out,
+    int out_dtype, void *workspace, size_t workspace_bytes, int n_splits, void *stream);
+
+/*
+ * ss_decode_attn_dense / _dense_hybrid over bfloat16 values on the matrix
+ * cores: values token-major [batch][n_kv_heads][cap][head_dim] (v_dtype
+ * SS_BF16, 16-byte aligned; others SS_ERR_UNSUPPORTED), the query x centroid
+ * table from the prepared codebook (ss_codebook_f16x2).  Buffer, workspace
+ * and argument conventions of ss_decode_attn_il8_hybrid; t_buf 0: no buffer.
+ * Heavy dims (k_heavy) are not taken (SS_ERR_UNSUPPORTED); pass NULL.
+ */
+int ss_decode_attn_dense_mfma(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
+    int n_centroids, const uint8_t *idx, const void *values, int v_dtype, int64_t cap,
+    int64_t t_kv, const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb,
+    int64_t buf_sh, int64_t buf_st, int64_t t_buf, const void *k_heavy,
+    const int32_t *heavy_dims, int n_heavy_dims, int causal, int64_t q_offset, void *out,
     int out_dtype, void *workspace, size_t workspace_bytes, int n_splits, void *stream);
 
 /*

@@ -93,6 +93,11 @@ _SIGNATURES = {
         _c_void_p, _c_void_p, _int, _i64, _i64,
         _c_void_p, _c_void_p, _int, _i64, _i64, _i64, _i64, _c_void_p, _c_void_p, _int,
         _int, _i64, _c_void_p, _int, _c_void_p, _size, _int, _c_void_p]),
+    "ss_decode_attn_dense_mfma": (_int, [
+        _c_void_p, _int, _i64, _int, _int, _i64, _int, _f32, _c_void_p, _c_void_p, _int, _int,
+        _c_void_p, _c_void_p, _int, _i64, _i64,
+        _c_void_p, _c_void_p, _int, _i64, _i64, _i64, _i64, _c_void_p, _c_void_p, _int,
+        _int, _i64, _c_void_p, _int, _c_void_p, _size, _int, _c_void_p]),
     "ss_decode_step_il8": (_int, [
         _c_void_p, _int, _i64, _int, _int, _i64, _int, _f32, _c_void_p, _c_void_p, _c_void_p,
         _int, _int, _c_void_p, _c_void_p, _i64, _i64,
@@ -494,6 +499,63 @@ class PreparedDecodeBuffered(PreparedDecode):
         if _check_waits:
             check_decode_waits(self.dev)
         return out
+
+
+class PreparedDecodeDense(PreparedDecode):
+    """:class:`PreparedDecode` over token-major bfloat16 values
+    (``ss_decode_attn_dense_mfma``), with a hybrid cache's buffered tokens
+    where the call passes them."""
+
+    __slots__ = ()
+
+    def __call__(self, q: torch.Tensor, t_kv: int, causal: bool = False, q_offset: int = 0,
+                 buf_keys: torch.Tensor | None = None, buf_values: torch.Tensor | None = None,
+                 buf_len: int = 0, out_dtype: torch.dtype | None = None) -> torch.Tensor:
+        if q.shape != self.shape or q.dtype != self.dtype or not q.is_contiguous() or \
+                q.device.index != self.dev:
+            raise ValueError(f"query must be contiguous {self.dtype} {self.shape} on cuda:{self.dev}")
+        if buf_len:
+            buf = _buffer_ptrs(self.shape[0], self.pre[3], self.shape[3], buf_keys, buf_values,
+                               buf_len)
+        else:
+            buf = (None, None, SS_F16, 0, 0, 0, 0)
+        out = torch.empty(self.shape, dtype=out_dtype or self.dtype, device=q.device)
+        _poll_waits(self.dev)
+        st = stream_handle(self.dev)
+        ws = _ws_cache.get((self.dev, st))
+        if ws is None:
+            ws = decode_workspace(self.dev, 1, st)
+        mid = (int(t_kv), *buf, None, None, 0, int(bool(causal)), int(q_offset), out.data_ptr(),
+               dtype_code(out.dtype))
+        rc = self.fn(q.data_ptr(), *self.pre, *mid, ws.data_ptr(), ws.numel(), 0, st)
+        if rc == SS_ERR_WORKSPACE:
+            _, need = decode_plan(KIND_IL8, *self.plan_args, int(t_kv), 0)
+            ws = decode_workspace(self.dev, need, st)
+            rc = self.fn(q.data_ptr(), *self.pre, *mid, ws.data_ptr(), ws.numel(), 0, st)
+        _launched(_attn_stat(self.stat, causal), rc)
+        if _check_waits:
+            check_decode_waits(self.dev)
+        return out
+
+
+def prepare_decode_dense(q: torch.Tensor, scale: float, perm: torch.Tensor | None,
+                         codebook: torch.Tensor, n_blocks: int, n_centroids: int,
+                         idx: torch.Tensor, values: torch.Tensor) -> PreparedDecodeDense:
+    """:class:`PreparedDecodeDense` for queries shaped like ``q`` over the
+    cache buffers ``idx`` / ``values`` (B, Hkv, cap, D) bfloat16."""
+    _check_decode_common(q, idx, None, perm)
+    require_gpu(values, codebook)
+    b_, hq, tq, d = q.shape
+    _, hkv, cap, nb = idx.shape
+    if nb != n_blocks or values.dtype != torch.bfloat16 or not values.is_contiguous() or \
+            tuple(values.shape) != (b_, hkv, cap, d):
+        raise ValueError(f"values must be contiguous bfloat16 {(b_, hkv, cap, d)}")
+    lib = load_library()
+    if codebook.numel() != lib.ss_codebook_f16x2_bytes(n_blocks, n_centroids):
+        raise ValueError("codebook does not match the centroids' shape")
+    pre = (dtype_code(q.dtype), b_, hq, hkv, tq, d, float(scale), ptr(perm), ptr(codebook),
+           nb, n_centroids, ptr(idx), ptr(values), SS_BF16, cap)
+    return PreparedDecodeDense(lib.ss_decode_attn_dense_mfma, pre, q, "sunshape_fused_attention_mfma")
 
 
 MAX_STEP_TOKENS = 4  # new tokens one fused decode step takes (kMaxStepTokens)

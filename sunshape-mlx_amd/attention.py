@@ -58,7 +58,7 @@ def _prepared_decode(cache, ops: dict, codec: SunShapeBlockCodec, q: torch.Tenso
     weak references, so it never keeps a replaced buffer alive)."""
     kind = ops["kind"]
     cb = codec.kernel_codebook()
-    if kind == "il8":
+    if kind in ("il8", "dense"):
         tensors = (ops["idx"], ops["values"], cb)
     else:
         tensors = (ops["idx"], ops["codes_il"], ops["scales"], ops["zeros"], cb)
@@ -77,6 +77,8 @@ def _prepared_decode(cache, ops: dict, codec: SunShapeBlockCodec, q: torch.Tenso
     if kind == "il8":
         plan = _hip.prepare_decode_il8(q, kscale, perm, cb, nb, nc, ops["idx"], ops["values"],
                                        buf_keys=bk)
+    elif kind == "dense":
+        plan = _hip.prepare_decode_dense(q, kscale, perm, cb, nb, nc, ops["idx"], ops["values"])
     else:
         plan = _hip.prepare_decode_grouped_il(q, kscale, perm, cb, nb, nc, ops["idx"],
                                               ops["codes_il"], ops["scales"], ops["zeros"],
@@ -253,8 +255,19 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
             return None
         codec.last_score_backend = "hip_fused_mfma" if kind == "il8" else "hip_fused_mfma_dequant"
         return out
-    # the same with a hybrid cache's buffered tokens (the buffer window
-    # passed per call); rotated codecs hand the kernel rotated buffer copies
+    # token-major bfloat16 values on the matrix cores, with or without
+    # buffered tokens
+    if kind == "dense" and ops["values"].dtype == torch.bfloat16:
+        try:
+            plan = _prepared_decode(cache, ops, codec, q, kscale, perm)
+            out = plan(q, t_kv, causal, q_offset, ops.get("buf_keys"), ops.get("buf_values"),
+                       buffered, out_dtype=out_dtype)
+        except _hip.SunShapeUnsupported:
+            return None
+        codec.last_score_backend = "hip_fused_buffer" if buffered else "hip_fused"
+        return out
+    # il8 and grouped_il with a hybrid cache's buffered tokens (the buffer
+    # window passed per call); rotated codecs hand the kernel rotated buffer copies
     # and take the checked launch below
     if buffered and kind in ("il8", "grouped_il") and hv["k_heavy"] is None and \
             (codec.mode in PERM_MODES or not codec.use_rotation):

@@ -1874,6 +1874,138 @@ struct VTq {
     }
 };
 
+// ds_read_b64_tr_b16 at LDS byte address `addr`: in each 16-lane group, lane j
+// reads 4 halves; lane i receives column i of the 4 x 16 block they form (row
+// r from lane 4r + i/4, element i%4).
+__device__ __forceinline__ f16x4 ds_read_tr16_at(uint32_t addr) {
+    typedef __attribute__((__vector_size__(4 * sizeof(__fp16)))) __fp16 hf16x4;
+    typedef __attribute__((address_space(3))) hf16x4 lhf16x4;
+    return __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4f16((lhf16x4 *)addr));
+}
+
+// bfloat16 values, token-major ([cap][D] per (b, h), the layout a bfloat16
+// cache keeps): P.V on v_mfma_f32_16x16x32_bf16 with B read from the ring by
+// LDS transpose reads (ds_read_b64_tr_b16: 4 tokens of 16 consecutive dims
+// per 16-lane group and read).  A holds p exactly as three bf16 parts (rows
+// 0-3 hi, 4-7 mid, 8-11 lo: 24 bits), so the products are those of float32
+// probabilities; 16 A rows leave room for all three at the cost of one.
+// A token's row is 2D bytes, a multiple of the LDS's 128-byte width, so the
+// four tokens of a transpose read would share banks: the loader copies 32-byte
+// pair c of tile token t to pair position c ^ (t % pairs), which spreads them
+// over distinct banks (the permutation stays inside a row, so the copies stay
+// coalesced).  HBM bounds it, as VIl8.  B=4, T=8003, 32/8 heads of 128 dims,
+// per dispatch under the profiler: 26.9 us and a 3.9 us merge launch on the
+// vector ALUs, 24.3 us here (69.7 MB, 2.9 TB/s).
+template <int D>
+struct VBf16 {
+    struct Args {
+        const __hip_bfloat16 *v;
+        // a hybrid cache's recent tokens, as VIl8Hyb
+        const void *kbuf, *vbuf;
+        int buf_dtype;
+        int64_t buf_sb, buf_sh, buf_st, t_buf;
+    };
+    static constexpr int NT = D / 16;
+    static constexpr int kSub = 1;
+    static constexpr bool kHybridBuffer = true;
+    static constexpr bool kHeavyCapable = false;
+    static constexpr float kMaxLag = 8.f;  // bf16 probabilities (float32's exponent range)
+    static constexpr bool kPrivateRing = false;
+    static constexpr int kTileV = kWave * D * 2;
+    static constexpr int kLoadsV = kTileV / 1024;
+    static constexpr int kPRows = 12;
+    static constexpr int kMaxSlots = 8;
+    static constexpr int kComputeWaves = 4;
+    static constexpr int CPR = D / 8;           // 16-byte chunks of a row
+    static constexpr int kSwz = CPR / 2 - 1;    // pair-position mask
+    struct Tile {
+        uint2 v[2][NT][2];  // [32-token half][dim tile][4-token quarter of the lane's 8]
+    };
+    struct State {};
+    __device__ static void issue(const Args &a, int64_t bh, int64_t cap, int64_t t0, int64_t t_last,
+                                 uint32_t sb, int lane) {
+        const char *vhead = reinterpret_cast<const char *>(a.v + bh * cap * D);
+#pragma unroll
+        for (int i = 0; i < kLoadsV; ++i) {
+            const int q = i * kWave + lane, tok = q / CPR, cpos = q % CPR;
+            const int chunk = cpos ^ ((tok & kSwz) << 1);
+            // rows past the split's last token reread it
+            const int64_t row = min(t0 + tok, t_last);
+            __builtin_amdgcn_global_load_lds(vhead + (row * CPR + chunk) * 16,
+                                             reinterpret_cast<lds_t<void> *>(sb + i * 1024), 16, 0,
+                                             kCpolNt);
+        }
+    }
+    // lane (g, l16): tokens 32 s2 + 8g + 4h .. +3 of dim 16n + l16 (row
+    // l16/4 and 8-byte piece l16%4 of the read's 4 x 16 block)
+    __device__ static void copy(Tile &tv, const char *sb, int, int lane) {
+        const int g = lane >> 4, l16 = lane & 15;
+        const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(sb));
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int tok = 8 * g + 4 * h + (l16 >> 2);
+            const uint32_t row = (uint32_t)(tok * D * 2 + ((tok & kSwz) << 5) + ((l16 & 3) << 3));
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int s2 = 0; s2 < 2; ++s2)
+                    tv.v[s2][n][h] = __builtin_bit_cast(
+                        uint2, ds_read_tr16_at(base + (row ^ (uint32_t)(n << 5)) + s2 * 32 * D * 2));
+        }
+    }
+    __device__ static void init(State &) {}
+    __device__ static void pv(Tile &tv, State &, f32x4 (&acc)[NT], const float (&p)[kMfmaRows],
+                              const float (&corr)[kMfmaRows], bool rescale, int, _Float16 *pw16,
+                              int lane) {
+        const int g = lane >> 4, l16 = lane & 15;
+        uint16_t *pw = reinterpret_cast<uint16_t *>(pw16);
+#pragma unroll
+        for (int r = 0; r < kMfmaRows; r += 2) {
+            float x0 = p[r], x1 = p[r + 1];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {  // hi, mid, lo: each the rounded rest
+                const uint32_t w = bf16x2_rn(x0, x1);
+                x0 -= __uint_as_float(w << 16);
+                x1 -= __uint_as_float(w & 0xffff0000u);
+                pw[(4 * k + r) * kPStride + lane] = (uint16_t)w;
+                pw[(4 * k + r + 1) * kPStride + lane] = (uint16_t)(w >> 16);
+            }
+        }
+        wave_lds_sync();
+        if (rescale) {
+            const f32x4 cv4 = f32x4{corr[0], corr[1], corr[2], corr[3]};
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[n] *= cv4;
+        }
+        // (tokens past the split's end hold its last token's values, p = 0)
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2) {
+            uint4 a = make_uint4(0u, 0u, 0u, 0u);
+            if (l16 < 12) a = *reinterpret_cast<const uint4 *>(pw + l16 * kPStride + 32 * s2 + 8 * g);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                const uint2 b0 = tv.v[s2][n][0], b1 = tv.v[s2][n][1];
+                acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    __builtin_bit_cast(bf16x8, a),
+                    __builtin_bit_cast(bf16x8, make_uint4(b0.x, b0.y, b1.x, b1.y)), acc[n], 0, 0, 0);
+            }
+        }
+        wave_lds_sync();
+    }
+    // lanes 0-15 hold rows 0-3 (hi), 16-31 the mid and 32-47 the lo parts:
+    // the combine's lo part is mid + lo
+    __device__ static void to_lds(const f32x4 (&acc)[NT], const State &, float *wa, int lane) {
+        const int g = lane >> 4, l16 = lane & 15;
+#pragma unroll
+        for (int r = 0; r < kMfmaRows; ++r)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                const float up = __shfl(acc[n][r], (lane + 16) & (kWave - 1));
+                if (g < 2) wa[(g * kMfmaRows + r) * D + 16 * n + l16] = g == 0 ? acc[n][r] : acc[n][r] + up;
+            }
+    }
+};
+
 template <int D, int NC, class VF>
 __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
     decode_attn_mfma_kernel(DecodeCommon c, typename VF::Args va) {
@@ -3564,14 +3696,9 @@ constexpr float kSvCodeOff = -32896.f;  // the operands sum to u/8 - kSvCodeOff
 static_assert(kSvLdsBytes <= kLdsMax, "SunShape-value MFMA LDS budget");
 static_assert(kSvVcbBytes <= 65536, "value codebook addressed with 16-bit LDS offsets");
 
-// ds_read_b64_tr_b16 at LDS byte offset `off` of the dynamic LDS block: in
-// each 16-lane group, lane j reads 4 halves; lane i receives column i of the
-// 4 x 16 block they form (row r from lane 4r + i/4, element i%4).
+// ds_read_tr16_at at byte offset `off` of the dynamic LDS block.
 __device__ __forceinline__ f16x4 ds_read_tr16(const char *lds_base, uint32_t off) {
-    typedef __attribute__((__vector_size__(4 * sizeof(__fp16)))) __fp16 hf16x4;
-    typedef __attribute__((address_space(3))) hf16x4 lhf16x4;
-    lhf16x4 *p = (lhf16x4 *)(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds_base)) + off);
-    return __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4f16(p));
+    return ds_read_tr16_at(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds_base)) + off);
 }
 
 template <int NH8>
@@ -5181,6 +5308,43 @@ extern "C" int ss_decode_attn_il8_hybrid(
                     q_offset, out, out_dtype, workspace, workspace_bytes, n_splits, k_buf, v_buf,
                     buf_dtype, buf_sb, buf_sh, buf_st, t_buf, stream, k_heavy, heavy_dims,
                     n_heavy_dims);
+}
+
+extern "C" int ss_decode_attn_dense_mfma(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
+    int n_centroids, const uint8_t *idx, const void *values, int v_dtype, int64_t cap,
+    int64_t t_kv, const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb,
+    int64_t buf_sh, int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims,
+    int n_heavy_dims, int causal, int64_t q_offset, void *out, int out_dtype, void *workspace,
+    size_t workspace_bytes, int n_splits, void *stream) {
+    const float *cents = static_cast<const float *>(codebook);
+    int rc = check_common(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, cents,
+                          n_blocks, n_centroids, idx, cap, t_kv, out, out_dtype);
+    if (rc) return rc;
+    if ((rc = dense_checks(values, v_dtype))) return rc;
+    SS_UNSUPPORTED(v_dtype == SS_BF16, "the matrix-core dense decode takes bfloat16 values");
+    const DecodeShape s = decode_shape(batch, n_q_heads, n_kv_heads, t_q, t_kv, n_splits,
+                                       kKindMfma);
+    DecodeCommon c;
+    rc = fill_common(c, s, q, q_dtype, n_q_heads, n_kv_heads, t_q, scale, perm, cents,
+                     n_centroids, idx, cap, t_kv, causal, q_offset, out, out_dtype, workspace,
+                     workspace_bytes, head_dim);
+    if (rc) return rc;
+    c.centroids = nullptr;
+    c.codebook = static_cast<const uint4 *>(codebook);
+    c.codebook_mul = reinterpret_cast<const float *>(
+        static_cast<const char *>(codebook) + (size_t)cb_tiles(n_blocks, n_centroids) * 2 * kWave * 16);
+    rc = check_buffer(k_buf, v_buf, buf_dtype, buf_sb, buf_sh, buf_st, t_buf, head_dim);
+    if (rc) return rc;
+    if ((rc = set_heavy(c, k_heavy, heavy_dims, n_heavy_dims))) return rc;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    const __hip_bfloat16 *v = static_cast<const __hip_bfloat16 *>(values);
+    if (head_dim == 128)
+        return launch_mfma<128, VBf16<128>>(
+            c, VBf16<128>::Args{v, k_buf, v_buf, buf_dtype, buf_sb, buf_sh, buf_st, t_buf}, s, st);
+    return launch_mfma<64, VBf16<64>>(
+        c, VBf16<64>::Args{v, k_buf, v_buf, buf_dtype, buf_sb, buf_sh, buf_st, t_buf}, s, st);
 }
 
 extern "C" int ss_decode_step_il8(

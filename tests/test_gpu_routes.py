@@ -61,3 +61,42 @@ def test_merge_attends_the_buffer(d, hq, t_kv, t_buf, t_q, bdt, pad):
         ref = O.sdpa_two_pass(q, scale, perm, cents, idx[:, :, :t_kv], kb.float().numpy(), v_all,
                               mask="causal" if t_q > 1 else None)
         assert rel_err(out.cpu().numpy(), ref) <= REL_TOL, name
+
+
+@pytest.mark.parametrize("b,hq,hkv,d,t_kv,t_buf,t_q,cap,qdt", [
+    (1, 4, 1, 128, 1, 0, 1, 256, torch.bfloat16),       # one token
+    (1, 8, 2, 128, 64, 0, 1, 64, torch.bfloat16),       # one whole tile, full cache
+    (2, 8, 2, 128, 1089, 0, 1, 1280, torch.bfloat16),   # 17 tiles and a token, several splits
+    (1, 8, 2, 64, 1023, 0, 1, 1024, torch.float16),     # head_dim 64, last tile one short
+    (1, 2, 2, 64, 130, 0, 5, 130, torch.bfloat16),      # causal rows, one query head per group
+    (1, 8, 2, 128, 600, 37, 3, 640, torch.bfloat16),    # buffered tokens, causal rows
+    (2, 6, 2, 128, 0, 20, 1, 64, torch.bfloat16),       # buffer only, three rows per group
+    (1, 8, 1, 128, 2000, 9, 1, 2048, torch.float32),    # float32 query, two row groups
+])
+def test_decode_bf16_values_on_the_matrix_cores(b, hq, hkv, d, t_kv, t_buf, t_q, cap, qdt):
+    """ss_decode_attn_dense_mfma: token-major bfloat16 values, with and
+    without buffered tokens, against the oracle over the same values."""
+    cents, perm, idx, _, q = decode_case(31 * t_kv + t_buf, b, hq, hkv, d, t_kv, t_q, cap)
+    rng = np.random.default_rng(t_kv + d)
+    # rows past t_kv hold NaN: nothing may read them into the result
+    vals = torch.full((b, hkv, cap, d), float("nan"), dtype=torch.bfloat16)
+    vals[:, :, :t_kv] = torch.from_numpy(rng.standard_normal((b, hkv, t_kv, d)).astype(np.float32))
+    kb = torch.from_numpy(rng.standard_normal((b, hkv, max(t_buf, 1), d)).astype(np.float32))
+    vb = torch.from_numpy(rng.standard_normal((b, hkv, max(t_buf, 1), d)).astype(np.float32))
+    kb, vb = kb.bfloat16(), vb.bfloat16()
+    qd = torch.from_numpy(q).to(qdt).cuda()
+    scale = 1.0 / np.sqrt(d)
+    total = t_kv + t_buf
+    # (kept alive for the plan's pointers)
+    idx_d, vals_d, perm_d, cb = t(idx), vals.cuda(), t(perm), _hip.codebook_f16x2(t(cents))
+    plan = _hip.prepare_decode_dense(qd, scale, perm_d, cb, d // 8, 256, idx_d, vals_d)
+    out = plan(qd, t_kv, t_q > 1, total - t_q if t_q > 1 else 0, kb.cuda(), vb.cuda(), t_buf,
+               out_dtype=torch.float32)
+    # queries scaled and rounded in their own type, then exact
+    qs = (qd * scale).float().cpu().numpy()
+    v_all = np.concatenate([vals[:, :, :t_kv].float().numpy(), vb[:, :, :t_buf].float().numpy()],
+                           axis=2)
+    ref = O.sdpa_two_pass(qs, 1.0, perm, cents, idx[:, :, :t_kv],
+                          kb[:, :, :t_buf].float().numpy() if t_buf else None, v_all,
+                          mask="causal" if t_q > 1 else None)
+    assert rel_err(out.cpu().numpy(), ref) <= REL_TOL
