@@ -664,6 +664,101 @@ int ss_decode_attn_grouped_il_hybrid(const void *q, int q_dtype, int64_t batch, 
                                      int n_splits, void *stream);
 
 /*
+ * Attention masks.  Element (b, query head, query position, key position t)
+ * is at data[b*sb + h*sh + q*sq + t] (strides in elements, 0 to broadcast;
+ * keys contiguous, over every attended position: compressed tokens, then
+ * buffered ones).  SS_MASK_BOOL: one byte, 0 hides the key (its score becomes
+ * float32's lowest value, so a row with every key hidden averages the
+ * values, as the reference's where() does, attention.py:329-341); the float
+ * types are added to the scores (attention.py:342-343).
+ */
+#define SS_MASK_BOOL 1
+#define SS_MASK_F16 2
+#define SS_MASK_BF16 3
+#define SS_MASK_F32 4
+typedef struct {
+    const void *data;
+    int type;
+    int64_t sb, sh, sq;
+} ss_attn_mask;
+
+/*
+ * The decodes above under a mask (the reference takes its two-pass path,
+ * attention.py:236-246, 307-350): ss_decode_attn_il8_hybrid,
+ * _dense_mfma, _grouped_il_hybrid, _turboquant_il, _turboquant,
+ * _grouped_hybrid, _dense_hybrid and _sunshape_v with `mask` before the
+ * stream (NULL or data NULL: none).  causal must be 0 with a mask; fp16 heavy
+ * key dims and a mask together are SS_ERR_UNSUPPORTED in the first four.
+ */
+int ss_decode_attn_il8_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
+    int n_centroids, const uint8_t *idx, const void *values_il8, int v_dtype, int64_t cap,
+    int64_t t_kv, const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb,
+    int64_t buf_sh, int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims,
+    int n_heavy_dims, int causal, int64_t q_offset, void *out, int out_dtype, void *workspace,
+    size_t workspace_bytes, int n_splits, const ss_attn_mask *mask, void *stream);
+int ss_decode_attn_dense_mfma_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
+    int n_centroids, const uint8_t *idx, const void *values, int v_dtype, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims, int n_heavy_dims,
+    int causal, int64_t q_offset, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
+    int n_splits, const ss_attn_mask *mask, void *stream);
+int ss_decode_attn_grouped_il_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint32_t *codes_il, const void *scales,
+    const void *zeros, int sz_dtype, int bits, int group_size, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims,
+    int n_heavy_dims, int causal, int64_t q_offset, void *out, int out_dtype, void *workspace,
+    size_t workspace_bytes, int n_splits, const ss_attn_mask *mask, void *stream);
+int ss_decode_attn_turboquant_il_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint32_t *codes_il, const float *norms,
+    const float *levels, const float *rotation, int64_t cap, int64_t t_kv, const void *k_buf,
+    const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh, int64_t buf_st, int64_t t_buf,
+    const void *k_heavy, const int32_t *heavy_dims, int n_heavy_dims, int causal, int64_t q_offset,
+    void *out, int out_dtype, void *workspace, size_t workspace_bytes, int n_splits,
+    const ss_attn_mask *mask, void *stream);
+int ss_decode_attn_turboquant_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint32_t *packed, const float *norms,
+    const float *levels, const float *rotation, int bits, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims, int n_heavy_dims,
+    int causal, int64_t q_offset, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
+    int n_splits, const ss_attn_mask *mask, void *stream);
+int ss_decode_attn_grouped_hybrid_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint32_t *packed, const void *scales,
+    const void *zeros, int sz_dtype, int bits, int group_size, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, int causal, int64_t q_offset, void *out, int out_dtype,
+    void *workspace, size_t workspace_bytes, int n_splits, const ss_attn_mask *mask, void *stream);
+int ss_decode_attn_dense_hybrid_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
+    int n_centroids, const uint8_t *idx, const void *values, int v_dtype, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, int causal, int64_t q_offset, void *out, int out_dtype,
+    void *workspace, size_t workspace_bytes, int n_splits, const ss_attn_mask *mask, void *stream);
+int ss_decode_attn_sunshape_v_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint8_t *v_idx, const float *v_centroids,
+    int v_block_dim, int v_n_centroids, const float *v_transform, const void *k_heavy,
+    const int32_t *heavy_dims, int n_heavy_dims, int64_t cap, int64_t t_kv, const void *k_buf,
+    const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh, int64_t buf_st, int64_t t_buf,
+    int causal, int64_t q_offset, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
+    int n_splits, const ss_attn_mask *mask, void *stream);
+
+/*
  * Repack grouped codes (pack_indices words, one row of packed_dim words per
  * token: word w of token (b,h,t) at packed[b*p_sb + h*p_sh + t*p_st + w]) into
  * the interleaved layout of ss_decode_attn_grouped_il at cache positions

@@ -201,6 +201,15 @@ _SIGNATURES = {
     "ss_dequantize_blockvq": (_int, [_c_void_p, _i64, _i64, _c_void_p, _int, _int, _int,
                                      _c_void_p, _c_void_p, _int, _c_void_p]),
 }
+# the masked decodes: a mask descriptor before the stream
+_MASKED = {"ss_decode_attn_il8_hybrid": "ss_decode_attn_il8_masked",
+           "ss_decode_attn_grouped_il_hybrid": "ss_decode_attn_grouped_il_masked",
+           **{f"ss_decode_attn_{n}": f"ss_decode_attn_{n}_masked"
+              for n in ("dense_mfma", "turboquant_il", "turboquant", "grouped_hybrid",
+                        "dense_hybrid", "sunshape_v")}}
+for _plain, _masked in _MASKED.items():
+    _r, _a = _SIGNATURES[_plain]
+    _SIGNATURES[_masked] = (_r, [*_a[:-1], _c_void_p, _a[-1]])
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
@@ -510,7 +519,8 @@ class PreparedDecodeDense(PreparedDecode):
 
     def __call__(self, q: torch.Tensor, t_kv: int, causal: bool = False, q_offset: int = 0,
                  buf_keys: torch.Tensor | None = None, buf_values: torch.Tensor | None = None,
-                 buf_len: int = 0, out_dtype: torch.dtype | None = None) -> torch.Tensor:
+                 buf_len: int = 0, out_dtype: torch.dtype | None = None,
+                 mask: AttnMask | None = None) -> torch.Tensor:
         if q.shape != self.shape or q.dtype != self.dtype or not q.is_contiguous() or \
                 q.device.index != self.dev:
             raise ValueError(f"query must be contiguous {self.dtype} {self.shape} on cuda:{self.dev}")
@@ -527,11 +537,14 @@ class PreparedDecodeDense(PreparedDecode):
             ws = decode_workspace(self.dev, 1, st)
         mid = (int(t_kv), *buf, None, None, 0, int(bool(causal)), int(q_offset), out.data_ptr(),
                dtype_code(out.dtype))
-        rc = self.fn(q.data_ptr(), *self.pre, *mid, ws.data_ptr(), ws.numel(), 0, st)
+        fn, last = self.fn, (st,)
+        if mask is not None:
+            fn, last = load_library().ss_decode_attn_dense_mfma_masked, (ctypes.addressof(mask), st)
+        rc = fn(q.data_ptr(), *self.pre, *mid, ws.data_ptr(), ws.numel(), 0, *last)
         if rc == SS_ERR_WORKSPACE:
             _, need = decode_plan(KIND_IL8, *self.plan_args, int(t_kv), 0)
             ws = decode_workspace(self.dev, need, st)
-            rc = self.fn(q.data_ptr(), *self.pre, *mid, ws.data_ptr(), ws.numel(), 0, st)
+            rc = fn(q.data_ptr(), *self.pre, *mid, ws.data_ptr(), ws.numel(), 0, *last)
         _launched(_attn_stat(self.stat, causal), rc)
         if _check_waits:
             check_decode_waits(self.dev)
@@ -989,6 +1002,41 @@ def default_splits(batch, n_q_heads, n_kv_heads, t_q, head_dim, t_kv) -> int:
                                                        head_dim, t_kv))
 
 
+class AttnMask(ctypes.Structure):
+    """``ss_attn_mask``; :func:`attn_mask` builds it and keeps its tensor."""
+
+    _fields_ = [("data", _c_void_p), ("type", _int), ("sb", _i64), ("sh", _i64), ("sq", _i64)]
+
+
+_MASK_TYPE = {torch.bool: 1, torch.float16: 2, torch.bfloat16: 3, torch.float32: 4}
+
+
+def attn_mask(mask: torch.Tensor, shape: tuple) -> AttnMask | None:
+    """The descriptor of a boolean or additive mask broadcastable to ``shape``
+    = (B, Hq, T_q, T_kv) (other types are added as float32, as the two-pass
+    path adds them); None where it does not broadcast."""
+    if mask.dtype not in _MASK_TYPE:
+        mask = mask.float()
+    try:
+        full = mask.expand(shape)
+    except RuntimeError:
+        return None
+    if full.stride(3) != 1 and shape[3] != 1:
+        full = mask.expand(*mask.shape[:-1], shape[3]).contiguous().expand(shape)
+    require_gpu(full)
+    d = AttnMask(full.data_ptr(), _MASK_TYPE[full.dtype], *full.stride()[:3])
+    d.tensor = full
+    return d
+
+
+def _masked_call(name: str, args: tuple, mask: AttnMask | None) -> int:
+    """``name`` with ``args``, or its masked form when there is a mask."""
+    lib = load_library()
+    if mask is None:
+        return getattr(lib, name)(*args)
+    return getattr(lib, _MASKED[name])(*args[:-1], ctypes.addressof(mask), args[-1])
+
+
 def _check_decode_common(q, idx, centroids, perm):
     require_gpu(q, idx, centroids, perm)
     if q.dim() != 4 or not q.is_contiguous():
@@ -1006,7 +1054,8 @@ def decode_attn_dense(q: torch.Tensor, scale: float, perm: torch.Tensor | None,
                       t_kv: int, causal: bool = False, q_offset: int = 0,
                       out: torch.Tensor | None = None, out_dtype: torch.dtype | None = None,
                       n_splits: int = 0, buf_keys: torch.Tensor | None = None,
-                      buf_values: torch.Tensor | None = None, buf_len: int = 0) -> torch.Tensor:
+                      buf_values: torch.Tensor | None = None, buf_len: int = 0,
+                      mask: AttnMask | None = None) -> torch.Tensor:
     """Fused decode over a (B, Hkv, cap, NB) index buffer and (B, Hkv, cap, D)
     dense values; returns (B, Hq, T_q, D).  A hybrid cache's recent tokens
     ``buf_keys``/``buf_values`` (B, Hkv, >= buf_len, D) join the same
@@ -1024,19 +1073,19 @@ def decode_attn_dense(q: torch.Tensor, scale: float, perm: torch.Tensor | None,
     if out is None:
         out = torch.empty((b_, hq, tq, d), dtype=out_dtype or q.dtype, device=q.device)
     buf_len = int(buf_len)
-    if buf_len > 0:
+    if buf_len > 0 or mask is not None:
         buf_keys, buf_values, bdt, bsb, bsh, bst = _buffer_args(buf_keys, buf_values, buf_len,
                                                                 b_, hkv, d)
         lib = load_library()
         ws_bytes = lib.ss_decode_turboquant_workspace_bytes(b_, hq, hkv, tq, d, int(t_kv),
                                                             buf_len, int(n_splits))
         ws = decode_workspace(q.device, ws_bytes)
-        _launched(_attn_stat("sunshape_fused_attention", causal), lib.ss_decode_attn_dense_hybrid(
+        _launched(_attn_stat("sunshape_fused_attention", causal), _masked_call("ss_decode_attn_dense_hybrid", (
             ptr(q), dtype_code(q.dtype), b_, hq, hkv, tq, d, float(scale), ptr(perm),
             ptr(centroids), nb, nc, ptr(idx), ptr(values), dtype_code(values.dtype), cap,
             int(t_kv), ptr(buf_keys), ptr(buf_values), bdt, bsb, bsh, bst, buf_len,
             int(bool(causal)), int(q_offset), ptr(out), dtype_code(out.dtype), ptr(ws),
-            ws_bytes if ws is not None else 0, int(n_splits), stream_handle(q.device)))
+            ws_bytes if ws is not None else 0, int(n_splits), stream_handle(q.device)), mask))
         return out
     ws_bytes = decode_workspace_bytes(b_, hq, hkv, tq, d, t_kv, n_splits)
     ws = decode_workspace(q.device, ws_bytes)
@@ -1105,7 +1154,8 @@ def decode_attn_il8(q: torch.Tensor, scale: float, perm: torch.Tensor | None,
                     buf_keys: torch.Tensor | None = None,
                     buf_values: torch.Tensor | None = None, buf_len: int = 0,
                     k_heavy: torch.Tensor | None = None,
-                    heavy_dims: torch.Tensor | None = None) -> torch.Tensor:
+                    heavy_dims: torch.Tensor | None = None,
+                    mask: AttnMask | None = None) -> torch.Tensor:
     """Fused decode (matrix-core LUT and P.V) over fp16 values in the 8-token
     interleaved layout ``values_il8`` (B, Hkv, cap/8, D, 8).  ``codebook`` is
     :func:`codebook_f16x2` of ``centroids`` (prepared here when None).  A
@@ -1138,11 +1188,11 @@ def decode_attn_il8(q: torch.Tensor, scale: float, perm: torch.Tensor | None,
     stat = _attn_stat("sunshape_fused_attention_mfma", causal)
     heavy = _heavy_args(k_heavy, heavy_dims, b_, hkv, cap, 32)
     _poll_waits(q.device)
-    if (buf_keys is None or buf_len == 0) and k_heavy is None:
+    if (buf_keys is None or buf_len == 0) and k_heavy is None and mask is None:
         _launched(stat, load_library().ss_decode_attn_il8(*common, *tail))
     else:
         buf = _buffer_ptrs(b_, hkv, d, buf_keys, buf_values, buf_len if buf_keys is not None else 0)
-        _launched(stat, load_library().ss_decode_attn_il8_hybrid(*common, *buf, *heavy, *tail))
+        _launched(stat, _masked_call("ss_decode_attn_il8_hybrid", (*common, *buf, *heavy, *tail), mask))
     if _check_waits:
         check_decode_waits(q.device)
     return out
@@ -1360,7 +1410,8 @@ def decode_attn_grouped(q: torch.Tensor, scale: float, perm: torch.Tensor | None
                         out: torch.Tensor | None = None, out_dtype: torch.dtype | None = None,
                         n_splits: int = 0, buf_keys: torch.Tensor | None = None,
                         buf_values: torch.Tensor | None = None,
-                        buf_len: int = 0) -> torch.Tensor:
+                        buf_len: int = 0,
+                        mask: AttnMask | None = None) -> torch.Tensor:
     """Fused decode with grouped-quantised values decoded in registers.  A
     hybrid cache's recent tokens join the softmax as in
     :func:`decode_attn_dense` (``ss_decode_attn_grouped_hybrid``)."""
@@ -1379,7 +1430,7 @@ def decode_attn_grouped(q: torch.Tensor, scale: float, perm: torch.Tensor | None
     if out is None:
         out = torch.empty((b_, hq, tq, d), dtype=out_dtype or q.dtype, device=q.device)
     buf_len = int(buf_len)
-    if buf_len > 0:
+    if buf_len > 0 or mask is not None:
         buf_keys, buf_values, bdt, bsb, bsh, bst = _buffer_args(buf_keys, buf_values, buf_len,
                                                                 b_, hkv, d)
         lib = load_library()
@@ -1387,13 +1438,13 @@ def decode_attn_grouped(q: torch.Tensor, scale: float, perm: torch.Tensor | None
                                                             buf_len, int(n_splits))
         ws = decode_workspace(q.device, ws_bytes)
         _launched(_attn_stat("sunshape_fused_attention_dequant", causal),
-                  lib.ss_decode_attn_grouped_hybrid(
+                  _masked_call("ss_decode_attn_grouped_hybrid", (
                       ptr(q), dtype_code(q.dtype), b_, hq, hkv, tq, d, float(scale), ptr(perm),
                       ptr(centroids), nb, nc, ptr(idx), ptr(packed), ptr(scales), ptr(zeros),
                       dtype_code(scales.dtype), int(bits), int(group_size), cap, int(t_kv),
                       ptr(buf_keys), ptr(buf_values), bdt, bsb, bsh, bst, buf_len,
                       int(bool(causal)), int(q_offset), ptr(out), dtype_code(out.dtype), ptr(ws),
-                      ws_bytes if ws is not None else 0, int(n_splits), stream_handle(q.device)))
+                      ws_bytes if ws is not None else 0, int(n_splits), stream_handle(q.device)), mask))
         return out
     ws_bytes = decode_workspace_bytes(b_, hq, hkv, tq, d, t_kv, n_splits)
     ws = decode_workspace(q.device, ws_bytes)
@@ -1450,7 +1501,8 @@ def decode_attn_sunshape_v(q: torch.Tensor, scale: float, perm: torch.Tensor | N
                            n_splits: int = 0, buf_keys: torch.Tensor | None = None,
                            buf_values: torch.Tensor | None = None,
                            buf_len: int = 0, k_heavy: torch.Tensor | None = None,
-                           heavy_dims: torch.Tensor | None = None) -> torch.Tensor:
+                           heavy_dims: torch.Tensor | None = None,
+                           mask: AttnMask | None = None) -> torch.Tensor:
     """Fused decode over SunShape block-VQ values: ``v_idx`` (B, Hkv, cap,
     D / bd) uint8, ``v_centroids`` (D / bd, nc, bd) float32, ``v_transform``
     (D, D) float32 taking a codec-space row to the original basis.  Buffered
@@ -1491,13 +1543,13 @@ def decode_attn_sunshape_v(q: torch.Tensor, scale: float, perm: torch.Tensor | N
     ws_bytes = lib.ss_decode_turboquant_workspace_bytes(b_, hq, hkv, tq, d, int(t_kv), buf_len,
                                                         int(n_splits))
     ws = decode_workspace(q.device, ws_bytes)
-    _launched(_attn_stat("sunshape_fused_attention_sunshape_v", causal), lib.ss_decode_attn_sunshape_v(
+    _launched(_attn_stat("sunshape_fused_attention_sunshape_v", causal), _masked_call("ss_decode_attn_sunshape_v", (
         ptr(q), dtype_code(q.dtype), b_, hq, hkv, tq, d, float(scale), ptr(perm), ptr(centroids),
         nb, nc, ptr(idx), ptr(v_idx), ptr(v_centroids), vbd, vnc, ptr(v_transform),
         ptr(k_heavy), ptr(heavy_dims), nhd, cap,
         int(t_kv), ptr(buf_keys), ptr(buf_values), bdt, bsb, bsh, bst, buf_len,
         int(bool(causal)), int(q_offset), ptr(out), dtype_code(out.dtype), ptr(ws),
-        ws_bytes if ws is not None else 0, int(n_splits), stream_handle(q.device)))
+        ws_bytes if ws is not None else 0, int(n_splits), stream_handle(q.device)), mask))
     return out
 
 
@@ -1509,7 +1561,8 @@ def decode_attn_turboquant(q: torch.Tensor, scale: float, perm: torch.Tensor | N
                            n_splits: int = 0, buf_keys: torch.Tensor | None = None,
                            buf_values: torch.Tensor | None = None,
                            buf_len: int = 0, k_heavy: torch.Tensor | None = None,
-                           heavy_dims: torch.Tensor | None = None) -> torch.Tensor:
+                           heavy_dims: torch.Tensor | None = None,
+                           mask: AttnMask | None = None) -> torch.Tensor:
     """Fused decode over TurboQuant values: ``packed`` (B, Hkv, cap,
     packed_dim) codes, ``norms`` (B, Hkv, cap) float32, ``levels`` the 2^bits
     scaled Lloyd-Max levels (any float sequence; copied to the kernel
@@ -1544,12 +1597,12 @@ def decode_attn_turboquant(q: torch.Tensor, scale: float, perm: torch.Tensor | N
     ws_bytes = lib.ss_decode_turboquant_workspace_bytes(b_, hq, hkv, tq, d, int(t_kv), buf_len,
                                                         int(n_splits))
     ws = decode_workspace(q.device, ws_bytes)
-    _launched(_attn_stat("sunshape_fused_attention_turboquant", causal), lib.ss_decode_attn_turboquant(
+    _launched(_attn_stat("sunshape_fused_attention_turboquant", causal), _masked_call("ss_decode_attn_turboquant", (
         ptr(q), dtype_code(q.dtype), b_, hq, hkv, tq, d, float(scale), ptr(perm), ptr(centroids),
         nb, nc, ptr(idx), ptr(packed), ptr(norms), ctypes.cast(lv_host, ctypes.c_void_p).value,
         ptr(rotation), int(bits), cap, int(t_kv), ptr(buf_keys), ptr(buf_values), bdt, bsb, bsh,
         bst, buf_len, *_heavy_args(k_heavy, heavy_dims, b_, hkv, cap, 64), int(bool(causal)), int(q_offset), ptr(out), dtype_code(out.dtype), ptr(ws),
-        ws_bytes if ws is not None else 0, int(n_splits), stream_handle(q.device)))
+        ws_bytes if ws is not None else 0, int(n_splits), stream_handle(q.device)), mask))
     return out
 
 
@@ -1571,7 +1624,8 @@ def decode_attn_turboquant_il(q: torch.Tensor, scale: float, perm: torch.Tensor 
                               buf_keys: torch.Tensor | None = None,
                               buf_values: torch.Tensor | None = None,
                               buf_len: int = 0, k_heavy: torch.Tensor | None = None,
-                              heavy_dims: torch.Tensor | None = None) -> torch.Tensor:
+                              heavy_dims: torch.Tensor | None = None,
+                              mask: AttnMask | None = None) -> torch.Tensor:
     """Fused decode (matrix-core LUT and P.V) over 2-bit TurboQuant values
     whose codes are token-interleaved (``codes_il`` (B, Hkv, cap/16, D) words,
     written by :func:`pack_grouped_il`), ``norms`` (B, Hkv, cap) float32,
@@ -1612,13 +1666,13 @@ def decode_attn_turboquant_il(q: torch.Tensor, scale: float, perm: torch.Tensor 
     ws = decode_workspace(q.device, ws_bytes)
     _poll_waits(q.device)
     _launched(_attn_stat("sunshape_fused_attention_turboquant", causal),
-              lib.ss_decode_attn_turboquant_il(
+              _masked_call("ss_decode_attn_turboquant_il", (
         ptr(q), dtype_code(q.dtype), b_, hq, hkv, tq, d, float(scale), ptr(perm), ptr(codebook),
         nb, nc, ptr(idx), ptr(codes_il), ptr(norms), ctypes.cast(lv_host, ctypes.c_void_p).value,
         ptr(rotation), cap, int(t_kv), ptr(buf_keys), ptr(buf_values), bdt, bsb, bsh,
         bst, buf_len, *_heavy_args(k_heavy, heavy_dims, b_, hkv, cap, 32), int(bool(causal)),
         int(q_offset), ptr(out), dtype_code(out.dtype), ptr(ws),
-        ws_bytes if ws is not None else 0, int(n_splits), stream_handle(q.device)))
+        ws_bytes if ws is not None else 0, int(n_splits), stream_handle(q.device)), mask))
     if _check_waits:
         check_decode_waits(q.device)
     return out
@@ -1633,7 +1687,8 @@ def decode_attn_grouped_il(q: torch.Tensor, scale: float, perm: torch.Tensor | N
                            buf_keys: torch.Tensor | None = None,
                            buf_values: torch.Tensor | None = None,
                            buf_len: int = 0, k_heavy: torch.Tensor | None = None,
-                           heavy_dims: torch.Tensor | None = None) -> torch.Tensor:
+                           heavy_dims: torch.Tensor | None = None,
+                           mask: AttnMask | None = None) -> torch.Tensor:
     """Fused decode (matrix-core LUT and P.V) over grouped values whose codes
     are token-interleaved: ``codes_il`` (B, Hkv, cap * bits / 32, D) 32-bit
     words (see :func:`pack_grouped_il`), ``scales``/``zeros`` (B, Hkv, cap, D
@@ -1669,15 +1724,16 @@ def decode_attn_grouped_il(q: torch.Tensor, scale: float, perm: torch.Tensor | N
             int(n_splits), stream_handle(q.device))
     heavy = _heavy_args(k_heavy, heavy_dims, b_, hkv, cap, 32)
     _poll_waits(q.device)
-    if (buf_keys is None or buf_len == 0) and k_heavy is None:
+    if (buf_keys is None or buf_len == 0) and k_heavy is None and mask is None:
         _launched(_attn_stat("sunshape_fused_attention_dequant_mfma", causal), load_library().ss_decode_attn_grouped_il(
             *common, int(bool(causal)), int(q_offset), *tail))
         if _check_waits:
             check_decode_waits(q.device)
         return out
     buf = _buffer_ptrs(b_, hkv, d, buf_keys, buf_values, buf_len if buf_keys is not None else 0)
-    _launched(_attn_stat("sunshape_fused_attention_dequant_mfma", causal), load_library().ss_decode_attn_grouped_il_hybrid(
-        *common, *buf, *heavy, int(bool(causal)), int(q_offset), *tail))
+    _launched(_attn_stat("sunshape_fused_attention_dequant_mfma", causal), _masked_call(
+        "ss_decode_attn_grouped_il_hybrid",
+        (*common, *buf, *heavy, int(bool(causal)), int(q_offset), *tail), mask))
     if _check_waits:
         check_decode_waits(q.device)
     return out

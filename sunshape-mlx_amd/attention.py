@@ -9,11 +9,11 @@ the cache, for every query head of every KV group in a single launch (the
 reference loops over (batch, KV head, q head) with one Metal dispatch each,
 attention.py:268-305).
 
-Routing follows the reference (attention.py:236-246): a compressed-only cache
-with no mask or a causal mask takes a fused kernel; a hybrid cache with
-buffered full-precision tokens, or an explicit mask array, takes the two-pass
-path (attention.py:307-350), which here also runs on the GPU (HIP LUT and
-score kernels, torch softmax and matmul).
+The reference sends a compressed-only cache with no mask or a causal mask to a
+fused kernel and everything else to its two-pass path (attention.py:236-246,
+307-350).  Here buffered tokens and, over few query rows, explicit mask arrays
+stay on the fused kernels as well; the two-pass path, which also runs on the
+GPU (HIP LUT and score kernels, torch softmax and matmul), takes the rest.
 """
 
 from __future__ import annotations
@@ -171,12 +171,22 @@ def _fused_hybrid_step(cache: HybridSunShapeKVCache, queries: torch.Tensor, scal
     return out
 
 
+# Query rows of a KV head (heads of its group x positions) up to which an
+# array mask stays on the fused decodes: they stream the cache once per four
+# rows, the two-pass path materialises every score once.  Measured with 32/8
+# heads at 512 to 131072 tokens in all: at 4 rows 23-61 us against 106-761 us,
+# at 64 rows 17-382 us against 104-954 us (fused ahead for every value type),
+# at 256 rows 912 against 772 us (bf16) and 1435 against 1139 us (3-bit) at
+# 32768 tokens, the other types still ahead.
+_MASKED_ROWS = 64
+
+
 def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: int,
-           out_dtype: torch.dtype):
+           out_dtype: torch.dtype, mask=None):
     """One fused launch over the whole cache, or None when no fused kernel
     applies to this cache / shape (the reference's None-fallback,
-    kernels.py:259-291)."""
-    if getattr(cache, "_pending", None) is not None and queries.shape[2] <= _hip.MAX_STEP_TOKENS:
+    kernels.py:259-291).  ``mask``: an array mask's ``_hip.AttnMask``."""
+    if mask is None and getattr(cache, "_pending", None) is not None and queries.shape[2] <= _hip.MAX_STEP_TOKENS:
         if isinstance(cache, HybridSunShapeKVCache):
             out = _fused_hybrid_step(cache, queries, scale, causal, q_offset, out_dtype)
         else:
@@ -201,7 +211,8 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
         # which for bf16 (8 significant bits) moves outputs by ~2^-9 of
         # their scale, so bf16 caches keep the reference's two passes
         return None
-    if isinstance(cache, HybridSunShapeKVCache) and tq > 1 and ops.get("k_heavy") is None and \
+    if mask is None and isinstance(cache, HybridSunShapeKVCache) and tq > 1 and \
+            ops.get("k_heavy") is None and \
             cache.dtype == torch.float16 and \
             q.dtype in (torch.float16, torch.bfloat16) and \
             _hip.prefill_supported(hq, cache.n_kv_heads, tq, d, codec.n_blocks):
@@ -235,7 +246,7 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
     # reconstructed from the codebook, both products on the matrix cores
     b_, hq, tq, d = queries.shape
     hv = {"k_heavy": ops.get("k_heavy"), "heavy_dims": ops.get("heavy_dims")}
-    if not buffered and kind == "il8" and tq > 1 and hv["k_heavy"] is None and \
+    if mask is None and not buffered and kind == "il8" and tq > 1 and hv["k_heavy"] is None and \
             _hip.prefill_supported(hq, cache.n_kv_heads, tq, d, codec.n_blocks):
         try:
             out = _hip.prefill_attn_il8(q, kscale, perm, codec.kernel_codebook(), codec.n_centroids,
@@ -247,7 +258,7 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
         return out
     # the matrix-core decodes without a token buffer: one prepared launch
     # (argument checks, codebook and split plan done once per cache layout)
-    if not buffered and kind in ("il8", "grouped_il") and hv["k_heavy"] is None:
+    if mask is None and not buffered and kind in ("il8", "grouped_il") and hv["k_heavy"] is None:
         try:
             plan = _prepared_decode(cache, ops, codec, q, kscale, perm)
             out = plan(q, t_kv, causal, q_offset, out_dtype=out_dtype)
@@ -261,7 +272,7 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
         try:
             plan = _prepared_decode(cache, ops, codec, q, kscale, perm)
             out = plan(q, t_kv, causal, q_offset, ops.get("buf_keys"), ops.get("buf_values"),
-                       buffered, out_dtype=out_dtype)
+                       buffered, out_dtype=out_dtype, mask=mask)
         except _hip.SunShapeUnsupported:
             return None
         codec.last_score_backend = "hip_fused_buffer" if buffered else "hip_fused"
@@ -269,7 +280,7 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
     # il8 and grouped_il with a hybrid cache's buffered tokens (the buffer
     # window passed per call); rotated codecs hand the kernel rotated buffer copies
     # and take the checked launch below
-    if buffered and kind in ("il8", "grouped_il") and hv["k_heavy"] is None and \
+    if mask is None and buffered and kind in ("il8", "grouped_il") and hv["k_heavy"] is None and \
             (codec.mode in PERM_MODES or not codec.use_rotation):
         try:
             plan = _prepared_decode(cache, ops, codec, q, kscale, perm, buffered=True)
@@ -280,14 +291,16 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
         codec.last_score_backend = ("hip_fused_mfma_buffer" if kind == "il8"
                                     else "hip_fused_mfma_dequant_buffer")
         return out
-    kw = dict(t_kv=t_kv, causal=causal, q_offset=q_offset, out_dtype=out_dtype)
+    kw = dict(t_kv=t_kv, causal=causal, q_offset=q_offset, out_dtype=out_dtype, mask=mask)
     try:
         if kind == "il8":
             out = _hip.decode_attn_il8(q, kscale, perm, codec.scoring_centroids(), ops["idx"],
                                        ops["values"], codebook=codec.kernel_codebook(),
-                                       buf_keys=ops["buf_keys"], buf_values=ops["buf_values"],
+                                       buf_keys=ops.get("buf_keys"),
+                                       buf_values=ops.get("buf_values"),
                                        buf_len=buffered, **hv, **kw)
             codec.last_score_backend = ("hip_fused_mfma_buffer" if buffered
+                                        else "hip_fused_mfma" if hv["k_heavy"] is None
                                         else "hip_fused_mfma_heavy")
         elif kind == "grouped_il":
             out = _hip.decode_attn_grouped_il(q, kscale, perm, codec.scoring_centroids(),
@@ -432,10 +445,16 @@ def sunshape_sdpa(queries: torch.Tensor, cache: SunShapeKVCache | HybridSunShape
     compressed = cache.compressed_offset if is_hybrid else t_kv
     # a non-empty hybrid buffer stays on the fused path where the kernel
     # takes it (_fused returns None otherwise)
+    # and so does an array mask over few query rows
     can_fuse = (mask is None or use_causal) and compressed > 0
-    if can_fuse:
+    array = None
+    if isinstance(mask, torch.Tensor) and compressed > 0 and hq // hkv * tq <= _MASKED_ROWS:
+        array = _hip.attn_mask(mask.to(queries.device), (b_, hq, tq, t_kv))
+    if can_fuse or array is not None:
         out = _fused(cache, queries, scale, use_causal, t_kv - tq if use_causal else 0,
-                     out_dtype)
+                     out_dtype, array)
         if out is not None:
+            if array is not None:  # the name the two-pass path reports for a mask
+                cache.codec.last_score_backend = "hip"
             return out
     return _two_pass(cache, queries, scale, mask, out_dtype)

@@ -296,7 +296,8 @@ static int il8_impl(const void *q, int q_dtype, int64_t batch, int n_q_heads, in
                     size_t workspace_bytes, int n_splits, const void *k_buf, const void *v_buf,
                     int buf_dtype, int64_t buf_sb, int64_t buf_sh, int64_t buf_st,
                     int64_t t_buf, void *stream, const void *k_heavy = nullptr,
-                    const int32_t *heavy_dims = nullptr, int n_heavy_dims = 0) {
+                    const int32_t *heavy_dims = nullptr, int n_heavy_dims = 0,
+                    const ss_attn_mask *mask = nullptr) {
     const float *cents = static_cast<const float *>(codebook);
     int rc = check_common(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, cents,
                           n_blocks, n_centroids, idx, cap, t_kv, out, out_dtype);
@@ -321,9 +322,11 @@ static int il8_impl(const void *q, int q_dtype, int64_t batch, int n_q_heads, in
     if (rc) return rc;
     rc = set_heavy(c, k_heavy, heavy_dims, n_heavy_dims);
     if (rc) return rc;
+    if ((rc = set_mask(c, mask))) return rc;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const __half *v8 = reinterpret_cast<const __half *>(values_il8);
-    if (t_buf > 0 || c.nhd > 0) {  // the hybrid cache's kernel (buffer share, heavy dims)
+    // the hybrid cache's kernel (buffer share, heavy dims, masks)
+    if (t_buf > 0 || c.nhd > 0 || c.mask_dt != kMaskNone) {
         if (head_dim == 128)
             return launch_mfma<128, VIl8Hyb<128>>(
                 c, VIl8Hyb<128>::Args{v8, k_buf, v_buf, buf_dtype, buf_sb, buf_sh, buf_st, t_buf},
@@ -364,14 +367,29 @@ extern "C" int ss_decode_attn_il8_hybrid(
                     n_heavy_dims);
 }
 
-extern "C" int ss_decode_attn_dense_mfma(
+extern "C" int ss_decode_attn_il8_masked(
     const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
     int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
-    int n_centroids, const uint8_t *idx, const void *values, int v_dtype, int64_t cap,
+    int n_centroids, const uint8_t *idx, const void *values_il8, int v_dtype, int64_t cap,
     int64_t t_kv, const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb,
     int64_t buf_sh, int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims,
     int n_heavy_dims, int causal, int64_t q_offset, void *out, int out_dtype, void *workspace,
-    size_t workspace_bytes, int n_splits, void *stream) {
+    size_t workspace_bytes, int n_splits, const ss_attn_mask *mask, void *stream) {
+    return il8_impl(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, scale, perm,
+                    codebook, n_blocks, n_centroids, idx, values_il8, v_dtype, cap, t_kv, causal,
+                    q_offset, out, out_dtype, workspace, workspace_bytes, n_splits, k_buf, v_buf,
+                    buf_dtype, buf_sb, buf_sh, buf_st, t_buf, stream, k_heavy, heavy_dims,
+                    n_heavy_dims, mask);
+}
+
+static int decode_attn_dense_mfma_impl(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
+    int n_centroids, const uint8_t *idx, const void *values, int v_dtype, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims, int n_heavy_dims,
+    int causal, int64_t q_offset, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
+    int n_splits, const ss_attn_mask *mask, void *stream) {
     const float *cents = static_cast<const float *>(codebook);
     int rc = check_common(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, cents,
                           n_blocks, n_centroids, idx, cap, t_kv, out, out_dtype);
@@ -392,6 +410,7 @@ extern "C" int ss_decode_attn_dense_mfma(
     rc = check_buffer(k_buf, v_buf, buf_dtype, buf_sb, buf_sh, buf_st, t_buf, head_dim);
     if (rc) return rc;
     if ((rc = set_heavy(c, k_heavy, heavy_dims, n_heavy_dims))) return rc;
+    if ((rc = set_mask(c, mask))) return rc;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const __hip_bfloat16 *v = static_cast<const __hip_bfloat16 *>(values);
     if (head_dim == 128)
@@ -399,6 +418,38 @@ extern "C" int ss_decode_attn_dense_mfma(
             c, VBf16<128>::Args{v, k_buf, v_buf, buf_dtype, buf_sb, buf_sh, buf_st, t_buf}, s, st);
     return launch_mfma<64, VBf16<64>>(
         c, VBf16<64>::Args{v, k_buf, v_buf, buf_dtype, buf_sb, buf_sh, buf_st, t_buf}, s, st);
+}
+
+extern "C" int ss_decode_attn_dense_mfma(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
+    int n_centroids, const uint8_t *idx, const void *values, int v_dtype, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims, int n_heavy_dims,
+    int causal, int64_t q_offset, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
+    int n_splits, void *stream) {
+    return decode_attn_dense_mfma_impl(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim,
+                                       scale, perm, codebook, n_blocks, n_centroids, idx, values,
+                                       v_dtype, cap, t_kv, k_buf, v_buf, buf_dtype, buf_sb, buf_sh,
+                                       buf_st, t_buf, k_heavy, heavy_dims, n_heavy_dims, causal,
+                                       q_offset, out, out_dtype, workspace, workspace_bytes,
+                                       n_splits, nullptr, stream);
+}
+
+extern "C" int ss_decode_attn_dense_mfma_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
+    int n_centroids, const uint8_t *idx, const void *values, int v_dtype, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims, int n_heavy_dims,
+    int causal, int64_t q_offset, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
+    int n_splits, const ss_attn_mask *mask, void *stream) {
+    return decode_attn_dense_mfma_impl(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim,
+                                       scale, perm, codebook, n_blocks, n_centroids, idx, values,
+                                       v_dtype, cap, t_kv, k_buf, v_buf, buf_dtype, buf_sb, buf_sh,
+                                       buf_st, t_buf, k_heavy, heavy_dims, n_heavy_dims, causal,
+                                       q_offset, out, out_dtype, workspace, workspace_bytes,
+                                       n_splits, mask, stream);
 }
 
 // ---------------------------------------------------------------------------

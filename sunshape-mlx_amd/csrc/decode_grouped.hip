@@ -14,7 +14,8 @@ static int grouped_il_impl(const void *q, int q_dtype, int64_t batch, int n_q_he
                            const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
                            int64_t buf_st, int64_t t_buf, void *stream,
                            const void *k_heavy = nullptr, const int32_t *heavy_dims = nullptr,
-                           int n_heavy_dims = 0) {
+                           int n_heavy_dims = 0,
+                           const ss_attn_mask *mask = nullptr) {
     const float *cents = static_cast<const float *>(codebook);
     int rc = check_common(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, cents,
                           n_blocks, n_centroids, idx, cap, t_kv, out, out_dtype);
@@ -45,6 +46,7 @@ static int grouped_il_impl(const void *q, int q_dtype, int64_t batch, int n_q_he
     if (rc) return rc;
     rc = set_heavy(c, k_heavy, heavy_dims, n_heavy_dims);
     if (rc) return rc;
+    if ((rc = set_mask(c, mask))) return rc;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const int ng = head_dim / group_size;
 #define SS_GIL(DD, BB, NGG, SZT)                                                              \
@@ -113,14 +115,32 @@ extern "C" int ss_decode_attn_grouped_il_hybrid(
                            buf_st, t_buf, stream, k_heavy, heavy_dims, n_heavy_dims);
 }
 
-extern "C" int ss_decode_attn_turboquant_il(
+extern "C" int ss_decode_attn_grouped_il_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint32_t *codes_il, const void *scales,
+    const void *zeros, int sz_dtype, int bits, int group_size, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims,
+    int n_heavy_dims, int causal, int64_t q_offset, void *out, int out_dtype, void *workspace,
+    size_t workspace_bytes, int n_splits, const ss_attn_mask *mask, void *stream) {
+    SS_REQUIRE(t_buf >= 0, "negative buffer length");
+    return grouped_il_impl(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, scale, perm,
+                           codebook, n_blocks, n_centroids, idx, codes_il, scales, zeros, sz_dtype,
+                           bits, group_size, cap, t_kv, causal, q_offset, out, out_dtype, workspace,
+                           workspace_bytes, n_splits, k_buf, v_buf, buf_dtype, buf_sb, buf_sh,
+                           buf_st, t_buf, stream, k_heavy, heavy_dims, n_heavy_dims, mask);
+}
+
+static int decode_attn_turboquant_il_impl(
     const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
     int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
     int n_centroids, const uint8_t *idx, const uint32_t *codes_il, const float *norms,
     const float *levels, const float *rotation, int64_t cap, int64_t t_kv, const void *k_buf,
     const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh, int64_t buf_st, int64_t t_buf,
     const void *k_heavy, const int32_t *heavy_dims, int n_heavy_dims, int causal, int64_t q_offset,
-    void *out, int out_dtype, void *workspace, size_t workspace_bytes, int n_splits, void *stream) {
+    void *out, int out_dtype, void *workspace, size_t workspace_bytes, int n_splits,
+    const ss_attn_mask *mask, void *stream) {
     const float *cents = static_cast<const float *>(codebook);
     int rc = check_common(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, cents, n_blocks,
                           n_centroids, idx, cap, t_kv, out, out_dtype);
@@ -152,6 +172,12 @@ extern "C" int ss_decode_attn_turboquant_il(
             c.fused_merge = 0;
         const int hrc = set_heavy(c, k_heavy, heavy_dims, n_heavy_dims);
         if (hrc) return hrc;
+        if (c.mask_dt != kMaskNone) {
+            SS_UNSUPPORTED(c.nhd == 0, "a mask and fp16 heavy key dims are not taken together here");
+            if (head_dim == 128) return launch_mfma_masked<128, VTq<128>>(c, va128, s, st, false);
+            const typename VTq<64>::Args va64{va128.codes, va128.norms, va128.l0, va128.l1, va128.l2};
+            return launch_mfma_masked<64, VTq<64>>(c, va64, s, st, false);
+        }
         auto go = [&](auto dd, auto vf) -> int {
             constexpr int DD = decltype(dd)::value;
             using VF = typename decltype(vf)::type;
@@ -182,6 +208,7 @@ extern "C" int ss_decode_attn_turboquant_il(
                          head_dim);
         if (rc) return rc;
         SS_REQUIRE(((uintptr_t)rotation % 4) == 0, "misaligned rotation matrix");
+        if ((rc = set_mask(c, mask))) return rc;
         if (s.S == 1 || c.fused_merge)
             return launch_tq(c, s, reinterpret_cast<hipStream_t>(stream), true);
     }
@@ -191,5 +218,40 @@ extern "C" int ss_decode_attn_turboquant_il(
     return transformed_decode(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, scale, perm, cents,
                               n_centroids, idx, cap, t_kv, rotation, k_buf, v_buf, buf_dtype, buf_sb, buf_sh,
                               buf_st, t_buf, causal, q_offset, out, out_dtype, workspace, workspace_bytes,
-                              n_splits, stream, main, kKindMfma);
+                              n_splits, stream, main, kKindMfma, mask);
+}
+
+extern "C" int ss_decode_attn_turboquant_il(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint32_t *codes_il, const float *norms,
+    const float *levels, const float *rotation, int64_t cap, int64_t t_kv, const void *k_buf,
+    const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh, int64_t buf_st, int64_t t_buf,
+    const void *k_heavy, const int32_t *heavy_dims, int n_heavy_dims, int causal, int64_t q_offset,
+    void *out, int out_dtype, void *workspace, size_t workspace_bytes, int n_splits, void *stream) {
+    return decode_attn_turboquant_il_impl(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim,
+                                          scale, perm, codebook, n_blocks, n_centroids, idx,
+                                          codes_il, norms, levels, rotation, cap, t_kv, k_buf,
+                                          v_buf, buf_dtype, buf_sb, buf_sh, buf_st, t_buf, k_heavy,
+                                          heavy_dims, n_heavy_dims, causal, q_offset, out,
+                                          out_dtype, workspace, workspace_bytes, n_splits, nullptr,
+                                          stream);
+}
+
+extern "C" int ss_decode_attn_turboquant_il_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint32_t *codes_il, const float *norms,
+    const float *levels, const float *rotation, int64_t cap, int64_t t_kv, const void *k_buf,
+    const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh, int64_t buf_st, int64_t t_buf,
+    const void *k_heavy, const int32_t *heavy_dims, int n_heavy_dims, int causal, int64_t q_offset,
+    void *out, int out_dtype, void *workspace, size_t workspace_bytes, int n_splits,
+    const ss_attn_mask *mask, void *stream) {
+    return decode_attn_turboquant_il_impl(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim,
+                                          scale, perm, codebook, n_blocks, n_centroids, idx,
+                                          codes_il, norms, levels, rotation, cap, t_kv, k_buf,
+                                          v_buf, buf_dtype, buf_sb, buf_sh, buf_st, t_buf, k_heavy,
+                                          heavy_dims, n_heavy_dims, causal, q_offset, out,
+                                          out_dtype, workspace, workspace_bytes, n_splits, mask,
+                                          stream);
 }

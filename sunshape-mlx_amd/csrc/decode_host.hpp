@@ -112,7 +112,7 @@ static int mfma_kernel_setup() {
 
 template <int D, class VF>
 static int launch_mfma_kernel(DecodeCommon c, const typename VF::Args &va, const DecodeShape &s,
-                              hipStream_t st) {
+                              hipStream_t st, bool merge = true) {
     constexpr int NC = VF::kComputeWaves;
     using K = WsCfg<D, NC, VF>;
     auto kern = decode_attn_mfma_kernel<D, NC, VF>;
@@ -120,15 +120,27 @@ static int launch_mfma_kernel(DecodeCommon c, const typename VF::Args &va, const
     if (rc) return rc;
     hipLaunchKernelGGL(kern, dim3(s.S, s.n_cols), dim3(K::kWaves * kWave), K::kLds, st, c, va);
     SS_LAUNCH_CHECK("decode_attn_mfma_kernel launch");
-    if (c.fused_merge) return SS_OK;  // the kernel merges its splits itself
+    if (c.fused_merge || !merge) return SS_OK;  // the kernel (or the caller) merges the splits
     return launch_merge<D>(c, s, st);
 }
 
+// launch_mfma_kernel<D, WithMask<VF>>, compiled in decode_masked.hip for the
+// formats launch_mfma passes on
+template <int D, class VF>
+int launch_mfma_masked(const DecodeCommon &c, const typename VF::Args &va, const DecodeShape &s,
+                       hipStream_t st, bool merge = true);
+
 // the format's kernel, or its heavy-dim variant when the call carries fp16
-// heavy key dims
+// heavy key dims, or its masked one
 template <int D, class VF>
 static int launch_mfma(DecodeCommon c, const typename VF::Args &va, const DecodeShape &s,
                        hipStream_t st) {
+    if (c.mask_dt != kMaskNone) {
+        SS_UNSUPPORTED(c.nhd == 0, "a mask and fp16 heavy key dims are not taken together here");
+        if constexpr (!StepShareOf<VF>::value && !std::is_same<VF, VIl8<D>>::value)
+            return launch_mfma_masked<D, VF>(c, va, s, st);
+        SS_UNSUPPORTED(false, "this decode shape takes no mask");
+    }
     if (c.nhd > 0) {
         if constexpr (VfHeavyCapable<VF>::value)
             return launch_mfma_kernel<D, WithHeavy<VF>>(c, va, s, st);
@@ -137,10 +149,10 @@ static int launch_mfma(DecodeCommon c, const typename VF::Args &va, const Decode
     return launch_mfma_kernel<D, VF>(c, va, s, st);
 }
 
-template <int NH8>
+template <int NH8, bool MK = false>
 static int launch_sunv_mfma(const DecodeCommon &c, const typename VSunV<128, 4>::Args &va,
                             const DecodeShape &s, hipStream_t st) {
-    auto kern = sunv_mfma_kernel<NH8>;
+    auto kern = sunv_mfma_kernel<NH8, MK>;
     static bool attr_set = false;  // per instantiation
     if (!attr_set) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
@@ -153,6 +165,11 @@ static int launch_sunv_mfma(const DecodeCommon &c, const typename VSunV<128, 4>:
     SS_LAUNCH_CHECK("sunv_mfma_kernel launch");
     return SS_OK;
 }
+
+// launch_sunv_mfma<NH8, true>, compiled in decode_masked.hip
+template <int NH8>
+int launch_sunv_masked(const DecodeCommon &c, const typename VSunV<128, 4>::Args &va,
+                       const DecodeShape &s, hipStream_t st);
 
 template <int D, int R, class VF>
 static int launch(DecodeCommon c, const typename VF::Args &va, const DecodeShape &s,
@@ -197,6 +214,24 @@ static int check_common(const void *q, int q_dtype, int64_t batch, int hq, int h
                (long long)cap);
     SS_REQUIRE(((uintptr_t)idx % 16) == 0, "idx must be 16-byte aligned");
     SS_REQUIRE(((uintptr_t)centroids % 16) == 0, "centroids must be 16-byte aligned");
+    return SS_OK;
+}
+
+// A call's attention mask (null or data null: none).
+static int set_mask(DecodeCommon &c, const ss_attn_mask *mask) {
+    if (!mask || !mask->data) return SS_OK;
+    SS_REQUIRE(mask->type >= SS_MASK_BOOL && mask->type <= SS_MASK_F32, "bad mask type %d", mask->type);
+    SS_REQUIRE(mask->sb >= 0 && mask->sh >= 0 && mask->sq >= 0, "negative mask strides");
+    static_assert((int)kMaskBool == SS_MASK_BOOL && (int)kMaskF16 == SS_MASK_F16 &&
+                      (int)kMaskBf16 == SS_MASK_BF16 && (int)kMaskF32 == SS_MASK_F32, "mask types");
+    const int es = mask->type == SS_MASK_BOOL ? 1 : mask->type == SS_MASK_F32 ? 4 : 2;
+    SS_REQUIRE((uintptr_t)mask->data % es == 0, "mask not aligned to its elements");
+    SS_REQUIRE(!c.causal, "an array mask replaces the causal one");
+    c.mask = mask->data;
+    c.mask_dt = mask->type;
+    c.m_sb = mask->sb;
+    c.m_sh = mask->sh;
+    c.m_sq = mask->sq;
     return SS_OK;
 }
 
@@ -266,7 +301,8 @@ static int transformed_decode(const void *q, int q_dtype, int64_t batch, int hq,
                               int64_t buf_sb, int64_t buf_sh, int64_t buf_st, int64_t t_buf,
                               int causal, int64_t q_offset, void *out, int out_dtype,
                               void *workspace, size_t workspace_bytes, int n_splits,
-                              void *stream, MainLaunch &&launch_main, int kind = kKindValu) {
+                              void *stream, MainLaunch &&launch_main, int kind = kKindValu,
+                              const ss_attn_mask *mask = nullptr) {
     const bool ident = transform == nullptr;
     SS_REQUIRE(((uintptr_t)transform % 4) == 0, "misaligned transform/rotation matrix");
     SS_REQUIRE(t_buf >= 0, "negative buffer length");
@@ -294,6 +330,7 @@ static int transformed_decode(const void *q, int q_dtype, int64_t batch, int hq,
                          idx, cap, t_kv, causal, q_offset, ident ? out : y,
                          ident ? out_dtype : SS_F32, workspace, workspace_bytes, head_dim);
     if (rc) return rc;
+    if ((rc = set_mask(c, mask))) return rc;
     c.tiles_per_split = s.tiles_per_split;  // the compressed tokens' splits: grid s.S
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     rc = launch_main(c, s, st);  // no merge: it follows, with the buffer

@@ -73,7 +73,53 @@ struct DecodeCommon {
     // in-kernel merge): rows accumulated in a transformed basis leave as
     // y @ rot ([D][D] float32, row k = basis vector k); null: as they are
     const float *rot = nullptr;
+    // attention mask: element (b, head, query position, key position t) at
+    // mask[b*m_sb + head*m_sh + q*m_sq + t], kMask* type (kMaskNone: none)
+    const void *mask = nullptr;
+    int mask_dt = 0;
+    int64_t m_sb = 0, m_sh = 0, m_sq = 0;
 };
+enum MaskKind { kMaskNone = 0, kMaskBool = 1, kMaskF16 = 2, kMaskBf16 = 3, kMaskF32 = 4 };
+
+// Running maxima start at float32's lowest value, and a key that a boolean
+// mask hides scores exactly that (the reference fills with it,
+// attention.py:329-341): a row whose keys are all hidden then averages the
+// values, and one visible key outweighs any number of hidden ones.
+constexpr float kLowest = -3.402823466e38f;
+
+__device__ __forceinline__ uint32_t mask_load(const DecodeCommon &c, int64_t off) {
+    if (c.mask_dt == kMaskBool) return static_cast<const uint8_t *>(c.mask)[off];
+    if (c.mask_dt == kMaskF32) return static_cast<const uint32_t *>(c.mask)[off];
+    return static_cast<const uint16_t *>(c.mask)[off];
+}
+
+// A score in log2 units under mask element w (mask_load's bits), as hi + lo:
+// hidden or kept by a boolean, else the element added in natural units, where
+// the sum rounds as the reference's does (a mask of -1e9 absorbs the score in
+// float32, one of -65504 keeps its part above 2^-8).  hi is the sum in log2
+// units and lo what its rounding there left off, added back after the
+// running maximum is subtracted: a row hidden throughout by -65504 keeps the
+// reference's differences.  A finite sum stays finite, so float32's lowest
+// value hides as a boolean does; -inf and NaN keep their effect.
+__device__ __forceinline__ float mask_score(const DecodeCommon &c, uint32_t w, float s, float &lo) {
+    lo = 0.f;
+    if (c.mask_dt == kMaskBool) return w ? s : kLowest;
+    const float x = c.mask_dt == kMaskF32   ? __uint_as_float(w)
+                    : c.mask_dt == kMaskF16 ? __half2float(__ushort_as_half((unsigned short)w))
+                                            : __uint_as_float(w << 16);
+    const float y = fmaf(s, 0.6931471805599453f, x);
+    const float hi = y * kLog2e;
+    if (fabsf(hi) == INFINITY) return fabsf(y) == INFINITY ? y : (y < 0.f ? kLowest : -kLowest);
+    lo = fmaf(y, kLog2e, -hi);
+    return hi;
+}
+
+// What a row with no probability mass returns: zeros (an empty cache, a
+// causal row that sees no key), but under a mask NaN, as a softmax over
+// -inf or NaN scores does.
+__device__ __forceinline__ float no_mass(const DecodeCommon &c) {
+    return c.mask_dt != kMaskNone ? __uint_as_float(0x7fc00000u) : 0.f;
+}
 constexpr int kMaxHeavyMfma = 32;  // heavy dims the matrix-core kernels take
 
 // Bits of the wait-failure word: which bounded wait gave up.
@@ -417,6 +463,16 @@ template <class VF>
 struct WithHeavy : VF {
     static constexpr bool kHeavyMfma = true;
 };
+// A value format whose kernel applies an attention mask (WithMask): a
+// separate kernel for the same reason.
+template <class VF, class = void>
+struct VfMasked : std::false_type {};
+template <class VF>
+struct VfMasked<VF, std::void_t<decltype(VF::kMasked)>> : std::bool_constant<VF::kMasked> {};
+template <class VF>
+struct WithMask : VF {
+    static constexpr bool kMasked = true;
+};
 template <class T>
 struct TypeTag {
     using type = T;
@@ -650,10 +706,17 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
             lim[r] = INT64_MAX;
     }
 
+    int64_t mrow[R];  // the rows' mask offsets (a row past the last takes row 0's)
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int64_t gr = row_ok(r) ? (int64_t)rg * R + r : (int64_t)rg * R;
+        mrow[r] = bb * c.m_sb + (kvh * c.rep + gr / c.t_q) * c.m_sh + (gr % c.t_q) * c.m_sq;
+    }
+
     float m[R], l[R], acc[R][DPL];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        m[r] = -1e30f;
+        m[r] = kLowest;
         l[r] = 0.f;
 #pragma unroll
         for (int k = 0; k < DPL; ++k) acc[r][k] = 0.f;
@@ -672,6 +735,10 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
         const bool kok = tk < t_end;
         IdxRow<NB> ir;
         ir.load(idx_head + tk * NB, kok);
+        uint32_t mk[R];
+        if (c.mask_dt != kMaskNone)
+#pragma unroll
+            for (int r = 0; r < R; ++r) mk[r] = kok ? mask_load(c, mrow[r] + tk) : 0u;
 
         float s[R];
 #pragma unroll
@@ -702,6 +769,10 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
                 for (int r = 0; r < R; ++r) s[r] += hs[r];
             }
         }
+        float slo[R] = {};
+        if (c.mask_dt != kMaskNone)
+#pragma unroll
+            for (int r = 0; r < R; ++r) s[r] = mask_score(c, mk[r], s[r], slo[r]);
 #pragma unroll
         for (int r = 0; r < R; ++r) s[r] = (kok && tk <= lim[r]) ? s[r] : -INFINITY;
         // a tile whose scores stay at most kValuLag log2 units above the
@@ -724,7 +795,7 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
             for (int r = 0; r < R; ++r) {
                 const float mn = fmaxf(m[r], tmax[r]);
                 corr[r] = fast_exp2(m[r] - mn);
-                const float p = fast_exp2(s[r] - mn);
+                const float p = fast_exp2((s[r] - mn) + slo[r]);
                 l[r] = fmaf(l[r], corr[r], p);
                 m[r] = mn;
                 s[r] = p;
@@ -733,7 +804,7 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 corr[r] = 1.f;
-                s[r] = fast_exp2(s[r] - m[r]);
+                s[r] = fast_exp2((s[r] - m[r]) + slo[r]);
                 l[r] += s[r];
             }
         }
@@ -830,7 +901,7 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
     const int S = c.n_splits;
     for (int i = tid; i < R * DS; i += TH) {
         const int r = i / DS, d = i - r * DS, dd = slab * DS + d;
-        float M = -1e30f;
+        float M = kLowest;
 #pragma unroll
         for (int w = 0; w < WV; ++w) M = fmaxf(M, wm[w * R + r]);
         float L = 0.f, A = 0.f;
@@ -841,7 +912,7 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
             A = fmaf(wa[(w * R + r) * DS + d], f, A);
         }
         if (S == 1) {
-            if (row_ok(r)) store_from_f32(c.out, c.out_dtype, row_off(r) + dd, L > 0.f ? A / L : 0.f);
+            if (row_ok(r)) store_from_f32(c.out, c.out_dtype, row_off(r) + dd, L > 0.f ? A / L : no_mass(c));
         } else {
             const int64_t slot = ((int64_t)col * S + split) * R + r;
             c.part_acc[slot * D + dd] = A;
@@ -2150,14 +2221,37 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
     constexpr bool kRegs = VfRegUnits<VF>::value;
     constexpr float kLag = VfMaxLag<VF>::value;
     constexpr bool HV = VfHeavyMfma<VF>::value;
+    constexpr bool MK = VfMasked<VF>::value;  // an attention mask applies
+    constexpr int MKN = MK ? R : 1;
+    int64_t mrow[MKN];  // the rows' mask offsets (a row past the last takes row 0's)
+    if constexpr (MK)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int64_t gr = row_ok(r) ? (int64_t)rg * R + r : (int64_t)rg * R;
+            mrow[r] = bb * c.m_sb + (kvh * c.rep + gr / c.t_q) * c.m_sh + (gr % c.t_q) * c.m_sq;
+        }
+    // the mask elements of unit u's token `lane` (the split's last token past
+    // its end), loaded a unit ahead like the rest of the unit
+    struct MaskUnit {
+        uint32_t w[MKN];
+    };
+    auto load_mask = [&](MaskUnit &x, int u) {
+        if constexpr (MK) {
+            const int64_t tk = min(t_beg + (int64_t)u * kWave + lane, t_last);
+#pragma unroll
+            for (int r = 0; r < R; ++r) x.w[r] = mask_load(c, mrow[r] + tk);
+        }
+    };
     constexpr int HVN = HV ? kMaxHeavyMfma / 8 : 1;
     struct RegUnit {
         IdxRow<NB> ir;
         typename RawUnitOf<VF, kRegs>::type raw;
         uint4 khv[HVN];
+        MaskUnit mk;
     };
     auto load_ru = [&](RegUnit &x, int u) {
         if constexpr (kRegs) {
+            load_mask(x.mk, u);
             const int64_t t0 = t_beg + (int64_t)u * kWave;
             const int64_t tk = min(t0 + lane, t_last);
             x.ir.load(c.idx + (bh * c.cap + tk) * NB, true);
@@ -2173,6 +2267,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
         }
     };
     RegUnit ua, ub;
+    MaskUnit ring_mk;  // ring shapes: the mask of this wave's next unit
     // Wave w takes units w, w + NC, ... of the split.  Where wave 0 first
     // attends the split's share of buffered tokens (and, in a hybrid step,
     // scores the flushed tokens), it skips its first share_skip units, which
@@ -2229,7 +2324,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
     float m[R], lsum[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        m[r] = row_ok(r) ? -1e30f : 3e38f;
+        m[r] = row_ok(r) ? kLowest : 3e38f;
         lsum[r] = 0.f;
     }
 
@@ -2289,7 +2384,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
         float bm[R], bl[R], ba[R][DL];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            bm[r] = -1e30f;
+            bm[r] = kLowest;
             bl[r] = 0.f;
 #pragma unroll
             for (int k = 0; k < DL; ++k) ba[r][k] = 0.f;
@@ -2335,7 +2430,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                                 vc[j][k] = hv_raw[j][k];
                             }
                         }
-                    float sc[NSH][R];
+                    float sc[NSH][R], blo[NSH][MKN] = {};
 #pragma unroll
                     for (int j = 0; j < NSH; ++j) {
                         float part[R];
@@ -2348,8 +2443,14 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                         wave_sum4_dpp(part, sc[j]);
                         const int64_t pos = ex_pos0 + bj0 + c0 + j;
 #pragma unroll
-                        for (int r = 0; r < R; ++r)
-                            sc[j][r] = (c0 + j < n_sh && pos <= lim[r]) ? sc[j][r] * kLog2e : -INFINITY;
+                        for (int r = 0; r < R; ++r) {
+                            sc[j][r] *= kLog2e;
+                            if constexpr (MK)
+                                sc[j][r] =
+                                    mask_score(c, mask_load(c, mrow[r] + min(pos, c.t_kv + t_buf - 1)),
+                                               sc[j][r], blo[j][r]);
+                            sc[j][r] = (c0 + j < n_sh && pos <= lim[r]) ? sc[j][r] : -INFINITY;
+                        }
                     }
 #pragma unroll
                     for (int r = 0; r < R; ++r) {
@@ -2365,7 +2466,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                         for (int k = 0; k < DLh; ++k) ba[r][k] *= corr;
 #pragma unroll
                         for (int j = 0; j < NSH; ++j) {
-                            const float pj = fast_exp2(sc[j][r] - mn);
+                            const float pj = fast_exp2(MK ? (sc[j][r] - mn) + blo[j][r % MKN] : sc[j][r] - mn);
                             bl[r] += pj;
 #pragma unroll
                             for (int k = 0; k < DLh; ++k) ba[r][k] = fmaf(pj, f32(vc[j][k]), ba[r][k]);
@@ -2408,6 +2509,12 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                 for (int r = 0; r < R; ++r) sc[r] *= kLog2e;
             }
             const int64_t pos = (kStepOnly ? c.t_kv : ex_pos0) + j;
+            float blo[MKN] = {};
+            if constexpr (MK)
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    sc[r] = mask_score(c, mask_load(c, mrow[r] + min(pos, c.t_kv + t_buf - 1)), sc[r],
+                                       blo[r]);
 #pragma unroll
             for (int r = 0; r < R; ++r) sc[r] = (ok && pos <= lim[r]) ? sc[r] : -INFINITY;
             float tmax[R], p[R], corr[R];
@@ -2416,7 +2523,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
             for (int r = 0; r < R; ++r) {
                 const float mn = fmaxf(bm[r], tmax[r]);
                 corr[r] = fast_exp2(bm[r] - mn);
-                p[r] = fast_exp2(sc[r] - mn);
+                p[r] = fast_exp2(MK ? (sc[r] - mn) + blo[r % MKN] : sc[r] - mn);
                 bm[r] = mn;
             }
             float ps[R];
@@ -2748,7 +2855,10 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
             // this wave's first unit streams into registers while the LUT is built
             const int u0 = unit_of(0);
             if (u0 < n_units) load_ru(ua, u0);
-        } else if constexpr (K::kPriv) {
+        } else if constexpr (MK) {
+            if (wv < n_units) load_mask(ring_mk, wv);
+        }
+        if constexpr (!kRegs && K::kPriv) {
             // this wave's first units (u = wv + k*NC) stream in while the LUT is built
             for (; nq < K::kPrivSlots && wv + nq * NC < n_units; ++nq)
                 issue_at(wv + nq * NC, ring_l + priv_slot(nq));
@@ -3173,7 +3283,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
         _Float16 *pw = pst + wv * VF::kPRows * kPStride;
         // one 64-token unit of this wave: scores, online softmax, P.V
         auto step = [&](const IdxRow<NB> &ir, typename VF::Tile &tv, const uint4 (&khv)[HVN],
-                        int u) __attribute__((always_inline)) {
+                        const MaskUnit &mk, int u) __attribute__((always_inline)) {
             const int64_t t0 = t_beg + (int64_t)u * kWave;
             // tokens of this tile still inside the split (wave-uniform, 1..64)
             const int n_in = (int)min(t_end - t0, (int64_t)kWave);
@@ -3215,6 +3325,10 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                     for (int r = 0; r < R; ++r) sc[r] += hv[r];
                 }
             }
+            float mlo[MKN] = {};
+            if constexpr (MK)
+#pragma unroll
+                for (int r = 0; r < R; ++r) sc[r] = mask_score(c, mk.w[r], sc[r], mlo[r]);
             // A whole tile every row sees (no causal cut, no split end) whose
             // scores all stay at most kLag above the rows' running maxima
             // keeps the maxima: no reduction, no rescale (its probabilities
@@ -3245,7 +3359,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                 for (int r = 0; r < R; ++r) {
                     const float mn = fmaxf(m[r], tmax[r]);
                     corr[r] = fast_exp2(m[r] - mn);
-                    p[r] = fast_exp2(sc[r] - mn);
+                    p[r] = fast_exp2(MK ? (sc[r] - mn) + mlo[r % MKN] : sc[r] - mn);
                     lsum[r] = fmaf(lsum[r], corr[r], p[r]);
                     m[r] = mn;
                 }
@@ -3253,7 +3367,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     corr[r] = 1.f;
-                    p[r] = fast_exp2(sc[r] - m[r]);
+                    p[r] = fast_exp2(MK ? (sc[r] - m[r]) + mlo[r % MKN] : sc[r] - m[r]);
                     lsum[r] += p[r];
                 }
             }
@@ -3268,7 +3382,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                 {
                     typename VF::Tile tv;
                     VF::from_raw(tv, ua.raw, lane);
-                    step(ua.ir, tv, ua.khv, u);
+                    step(ua.ir, tv, ua.khv, ua.mk, u);
                 }
                 if (u1 >= n_units) break;
                 const int u2 = unit_of(++i);
@@ -3276,7 +3390,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                 {
                     typename VF::Tile tv;
                     VF::from_raw(tv, ub.raw, lane);
-                    step(ub.ir, tv, ub.khv, u1);
+                    step(ub.ir, tv, ub.khv, ub.mk, u1);
                 }
                 u = u2;
             }
@@ -3335,7 +3449,10 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
             } else {
                 if (lane == 0) done[slot * K::kSub + sub] = j;
             }
-            step(ir, tv, khv, u);
+            const MaskUnit mk = ring_mk;
+            if constexpr (MK)
+                if (u + NC < n_units) load_mask(ring_mk, u + NC);
+            step(ir, tv, khv, mk, u);
         }
         }
     }
@@ -3382,10 +3499,10 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
             hi[w] = wa4[(((w * 2 + 0) * R + r) * D + d0) / 4];
             lo[w] = wa4[(((w * 2 + 1) * R + r) * D + d0) / 4];
         }
-        M = -1e30f;
+        M = kLowest;
 #pragma unroll
         for (int w = 0; w < NC; ++w) M = fmaxf(M, mw[w]);
-        float mb = -1e30f, lb = 0.f;
+        float mb = kLowest, lb = 0.f;
         f32x4 ab = f32x4{0.f, 0.f, 0.f, 0.f};
         if (has_buf) {  // the split's share of the token buffer
             mb = bpart[r];
@@ -3441,7 +3558,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
             float M, L;
             f32x4 A;
             combine4(r, d0, M, L, A);
-            const float iv = L > 0.f ? 1.f / L : 0.f;
+            const float iv = L > 0.f ? 1.f / L : (MK ? no_mass(c) : 0.f);
             put4(r, d0, A * iv);
         }
         rot_rows();
@@ -3494,7 +3611,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
     if (kMergeParts >= 2 && S <= kMergeParts * kMergeLoads) {
         const int cidx = tid % CH, part = tid / CH;
         const int mr = cidx / (D / 4), md0 = (cidx - mr * (D / 4)) * 4;
-        float Mr = -1e30f, Lr = 0.f;
+        float Mr = kLowest, Lr = 0.f;
         f32x4 Ar = f32x4{0.f, 0.f, 0.f, 0.f};
         if (part < kMergeParts) {
             f32x4 av[kMergeLoads];
@@ -3541,7 +3658,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                 Lr = Lr * fo + l2 * fn;
                 Mr = Mn;
             }
-            const float iv = Lr > 0.f ? 1.f / Lr : 0.f;
+            const float iv = Lr > 0.f ? 1.f / Lr : (MK ? no_mass(c) : 0.f);
             put4(mr, md0, Ar * iv);
         }
         rot_rows();
@@ -3594,7 +3711,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
     __syncthreads();
     if (wv < R) {  // wave r: weights exp2(m_s - M) and the merged l of row r
         const int r = wv;
-        float M = -1e30f;
+        float M = kLowest;
         for (int s2 = lane; s2 < S; s2 += kWave) M = fmaxf(M, __uint_as_float(mlb[s2 * R + r][0]));
         M = wave_max(M);
         float L = 0.f;
@@ -3635,7 +3752,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
     if (tid < CH4) {
         const float L = lrow[mr];
         const f32x4 A = acc0 + acc1;
-        const float iv = L > 0.f ? 1.f / L : 0.f;
+        const float iv = L > 0.f ? 1.f / L : (MK ? no_mass(c) : 0.f);
         put4(mr, md0, A * iv);
     }
     rot_rows();
@@ -3702,14 +3819,15 @@ __device__ __forceinline__ f16x4 ds_read_tr16(const char *lds_base, uint32_t off
     return ds_read_tr16_at(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds_base)) + off);
 }
 
-template <int NH8>
+template <int NH8, bool MK>
 struct SvUnit {
     uint4 k;                          // key index row of token t0 + lane
     uint4 kh[NH8 > 0 ? NH8 : 1];      // its heavy key dims (fp16)
     uint2 vi[4];                      // value index bytes 8*(l16%4) .. +7 of token 16ks + 4g + l16/4
+    uint32_t mk[MK ? kMfmaRows : 1];  // the rows' mask elements of token t0 + lane
 };
 
-template <int NH8>
+template <int NH8, bool MK>
 __global__ void __launch_bounds__(kSvWaves * kWave)
     sunv_mfma_kernel(DecodeCommon c, typename VSunV<128, 4>::Args va) {
     constexpr int NC = kSvWaves, TH = NC * kWave, R = kMfmaRows, D = kSvD;
@@ -3874,11 +3992,21 @@ __global__ void __launch_bounds__(kSvWaves * kWave)
     const char *kh_b = reinterpret_cast<const char *>(va.kheavy + (NH8 > 0 ? vrow0 * (NH8 * 8) : 0));
     const char *vi_b = reinterpret_cast<const char *>(va.idx + vrow0 * kSvNBV);
     const uint32_t t_last32 = (uint32_t)t_last;
+    int64_t mrow[MK ? R : 1];  // the rows' mask offsets (a row past the last takes row 0's)
+    if constexpr (MK)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int64_t gr = row_ok(r) ? (int64_t)rg * R + r : (int64_t)rg * R;
+            mrow[r] = bb * c.m_sb + (kvh * c.rep + gr / c.t_q) * c.m_sh + (gr % c.t_q) * c.m_sq;
+        }
     auto at = [](const char *base, uint32_t byte_off) { return base + byte_off; };
-    auto load_unit = [&](SvUnit<NH8> &U, int u) {
+    auto load_unit = [&](SvUnit<NH8, MK> &U, int u) {
         const uint32_t t0 = (uint32_t)t_beg + (uint32_t)u * kWave;
         const uint32_t tk = min(t0 + (uint32_t)lane, t_last32);
         U.k = *reinterpret_cast<const uint4 *>(at(kidx_b, tk * kSvNB));
+        if constexpr (MK)
+#pragma unroll
+            for (int r = 0; r < R; ++r) U.mk[r] = mask_load(c, mrow[r] + tk);
         if constexpr (NH8 > 0) {
 #pragma unroll
             for (int j = 0; j < NH8; ++j)
@@ -3895,14 +4023,14 @@ __global__ void __launch_bounds__(kSvWaves * kWave)
     f32x4 acc[8];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        m[r] = -1e30f;
+        m[r] = kLowest;
         lsum[r] = 0.f;
     }
 #pragma unroll
     for (int nt = 0; nt < 8; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
     _Float16 *pw = pst + wv * 8 * kPStride;
 
-    auto compute_unit = [&](const SvUnit<NH8> &cur, int u) {
+    auto compute_unit = [&](const SvUnit<NH8, MK> &cur, int u) {
         const int64_t t0 = t_beg + (int64_t)u * kWave;
         const int n_in = (int)min(t_end - t0, (int64_t)kWave);
         // scores: the 16 LUT reads in flight at once, then a tree sum
@@ -3941,6 +4069,10 @@ __global__ void __launch_bounds__(kSvWaves * kWave)
             s4 += (hs + hl * (1.f / kSplitScale)) * (qsc * kLog2e);
         }
         float sc[R] = {s4.x, s4.y, s4.z, s4.w};
+        float mlo[R] = {};
+        if constexpr (MK)
+#pragma unroll
+            for (int r = 0; r < R; ++r) sc[r] = mask_score(c, cur.mk[r], sc[r], mlo[r]);
         bool moved = true;
         if (n_in == kWave && t0 + (kWave - 1) <= lim_min) {
             uint64_t above = 0;
@@ -3963,7 +4095,7 @@ __global__ void __launch_bounds__(kSvWaves * kWave)
             for (int r = 0; r < R; ++r) {
                 const float mn = fmaxf(m[r], tmax[r]);
                 corr[r] = fast_exp2(m[r] - mn);
-                p[r] = fast_exp2(sc[r] - mn);
+                p[r] = fast_exp2(MK ? (sc[r] - mn) + mlo[r] : sc[r] - mn);
                 lsum[r] = fmaf(lsum[r], corr[r], p[r]);
                 m[r] = mn;
             }
@@ -3971,7 +4103,7 @@ __global__ void __launch_bounds__(kSvWaves * kWave)
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 corr[r] = 1.f;
-                p[r] = fast_exp2(sc[r] - m[r]);
+                p[r] = fast_exp2(MK ? (sc[r] - m[r]) + mlo[r] : sc[r] - m[r]);
                 lsum[r] += p[r];
             }
         }
@@ -4029,7 +4161,7 @@ __global__ void __launch_bounds__(kSvWaves * kWave)
     };
     // two register sets in turn: the next unit's loads are issued before the
     // current unit is computed
-    SvUnit<NH8> ua, ub;
+    SvUnit<NH8, MK> ua, ub;
     if (wv < n_units) load_unit(ua, wv);
     for (int u = wv; u < n_units; u += 2 * NC) {
         load_unit(ub, min(u + NC, n_units - 1));
@@ -4071,7 +4203,7 @@ __global__ void __launch_bounds__(kSvWaves * kWave)
     const int S = c.n_splits;
     for (int i = tid; i < R * D; i += TH) {
         const int r = i / D, d = i - r * D;
-        float M = -1e30f;
+        float M = kLowest;
 #pragma unroll
         for (int w = 0; w < NC; ++w) M = fmaxf(M, wm[w * R + r]);
         float L = 0.f, A = 0.f;
@@ -4087,7 +4219,7 @@ __global__ void __launch_bounds__(kSvWaves * kWave)
             A = fmaf(8.f * sc, A, (z + (8.f * kSvCodeOff) * sc) * L);
         }
         if (S == 1) {
-            if (row_ok(r)) store_from_f32(c.out, c.out_dtype, row_off(r) + d, L > 0.f ? A / L : 0.f);
+            if (row_ok(r)) store_from_f32(c.out, c.out_dtype, row_off(r) + d, L > 0.f ? A / L : no_mass(c));
         } else {
             const int64_t slot = ((int64_t)col * S + split) * R + r;
             c.part_acc[slot * D + d] = A;
@@ -4166,9 +4298,9 @@ __global__ void __launch_bounds__(kDecodeThreads)
     constexpr int LPT = D / 8;                    // lanes per token
     constexpr int TPG = kDecodeThreads / LPT;     // tokens per pass of the workgroup
     constexpr int BT = 128, PASSES = BT / TPG;    // tokens of a chunk
-    __shared__ float bp[BUF ? BT : 1];
+    __shared__ float bp[BUF ? BT : 1], bplo[BUF ? BT : 1];  // scores, and what a mask left off
     __shared__ float bacc[BUF ? kDecodeThreads / kWave : 1][BUF ? D : 1];
-    float bm = -1e30f, bl = 0.f;
+    float bm = kLowest, bl = 0.f;
     if constexpr (BUF) {
         const int dl = tid % LPT, tg = tid / LPT;  // dims 8*dl .. +7 of tokens tg + i*TPG
         float qv[8], ba[8];
@@ -4181,6 +4313,7 @@ __global__ void __launch_bounds__(kDecodeThreads)
         const int64_t lim = c.causal ? c.q_offset + tq - c.t_kv + 1 : mb.n;
         const int64_t n = min(mb.n, lim);
         const int64_t base = bb * mb.sb + kvh * mb.sh + dl * 8;
+        const int64_t mrow = bb * c.m_sb + (kvh * c.rep + rr) * c.m_sh + tq * c.m_sq;
         for (int64_t j0 = 0; j0 < n; j0 += BT) {
             float kx[PASSES][8], vx[PASSES][8];
 #pragma unroll
@@ -4197,18 +4330,25 @@ __global__ void __launch_bounds__(kDecodeThreads)
 #pragma unroll
                 for (int o = LPT / 2; o > 0; o >>= 1) a += __shfl_xor(a, o);
                 const int tl = tg + i * TPG;
-                if (dl == 0) bp[tl] = j0 + tl < n ? a : -INFINITY;
+                if (dl == 0) {
+                    float lo = 0.f;
+                    if (c.mask_dt != kMaskNone && j0 + tl < n)
+                        a = mask_score(c, mask_load(c, mrow + c.t_kv + j0 + tl), a, lo);
+                    bp[tl] = j0 + tl < n ? a : -INFINITY;
+                    bplo[tl] = lo;
+                }
             }
             __syncthreads();
             float mx = wave_max(fmaxf(bp[lane], bp[lane + kWave]));
             const float mn = fmaxf(bm, mx), corr = fast_exp2(bm - mn);
             bm = mn;
-            bl = fmaf(bl, corr, wave_sum(fast_exp2(bp[lane] - mn) + fast_exp2(bp[lane + kWave] - mn)));
+            auto prob = [&](int i) { return fast_exp2((bp[i] - mn) + bplo[i]); };
+            bl = fmaf(bl, corr, wave_sum(prob(lane) + prob(lane + kWave)));
 #pragma unroll
             for (int e = 0; e < 8; ++e) ba[e] *= corr;
 #pragma unroll
             for (int i = 0; i < PASSES; ++i) {
-                const float p = fast_exp2(bp[tg + i * TPG] - mn);
+                const float p = prob(tg + i * TPG);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) ba[e] = fmaf(p, vx[i][e], ba[e]);
             }
@@ -4281,7 +4421,7 @@ __global__ void __launch_bounds__(kDecodeThreads)
             const float4 v = red[p * CH + chunk];
             A += (d & 3) == 0 ? v.x : (d & 3) == 1 ? v.y : (d & 3) == 2 ? v.z : v.w;
         }
-        const float y = lsh > 0.f ? A / lsh : 0.f;
+        const float y = lsh > 0.f ? A / lsh : no_mass(c);
         if (rot)
             yrow[d] = y;
         else

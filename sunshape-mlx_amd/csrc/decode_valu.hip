@@ -99,7 +99,7 @@ extern "C" int ss_decode_attn_grouped(const void *q, int q_dtype, int64_t batch,
                           zeros, sz_dtype, bits, group_size, true);
 }
 
-extern "C" int ss_decode_attn_turboquant(
+static int decode_attn_turboquant_impl(
     const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
     int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
     int n_centroids, const uint8_t *idx, const uint32_t *packed, const float *norms,
@@ -107,7 +107,7 @@ extern "C" int ss_decode_attn_turboquant(
     const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
     int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims, int n_heavy_dims,
     int causal, int64_t q_offset, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
-    int n_splits, void *stream) {
+    int n_splits, const ss_attn_mask *mask, void *stream) {
     int rc = check_common(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, centroids,
                           n_blocks, n_centroids, idx, cap, t_kv, out, out_dtype);
     if (rc) return rc;
@@ -146,17 +146,52 @@ extern "C" int ss_decode_attn_turboquant(
     return transformed_decode(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, scale, perm,
                               centroids, n_centroids, idx, cap, t_kv, rotation, k_buf, v_buf,
                               buf_dtype, buf_sb, buf_sh, buf_st, t_buf, causal, q_offset, out,
-                              out_dtype, workspace, workspace_bytes, n_splits, stream, main);
+                              out_dtype, workspace, workspace_bytes, n_splits, stream, main,
+                              kKindValu, mask);
 }
 
-extern "C" int ss_decode_attn_grouped_hybrid(
+extern "C" int ss_decode_attn_turboquant(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint32_t *packed, const float *norms,
+    const float *levels, const float *rotation, int bits, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims, int n_heavy_dims,
+    int causal, int64_t q_offset, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
+    int n_splits, void *stream) {
+    return decode_attn_turboquant_impl(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim,
+                                       scale, perm, centroids, n_blocks, n_centroids, idx, packed,
+                                       norms, levels, rotation, bits, cap, t_kv, k_buf, v_buf,
+                                       buf_dtype, buf_sb, buf_sh, buf_st, t_buf, k_heavy,
+                                       heavy_dims, n_heavy_dims, causal, q_offset, out, out_dtype,
+                                       workspace, workspace_bytes, n_splits, nullptr, stream);
+}
+
+extern "C" int ss_decode_attn_turboquant_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint32_t *packed, const float *norms,
+    const float *levels, const float *rotation, int bits, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims, int n_heavy_dims,
+    int causal, int64_t q_offset, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
+    int n_splits, const ss_attn_mask *mask, void *stream) {
+    return decode_attn_turboquant_impl(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim,
+                                       scale, perm, centroids, n_blocks, n_centroids, idx, packed,
+                                       norms, levels, rotation, bits, cap, t_kv, k_buf, v_buf,
+                                       buf_dtype, buf_sb, buf_sh, buf_st, t_buf, k_heavy,
+                                       heavy_dims, n_heavy_dims, causal, q_offset, out, out_dtype,
+                                       workspace, workspace_bytes, n_splits, mask, stream);
+}
+
+static int decode_attn_grouped_hybrid_impl(
     const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
     int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
     int n_centroids, const uint8_t *idx, const uint32_t *packed, const void *scales,
     const void *zeros, int sz_dtype, int bits, int group_size, int64_t cap, int64_t t_kv,
     const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
     int64_t buf_st, int64_t t_buf, int causal, int64_t q_offset, void *out, int out_dtype,
-    void *workspace, size_t workspace_bytes, int n_splits, void *stream) {
+    void *workspace, size_t workspace_bytes, int n_splits, const ss_attn_mask *mask, void *stream) {
     int rc = check_common(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, centroids,
                           n_blocks, n_centroids, idx, cap, t_kv, out, out_dtype);
     if (rc) return rc;
@@ -169,16 +204,49 @@ extern "C" int ss_decode_attn_grouped_hybrid(
     return transformed_decode(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, scale, perm,
                               centroids, n_centroids, idx, cap, t_kv, nullptr, k_buf, v_buf,
                               buf_dtype, buf_sb, buf_sh, buf_st, t_buf, causal, q_offset, out,
-                              out_dtype, workspace, workspace_bytes, n_splits, stream, main);
+                              out_dtype, workspace, workspace_bytes, n_splits, stream, main,
+                              kKindValu, mask);
 }
 
-extern "C" int ss_decode_attn_dense_hybrid(
+extern "C" int ss_decode_attn_grouped_hybrid(
     const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
     int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
-    int n_centroids, const uint8_t *idx, const void *values, int v_dtype, int64_t cap,
-    int64_t t_kv, const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb,
-    int64_t buf_sh, int64_t buf_st, int64_t t_buf, int causal, int64_t q_offset, void *out,
-    int out_dtype, void *workspace, size_t workspace_bytes, int n_splits, void *stream) {
+    int n_centroids, const uint8_t *idx, const uint32_t *packed, const void *scales,
+    const void *zeros, int sz_dtype, int bits, int group_size, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, int causal, int64_t q_offset, void *out, int out_dtype,
+    void *workspace, size_t workspace_bytes, int n_splits, void *stream) {
+    return decode_attn_grouped_hybrid_impl(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim,
+                                           scale, perm, centroids, n_blocks, n_centroids, idx,
+                                           packed, scales, zeros, sz_dtype, bits, group_size, cap,
+                                           t_kv, k_buf, v_buf, buf_dtype, buf_sb, buf_sh, buf_st,
+                                           t_buf, causal, q_offset, out, out_dtype, workspace,
+                                           workspace_bytes, n_splits, nullptr, stream);
+}
+
+extern "C" int ss_decode_attn_grouped_hybrid_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint32_t *packed, const void *scales,
+    const void *zeros, int sz_dtype, int bits, int group_size, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, int causal, int64_t q_offset, void *out, int out_dtype,
+    void *workspace, size_t workspace_bytes, int n_splits, const ss_attn_mask *mask, void *stream) {
+    return decode_attn_grouped_hybrid_impl(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim,
+                                           scale, perm, centroids, n_blocks, n_centroids, idx,
+                                           packed, scales, zeros, sz_dtype, bits, group_size, cap,
+                                           t_kv, k_buf, v_buf, buf_dtype, buf_sb, buf_sh, buf_st,
+                                           t_buf, causal, q_offset, out, out_dtype, workspace,
+                                           workspace_bytes, n_splits, mask, stream);
+}
+
+static int decode_attn_dense_hybrid_impl(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
+    int n_centroids, const uint8_t *idx, const void *values, int v_dtype, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, int causal, int64_t q_offset, void *out, int out_dtype,
+    void *workspace, size_t workspace_bytes, int n_splits, const ss_attn_mask *mask, void *stream) {
     int rc = check_common(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, centroids,
                           n_blocks, n_centroids, idx, cap, t_kv, out, out_dtype);
     if (rc) return rc;
@@ -189,18 +257,47 @@ extern "C" int ss_decode_attn_dense_hybrid(
     return transformed_decode(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, scale, perm,
                               centroids, n_centroids, idx, cap, t_kv, nullptr, k_buf, v_buf,
                               buf_dtype, buf_sb, buf_sh, buf_st, t_buf, causal, q_offset, out,
-                              out_dtype, workspace, workspace_bytes, n_splits, stream, main);
+                              out_dtype, workspace, workspace_bytes, n_splits, stream, main,
+                              kKindValu, mask);
 }
 
-extern "C" int ss_decode_attn_sunshape_v(
+extern "C" int ss_decode_attn_dense_hybrid(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
+    int n_centroids, const uint8_t *idx, const void *values, int v_dtype, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, int causal, int64_t q_offset, void *out, int out_dtype,
+    void *workspace, size_t workspace_bytes, int n_splits, void *stream) {
+    return decode_attn_dense_hybrid_impl(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim,
+                                         scale, perm, centroids, n_blocks, n_centroids, idx, values,
+                                         v_dtype, cap, t_kv, k_buf, v_buf, buf_dtype, buf_sb,
+                                         buf_sh, buf_st, t_buf, causal, q_offset, out, out_dtype,
+                                         workspace, workspace_bytes, n_splits, nullptr, stream);
+}
+
+extern "C" int ss_decode_attn_dense_hybrid_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
+    int n_centroids, const uint8_t *idx, const void *values, int v_dtype, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, int causal, int64_t q_offset, void *out, int out_dtype,
+    void *workspace, size_t workspace_bytes, int n_splits, const ss_attn_mask *mask, void *stream) {
+    return decode_attn_dense_hybrid_impl(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim,
+                                         scale, perm, centroids, n_blocks, n_centroids, idx, values,
+                                         v_dtype, cap, t_kv, k_buf, v_buf, buf_dtype, buf_sb,
+                                         buf_sh, buf_st, t_buf, causal, q_offset, out, out_dtype,
+                                         workspace, workspace_bytes, n_splits, mask, stream);
+}
+
+static int decode_attn_sunshape_v_impl(
     const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
     int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
     int n_centroids, const uint8_t *idx, const uint8_t *v_idx, const float *v_centroids,
     int v_block_dim, int v_n_centroids, const float *v_transform, const void *k_heavy,
-    const int32_t *heavy_dims, int n_heavy_dims, int64_t cap, int64_t t_kv,
-    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
-    int64_t buf_st, int64_t t_buf, int causal, int64_t q_offset, void *out, int out_dtype,
-    void *workspace, size_t workspace_bytes, int n_splits, void *stream) {
+    const int32_t *heavy_dims, int n_heavy_dims, int64_t cap, int64_t t_kv, const void *k_buf,
+    const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh, int64_t buf_st, int64_t t_buf,
+    int causal, int64_t q_offset, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
+    int n_splits, const ss_attn_mask *mask, void *stream) {
     int rc = check_common(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim, centroids,
                           n_blocks, n_centroids, idx, cap, t_kv, out, out_dtype);
     if (rc) return rc;
@@ -229,6 +326,15 @@ extern "C" int ss_decode_attn_sunshape_v(
             const typename VSunV<128, 4>::Args va{v_idx, v_centroids, v_n_centroids,
                                                   static_cast<const __half *>(k_heavy),
                                                   heavy_dims, k_heavy ? n_heavy_dims : 0};
+            if (c.mask_dt != kMaskNone) {
+                switch (nh8) {
+                    case 1: return launch_sunv_masked<1>(c, va, s, st);
+                    case 2: return launch_sunv_masked<2>(c, va, s, st);
+                    case 4: return launch_sunv_masked<4>(c, va, s, st);
+                    case 8: return launch_sunv_masked<8>(c, va, s, st);
+                    default: return launch_sunv_masked<0>(c, va, s, st);
+                }
+            }
             switch (nh8) {
                 case 1: return launch_sunv_mfma<1>(c, va, s, st);
                 case 2: return launch_sunv_mfma<2>(c, va, s, st);
@@ -259,5 +365,41 @@ extern "C" int ss_decode_attn_sunshape_v(
                               centroids, n_centroids, idx, cap, t_kv, v_transform, k_buf, v_buf,
                               buf_dtype, buf_sb, buf_sh, buf_st, t_buf, causal, q_offset, out,
                               out_dtype, workspace, workspace_bytes, n_splits, stream, main,
-                              sv_mfma ? kKindSunv : kKindValu);
+                              sv_mfma ? kKindSunv : kKindValu, mask);
+}
+
+extern "C" int ss_decode_attn_sunshape_v(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint8_t *v_idx, const float *v_centroids,
+    int v_block_dim, int v_n_centroids, const float *v_transform, const void *k_heavy,
+    const int32_t *heavy_dims, int n_heavy_dims, int64_t cap, int64_t t_kv, const void *k_buf,
+    const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh, int64_t buf_st, int64_t t_buf,
+    int causal, int64_t q_offset, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
+    int n_splits, void *stream) {
+    return decode_attn_sunshape_v_impl(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim,
+                                       scale, perm, centroids, n_blocks, n_centroids, idx, v_idx,
+                                       v_centroids, v_block_dim, v_n_centroids, v_transform,
+                                       k_heavy, heavy_dims, n_heavy_dims, cap, t_kv, k_buf, v_buf,
+                                       buf_dtype, buf_sb, buf_sh, buf_st, t_buf, causal, q_offset,
+                                       out, out_dtype, workspace, workspace_bytes, n_splits,
+                                       nullptr, stream);
+}
+
+extern "C" int ss_decode_attn_sunshape_v_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint8_t *v_idx, const float *v_centroids,
+    int v_block_dim, int v_n_centroids, const float *v_transform, const void *k_heavy,
+    const int32_t *heavy_dims, int n_heavy_dims, int64_t cap, int64_t t_kv, const void *k_buf,
+    const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh, int64_t buf_st, int64_t t_buf,
+    int causal, int64_t q_offset, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
+    int n_splits, const ss_attn_mask *mask, void *stream) {
+    return decode_attn_sunshape_v_impl(q, q_dtype, batch, n_q_heads, n_kv_heads, t_q, head_dim,
+                                       scale, perm, centroids, n_blocks, n_centroids, idx, v_idx,
+                                       v_centroids, v_block_dim, v_n_centroids, v_transform,
+                                       k_heavy, heavy_dims, n_heavy_dims, cap, t_kv, k_buf, v_buf,
+                                       buf_dtype, buf_sb, buf_sh, buf_st, t_buf, causal, q_offset,
+                                       out, out_dtype, workspace, workspace_bytes, n_splits, mask,
+                                       stream);
 }

@@ -9,7 +9,8 @@ import pytest
 import torch
 
 from oracle import sunshape_oracle as O
-from sunshape_mlx_amd import _hip
+import sunshape_mlx_amd as S
+from sunshape_mlx_amd import _hip, attention
 from test_gpu_kernels import REL_TOL, decode_case, rel_err, t
 
 pytestmark = pytest.mark.gpu
@@ -100,3 +101,68 @@ def test_decode_bf16_values_on_the_matrix_cores(b, hq, hkv, d, t_kv, t_buf, t_q,
                           kb[:, :, :t_buf].float().numpy() if t_buf else None, v_all,
                           mask="causal" if t_q > 1 else None)
     assert rel_err(out.cpu().numpy(), ref) <= REL_TOL
+
+
+def _masked_cache(backend, bits, dtype, d, hkv, b, t_kv, buffer):
+    rng = np.random.default_rng(t_kv + bits)
+    codec = S.SunShapeBlockCodec(d, device="cuda")
+    codec.load_state_dict({"centroids": rng.standard_normal((d // 8, 256, 8)).astype(np.float32),
+                           "permutation": rng.permutation(d).astype(np.int32)})
+    kw = {}
+    if backend == "sunshape":
+        vc = S.SunShapeBlockCodec(d, block_dim=4, device="cuda")
+        vc.load_state_dict({"centroids": rng.standard_normal((d // 4, 256, 4)).astype(np.float32),
+                            "permutation": rng.permutation(d).astype(np.int32)})
+        kw["value_codec"] = vc
+    cache = S.create_kv_cache(codec, n_kv_heads=hkv, dtype=dtype, value_backend=backend,
+                              value_bits=bits or None, buffer_size=buffer, **kw)
+    g = torch.Generator(device="cuda").manual_seed(t_kv)
+    k = torch.randn((b, hkv, t_kv, d), generator=g, device="cuda").to(dtype)
+    v = torch.randn((b, hkv, t_kv, d), generator=g, device="cuda").to(dtype)
+    cache.update_and_fetch(k, v)
+    return cache
+
+
+@pytest.mark.parametrize("backend,bits,dtype,d,hq,hkv,t_kv,t_q,buffer", [
+    ("fp16", 0, torch.float16, 128, 8, 2, 1, 1, 128),        # one key
+    ("fp16", 0, torch.float16, 128, 8, 2, 1089, 1, 128),     # several splits, a ragged tile
+    ("fp16", 0, torch.bfloat16, 64, 6, 2, 700, 3, 128),      # bf16 rows, three a head and query
+    ("fp16", 0, torch.float16, 64, 8, 2, 300, 2, 16),        # hybrid fp16 with a buffer
+    ("fp16", 0, torch.bfloat16, 128, 8, 2, 300, 1, 40),      # hybrid bf16 with a buffer
+    ("grouped", 2, torch.float16, 128, 8, 2, 900, 1, 128),   # register units
+    ("grouped", 4, torch.float16, 128, 8, 2, 900, 1, 20),    # loader-wave shape
+    ("grouped", 3, torch.float16, 128, 8, 2, 333, 1, 20),    # packed rows on the vector ALUs
+    ("turboquant", 2, torch.float16, 128, 8, 2, 600, 1, 30),
+    ("turboquant", 4, torch.float16, 64, 2, 2, 333, 1, 20),
+    ("sunshape", 8, torch.float16, 128, 8, 2, 1500, 1, 128),
+    ("sunshape", 8, torch.float16, 64, 8, 2, 200, 2, 10),
+])
+def test_masked_decodes_equal_the_two_pass_path(backend, bits, dtype, d, hq, hkv, t_kv, t_q, buffer):
+    """Boolean and additive masks on the fused decodes against the two-pass
+    path over the same cache: broadcast forms, per-head biases, rows with
+    every key hidden (they average the values), the type's lowest value,
+    -inf, and a row that is -inf throughout (NaN in both)."""
+    b = 2
+    cache = _masked_cache(backend, bits, dtype, d, hkv, b, t_kv, buffer)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q = torch.randn((b, hq, t_q, d), generator=g, device="cuda").to(dtype)
+    keep = torch.rand((b, 1, t_q, t_kv), generator=g, device="cuda") > 0.4
+    keep[1] = False
+    bias = torch.randn((1, hq, 1, t_kv), generator=g, device="cuda")
+    low = torch.where(keep, 0.0, torch.finfo(dtype).min).to(dtype)
+    lowest = torch.where(keep, 0.5, torch.finfo(torch.float32).min)
+    inf = torch.where(torch.rand((t_q, t_kv), generator=g, device="cuda") > 0.5, 0.0, -torch.inf)
+    all_inf = inf.clone()
+    all_inf[0] = -torch.inf
+    masks = {"bool": keep, "row": keep[0, 0, 0], "per head": bias.half(),
+             "expanded": bias.expand(b, hq, t_q, t_kv), "lowest f16": low,
+             "lowest f32": lowest, "inf": inf, "all inf": all_inf, "int": (bias > 0).int(),
+             "transposed": torch.randn((t_kv, t_q), generator=g, device="cuda").t()}
+    for name, mask in masks.items():
+        ref = attention._two_pass(cache, q, 0.11, mask, torch.float32)
+        before = S.get_kernel_stats().get("sunshape_block_vq_score_hip", 0)
+        got = S.sunshape_sdpa(q, cache, 0.11, mask, out_dtype=torch.float32)
+        assert S.get_kernel_stats().get("sunshape_block_vq_score_hip", 0) == before, name  # fused
+        assert torch.equal(torch.isnan(ref), torch.isnan(got)), name
+        err = (got - ref).nan_to_num().abs().max() / ref.nan_to_num().abs().max().clamp(min=1e-30)
+        assert float(err) <= REL_TOL, (name, float(err))
