@@ -354,6 +354,26 @@ int ss_prefill_attn_il8_hybrid(const void *q, int q_dtype, int64_t batch, int n_
                                int64_t q_offset, void *out, int out_dtype, void *stream);
 
 /*
+ * Prompt attention of fp16 or bf16 queries with the keys reconstructed once
+ * per (batch, KV head) in `workspace` (ss_prefill_workspace_bytes; at least one
+ * head's share, ceil(t_kv / 64) * 256 * head_dim bytes, else
+ * SS_ERR_WORKSPACE; with less than all heads the call goes through them in
+ * turn): head_dim 64 or 128, any GQA group size, values fp16 or bfloat16
+ * (v_dtype) in the 8-token interleaved layout with capacity cap_v, keys from
+ * idx (capacity cap) and, from position t_raw0 on, whole as in
+ * ss_prefill_attn_il8_hybrid (kraw NULL: none, t_raw0 ignored).  Other
+ * arguments as there (kernels.py:303-378, attention.py:307-350).
+ */
+size_t ss_prefill_workspace_bytes(int64_t batch, int n_kv_heads, int head_dim, int64_t t_kv);
+int ss_prefill_attn(const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads,
+                    int64_t t_q, int head_dim, float scale, const int32_t *perm,
+                    const void *codebook, int n_blocks, int n_centroids, const uint8_t *idx,
+                    int64_t cap, const void *values_il8, int v_dtype, int64_t cap_v,
+                    int64_t t_kv, const void *kraw, const float *kfac, int64_t t_raw0,
+                    int causal, int64_t q_offset, void *out, int out_dtype, void *workspace,
+                    size_t workspace_bytes, void *stream);
+
+/*
  * ss_decode_attn_il8 without a workspace: the same kernel, arguments and
  * result, with its split partials and per-column split counters in a static
  * device array of the library (ss_decode_static_scratch_bytes() = 4 MiB,
@@ -396,6 +416,10 @@ int ss_append_values_il8(const void *values, int v_dtype, int64_t n_b, int64_t n
                          int64_t n_t, int64_t v_sb, int64_t v_sh, int64_t v_st,
                          int head_dim, void *out_il8, int64_t cap, int64_t offset,
                          void *stream);
+/* The same layout holding bfloat16 values (copied as they are). */
+int ss_append_values_il8_bf16(const void *values, int64_t n_b, int64_t n_h, int64_t n_t,
+                              int64_t v_sb, int64_t v_sh, int64_t v_st, int head_dim,
+                              void *out_il8, int64_t cap, int64_t offset, void *stream);
 
 /*
  * The whole KV append of an fp16-value cache (reference

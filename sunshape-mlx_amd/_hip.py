@@ -111,6 +111,13 @@ _SIGNATURES = {
                                           _c_void_p, _c_void_p, _int, _int, _c_void_p, _i64,
                                           _c_void_p, _i64, _i64, _c_void_p, _c_void_p, _i64,
                                           _int, _i64, _c_void_p, _int, _c_void_p]),
+    "ss_prefill_workspace_bytes": (_size, [_i64, _int, _int, _i64]),
+    "ss_prefill_attn": (_int, [_c_void_p, _int, _i64, _int, _int, _i64, _int, _f32, _c_void_p,
+                               _c_void_p, _int, _int, _c_void_p, _i64, _c_void_p, _int, _i64,
+                               _i64, _c_void_p, _c_void_p, _i64, _int, _i64, _c_void_p, _int,
+                               _c_void_p, _size, _c_void_p]),
+    "ss_append_values_il8_bf16": (_int, [_c_void_p, _i64, _i64, _i64, _i64, _i64, _i64, _int,
+                                         _c_void_p, _i64, _i64, _c_void_p]),
     "ss_decode_attn_il8_noalloc": (_int, [_c_void_p, _int, _i64, _int, _int, _i64, _int, _f32,
                                           _c_void_p, _c_void_p, _int, _int, _c_void_p, _c_void_p,
                                           _int, _i64, _i64, _int, _i64, _c_void_p, _int, _int,
@@ -1263,6 +1270,44 @@ def prefill_attn_il8_hybrid(q: torch.Tensor, scale: float, perm: torch.Tensor | 
     return out
 
 
+def prefill_attn(q: torch.Tensor, scale: float, perm: torch.Tensor | None,
+                 codebook: torch.Tensor, n_centroids: int, idx: torch.Tensor,
+                 values_il8: torch.Tensor, t_kv: int, kraw: torch.Tensor | None = None,
+                 kfac: torch.Tensor | None = None, t_raw0: int = 0, causal: bool = True,
+                 q_offset: int = 0, out_dtype: torch.dtype | None = None) -> torch.Tensor:
+    """Prompt attention (``ss_prefill_attn``) of fp16 or bf16 queries (B, Hq,
+    T_q, 64 or 128): keys reconstructed once per KV head from the prepared
+    ``codebook``, values ``values_il8`` (B, Hkv, cap_v/8, D, 8) fp16 or
+    bf16; positions from ``t_raw0`` on are scored from the whole keys
+    ``kraw`` / ``kfac`` (:func:`raw_key_rows`) where those are given."""
+    _check_decode_common(q, idx, None, perm)
+    require_gpu(values_il8, codebook, kraw, kfac)
+    b_, hq, tq, d = q.shape
+    _, hkv, cap, nb = idx.shape
+    cap_v = values_il8.shape[2] * 8
+    if values_il8.dtype not in (torch.float16, torch.bfloat16) or not values_il8.is_contiguous() or \
+            tuple(values_il8.shape) != (b_, hkv, cap_v // 8, d, 8):
+        raise ValueError(f"values_il8 must be contiguous 16-bit floats (B, Hkv, cap/8, {d}, 8)")
+    if kraw is not None:
+        n_raw = max(int(t_kv) - int(t_raw0), 1)
+        if kraw.dtype != torch.float16 or not kraw.is_contiguous() or \
+                tuple(kraw.shape) != (b_, hkv, n_raw, 2, d) or kfac.dtype != torch.float32 or \
+                not kfac.is_contiguous() or tuple(kfac.shape) != (b_, hkv, n_raw):
+            raise ValueError("kraw / kfac do not match the buffered tokens")
+    lib = load_library()
+    if codebook.numel() != lib.ss_codebook_f16x2_bytes(nb, n_centroids):
+        raise ValueError("codebook does not match the centroids' shape")
+    out = torch.empty((b_, hq, tq, d), dtype=out_dtype or q.dtype, device=q.device)
+    ws = torch.empty(lib.ss_prefill_workspace_bytes(b_, hkv, d, int(t_kv)), dtype=torch.uint8,
+                     device=q.device)
+    _launched(_attn_stat("sunshape_prefill_attention_mfma", causal), lib.ss_prefill_attn(
+        ptr(q), dtype_code(q.dtype), b_, hq, hkv, tq, d, float(scale), ptr(perm), ptr(codebook),
+        nb, int(n_centroids), ptr(idx), cap, ptr(values_il8), dtype_code(values_il8.dtype), cap_v,
+        int(t_kv), ptr(kraw), ptr(kfac), int(t_raw0), int(bool(causal)), int(q_offset), ptr(out),
+        dtype_code(out.dtype), ptr(ws), ws.numel(), stream_handle(q.device)))
+    return out
+
+
 def raw_key_rows(keys: torch.Tensor, perm: torch.Tensor | None = None
                  ) -> tuple[torch.Tensor, torch.Tensor]:
     """Whole keys (B, H, T, D) -> (rows, factors) for
@@ -1296,6 +1341,23 @@ def prefill_supported(n_q_heads: int, n_kv_heads: int, t_q: int, head_dim: int,
     rep = n_q_heads // n_kv_heads
     return (head_dim == 128 and n_blocks == 16 and rows % rep == 0
             and t_q >= rows // rep)
+
+
+def prompt_supported(q: torch.Tensor, n_kv_heads: int, n_blocks: int, t_kv: int) -> bool:
+    """Whether :func:`prefill_attn` takes queries ``q`` (B, Hq, T_q, D) against
+    ``t_kv`` tokens and is the faster kernel for them.  It streams the keys
+    once per 128 rows of a KV head, one tile of 64 tokens per 1.7 us (1.1 at
+    head_dim 64) and chip-full of workgroups; the decodes stream them once
+    per 4 rows.  Measured crossings (32/8 heads, past tokens: new tokens):
+    0: 128, 2048: 64-128, 32768: 64-128, 4 x 4096: 16-32."""
+    b_, hq, tq, d = q.shape
+    if q.dtype not in (torch.float16, torch.bfloat16) or d not in (64, 128) or n_blocks * 8 != d \
+            or tq < 2:
+        return False
+    rows, heads = hq // n_kv_heads * tq, b_ * n_kv_heads
+    fill = max(1.0, -(-rows // 128) * heads / 256)
+    prompt_us = 25.0 + (1.7 if d == 128 else 1.1) * -(-t_kv // 64) * fill
+    return prompt_us < 15.0 + 9.2e-6 * rows * t_kv * heads
 
 
 def decode_attn_il8_noalloc(q: torch.Tensor, scale: float, perm: torch.Tensor | None,
@@ -1332,16 +1394,24 @@ def decode_attn_il8_noalloc(q: torch.Tensor, scale: float, perm: torch.Tensor | 
 
 def append_values_il8(values: torch.Tensor, out_il8: torch.Tensor, offset: int) -> None:
     """Write (B, H, T, D) values at cache positions [offset, offset+T) of the
-    interleaved buffer (B, H, cap/8, D, 8)."""
+    interleaved buffer (B, H, cap/8, D, 8): float16, or bfloat16 for bfloat16
+    values."""
     require_gpu(values, out_il8)
     if values.dim() != 4 or values.stride(-1) != 1:
         raise ValueError("values must be (B, H, T, D) with unit last stride")
-    if out_il8.dim() != 5 or out_il8.dtype != torch.float16 or not out_il8.is_contiguous():
+    bf = out_il8.dtype == torch.bfloat16 and values.dtype == torch.bfloat16
+    if out_il8.dim() != 5 or not (bf or out_il8.dtype == torch.float16) or \
+            not out_il8.is_contiguous():
         raise ValueError("out_il8 must be a contiguous float16 (B, H, cap/8, D, 8) buffer")
     b_, h_, t_, d = values.shape
     if tuple(out_il8.shape[:2]) != (b_, h_) or out_il8.shape[3] != d:
         raise ValueError("values and cache shapes differ")
     cap = out_il8.shape[2] * 8
+    if bf:
+        check(load_library().ss_append_values_il8_bf16(
+            ptr(values), b_, h_, t_, values.stride(0), values.stride(1), values.stride(2), d,
+            ptr(out_il8), cap, int(offset), stream_handle(values.device)))
+        return
     check(load_library().ss_append_values_il8(
         ptr(values), dtype_code(values.dtype), b_, h_, t_, values.stride(0), values.stride(1),
         values.stride(2), d, ptr(out_il8), cap, int(offset), stream_handle(values.device)))

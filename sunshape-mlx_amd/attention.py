@@ -199,37 +199,45 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
     codec = cache.codec
     buffered = cache.buffer_offset if isinstance(cache, HybridSunShapeKVCache) else 0
     q, kscale, perm = _kernel_query(codec, queries, scale)
-    # a prompt against a hybrid cache (fp16, grouped or TurboQuant values):
-    # compressed keys from the codebook, buffered keys whole, values
-    # materialised once in the interleaved fp16 layout
     b_, hq, tq, d = queries.shape
-    if buffered and cache.dtype == torch.bfloat16 and \
-            ops["kind"] in ("grouped_il", "grouped", "turboquant_il", "turboquant", "sunshape_v"):
-        # with buffered tokens the reference attends over cache.values, the
-        # dequantised values rounded to the cache dtype (cache.py:754-784,
-        # attention.py:307-350); the fused kernels keep them in float32,
-        # which for bf16 (8 significant bits) moves outputs by ~2^-9 of
-        # their scale, so bf16 caches keep the reference's two passes
-        return None
-    if mask is None and isinstance(cache, HybridSunShapeKVCache) and tq > 1 and \
-            ops.get("k_heavy") is None and \
-            cache.dtype == torch.float16 and \
-            q.dtype in (torch.float16, torch.bfloat16) and \
-            _hip.prefill_supported(hq, cache.n_kv_heads, tq, d, codec.n_blocks):
+    # with buffered tokens the reference attends over cache.values, the
+    # dequantised values rounded to the cache dtype (cache.py:754-784,
+    # attention.py:307-350); the fused kernels keep them in float32, which for
+    # bf16 (8 significant bits) moves outputs by ~2^-9 of their scale, so bf16
+    # caches attend over the rounded values here too
+    rounded = bool(buffered) and cache.dtype == torch.bfloat16 and \
+        ops["kind"] in ("grouped_il", "grouped", "turboquant_il", "turboquant", "sunshape_v")
+    # a prompt against a hybrid cache: compressed keys from the codebook,
+    # buffered keys whole, values materialised once in the interleaved layout
+    # (fp16 copies of quantised values only for the whole-group prompts at
+    # head_dim 128: elsewhere the decodes' float32 values are the more exact)
+    whole = ops["kind"] in ("il8", "dense") or rounded
+    if mask is None and isinstance(cache, HybridSunShapeKVCache) and ops.get("k_heavy") is None and \
+            (cache.dtype == torch.float16 or
+             (cache.dtype == torch.bfloat16 and whole)) and \
+            _hip.prompt_supported(q, cache.n_kv_heads, codec.n_blocks, cache.offset) and \
+            (whole or _hip.prefill_supported(hq, cache.n_kv_heads, tq, d, codec.n_blocks)):
         pf = cache.prefill_operands()
         if pf is not None:
             vil8, rows, fac, t_raw0 = pf
             try:
-                out = _hip.prefill_attn_il8_hybrid(q, kscale, perm, codec.kernel_codebook(),
-                                                   codec.n_centroids, ops["idx"], vil8,
-                                                   t_raw0 + buffered, rows, fac, t_raw0,
-                                                   causal=causal, q_offset=q_offset,
-                                                   out_dtype=out_dtype)
+                out = _hip.prefill_attn(q, kscale, perm, codec.kernel_codebook(),
+                                        codec.n_centroids, ops["idx"], vil8, t_raw0 + buffered,
+                                        rows, fac, t_raw0, causal=causal, q_offset=q_offset,
+                                        out_dtype=out_dtype)
             except _hip.SunShapeUnsupported:
                 out = None
             if out is not None:
-                codec.last_score_backend = "hip_prefill_mfma_hybrid"
+                codec.last_score_backend = "hip" if rounded else "hip_prefill_mfma_hybrid"
                 return out
+    if rounded:
+        if ops.get("k_heavy") is not None:
+            return None
+        # the compressed values in bf16, token-major, for the bf16 decode
+        tc = cache.compressed_offset
+        ops = {"kind": "dense", "idx": ops["idx"][:, :, :tc].contiguous(),
+               "values": cache._compressed_values().contiguous(),
+               "buf_keys": ops["buf_keys"], "buf_values": ops["buf_values"]}
     # the buffer joins the fused softmax on every fused kernel
     if buffered and codec.mode not in PERM_MODES and codec.use_rotation:
         # the kernels score buffered keys against the query they are given,
@@ -246,16 +254,30 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
     # reconstructed from the codebook, both products on the matrix cores
     b_, hq, tq, d = queries.shape
     hv = {"k_heavy": ops.get("k_heavy"), "heavy_dims": ops.get("heavy_dims")}
-    if mask is None and not buffered and kind == "il8" and tq > 1 and hv["k_heavy"] is None and \
-            _hip.prefill_supported(hq, cache.n_kv_heads, tq, d, codec.n_blocks):
+    if mask is None and not buffered and kind in ("il8", "dense") and hv["k_heavy"] is None and tq > 1:
+        out = None
         try:
-            out = _hip.prefill_attn_il8(q, kscale, perm, codec.kernel_codebook(), codec.n_centroids,
-                                        ops["idx"], ops["values"], t_kv, causal=causal,
+            if (kind == "il8" or ops["values"].dtype == torch.bfloat16) and \
+                    _hip.prompt_supported(q, cache.n_kv_heads, codec.n_blocks, t_kv):
+                v8 = ops["values"]
+                if kind == "dense":
+                    v8 = torch.empty((b_, cache.n_kv_heads, (t_kv + 7) // 8, d, 8),
+                                     dtype=torch.bfloat16, device=q.device)
+                    _hip.append_values_il8(ops["values"][:, :, :t_kv], v8, 0)
+                out = _hip.prefill_attn(q, kscale, perm, codec.kernel_codebook(),
+                                        codec.n_centroids, ops["idx"], v8, t_kv, causal=causal,
                                         q_offset=q_offset, out_dtype=out_dtype)
+            elif kind == "il8" and _hip.prefill_supported(hq, cache.n_kv_heads, tq, d,
+                                                          codec.n_blocks):  # float32 queries
+                out = _hip.prefill_attn_il8(q, kscale, perm, codec.kernel_codebook(),
+                                            codec.n_centroids, ops["idx"], ops["values"], t_kv,
+                                            causal=causal, q_offset=q_offset,
+                                            out_dtype=out_dtype)
         except _hip.SunShapeUnsupported:
-            return None
-        codec.last_score_backend = "hip_prefill_mfma"
-        return out
+            out = None
+        if out is not None:
+            codec.last_score_backend = "hip_prefill_mfma"
+            return out
     # the matrix-core decodes without a token buffer: one prepared launch
     # (argument checks, codebook and split plan done once per cache layout)
     if mask is None and not buffered and kind in ("il8", "grouped_il") and hv["k_heavy"] is None:
@@ -270,12 +292,19 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
     # buffered tokens
     if kind == "dense" and ops["values"].dtype == torch.bfloat16:
         try:
-            plan = _prepared_decode(cache, ops, codec, q, kscale, perm)
+            if rounded:  # values of this call only: no plan to keep
+                plan = _hip.prepare_decode_dense(q, kscale, perm, codec.kernel_codebook(),
+                                                 codec.n_blocks, codec.n_centroids, ops["idx"],
+                                                 ops["values"])
+            else:
+                plan = _prepared_decode(cache, ops, codec, q, kscale, perm)
             out = plan(q, t_kv, causal, q_offset, ops.get("buf_keys"), ops.get("buf_values"),
                        buffered, out_dtype=out_dtype, mask=mask)
         except _hip.SunShapeUnsupported:
             return None
-        codec.last_score_backend = "hip_fused_buffer" if buffered else "hip_fused"
+        # (over rounded values: the name the two-pass path reports)
+        codec.last_score_backend = ("hip" if rounded else
+                                    "hip_fused_buffer" if buffered else "hip_fused")
         return out
     # il8 and grouped_il with a hybrid cache's buffered tokens (the buffer
     # window passed per call); rotated codecs hand the kernel rotated buffer copies

@@ -948,29 +948,33 @@ class HybridSunShapeKVCache:
         return None
 
     def prefill_operands(self):
-        """What the prompt kernel (``ss_prefill_attn_il8_hybrid``) reads of
-        this cache: ``(values_il8, key_rows, key_factors, t_raw0)`` -- every
-        token's value in the 8-token interleaved fp16 layout (compressed values
-        dequantised, then the buffer's), and the buffered keys whole in the
-        codec's basis (``_hip.raw_key_rows``), which start at position t_raw0
-        = compressed_offset.  O(T) work, against the prompt's O(T x T_q).
-        None for SunShape-coded values (an fp16 copy of each value codeword
-        would move every token that uses it the same way) and for fp16 heavy
-        blocks."""
+        """What the prompt kernel (``ss_prefill_attn``) reads of this cache:
+        ``(values_il8, key_rows, key_factors, t_raw0)`` -- every token's value
+        in the 8-token interleaved layout in the cache's own 16-bit type
+        (compressed values dequantised, then the buffer's), and the buffered
+        keys whole in the codec's basis (``_hip.raw_key_rows``), which start
+        at position t_raw0 = compressed_offset.  O(T) work, against the
+        prompt's O(T x T_q).  None for SunShape-coded values of an fp16 cache
+        (an fp16 copy of each value codeword would move every token that uses
+        it the same way; a bf16 cache's are bf16 in the reference too) and
+        for fp16 heavy blocks."""
         self.flush()
-        if self.value_backend == "sunshape" or self._heavy_dims is not None or \
+        bf = self.dtype == torch.bfloat16
+        if (self.value_backend == "sunshape" and not bf) or self._heavy_dims is not None or \
                 self._key_buffer is None:
             return None
         tc, tb = self._compressed_offset, self._buffer_offset
         t_kv = tc + tb
         b_, h_, d = self._key_buffer.shape[0], self.n_kv_heads, self.head_dim
         dev = self._key_buffer.device
-        vil8 = torch.zeros((b_, h_, (t_kv + 7) // 8, d, 8), dtype=torch.float16, device=dev)
+        # (slots past the last token are never read as values)
+        vil8 = torch.empty((b_, h_, (t_kv + 7) // 8, d, 8),
+                           dtype=torch.bfloat16 if bf else torch.float16, device=dev)
         if tc:
             if self._values_il8 is not None:
                 nblk = (tc + 7) // 8
                 vil8[:, :, :nblk] = self._values_il8[:, :, :nblk]
-            elif self.value_backend == "grouped" and self._values_il is not None:
+            elif not bf and self.value_backend == "grouped" and self._values_il is not None:
                 gc = self._value_codec_impl
                 _hip.grouped_il_to_il8(self._values_il, gc.bits, gc.group_size,
                                        self._value_scales, self._value_zeros, tc, vil8)
@@ -978,7 +982,7 @@ class HybridSunShapeKVCache:
                 dense = self._compressed_values()
                 if dense is None:
                     return None
-                _hip.append_values_il8(dense.to(torch.float16).contiguous(), vil8, 0)
+                _hip.append_values_il8(dense.to(vil8.dtype).contiguous(), vil8, 0)
         if tb:
             _hip.append_values_il8(self.buffer_values, vil8, tc)
             kb = self.buffer_keys

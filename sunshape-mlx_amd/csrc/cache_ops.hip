@@ -10,20 +10,58 @@
 
 namespace ss {
 
+// A thread takes two dims of one 8-token block: eight 4-byte loads (a wave's
+// cover 256 consecutive bytes of each token's row) and two 16-byte stores (2
+// KB a wave).  Blocks at the ends of the range that hold other tokens too
+// store only their own.  HBM bounds it.  One element a thread, its 2-byte
+// stores 16 bytes apart, took 17.1 us for 8 heads x 4096 tokens of 128 dims.
+// OUT_BF: bfloat16 words out (the input must be bfloat16), else fp16.
+template <bool OUT_BF>
 __global__ void __launch_bounds__(256)
-    append_il8_kernel(const void *v, int v_dtype, int64_t n_h, int64_t n_t, int64_t n_tok,
-                      int64_t v_sb, int64_t v_sh, int64_t v_st, int d, __half *out, int64_t cap,
+    append_il8_kernel(const void *v, int v_dtype, int64_t n_h, int64_t n_t, int64_t n_blk, int64_t total,
+                      int64_t v_sb, int64_t v_sh, int64_t v_st, int d, int pairs, __half *out, int64_t cap,
                       int64_t offset) {
+    const int per = pairs ? (d + 1) / 2 : d;  // threads of a block's row
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n_tok * d) return;
-    const int64_t n = e / d;
-    const int j = (int)(e - n * d);
-    const int64_t b = n / (n_h * n_t);
-    const int64_t rem = n - b * n_h * n_t;
-    const int64_t h = rem / n_t;
-    const int64_t t = rem - h * n_t;
-    const float x = load_as_f32(v, v_dtype, b * v_sb + h * v_sh + t * v_st + j);
-    store_value_il8(out, b * n_h + h, cap, d, offset + t, j, x);
+    if (e >= total) return;
+    const int64_t n = e / per;
+    const int j = (int)(e - n * per) * (pairs ? 2 : 1);
+    const int64_t bh = n / n_blk, blk = offset / 8 + (n - bh * n_blk);
+    const int64_t b = bh / n_h, h = bh - b * n_h;
+    const int64_t t0 = blk * 8 - offset;  // token of the block's first slot (may be < 0)
+    const int64_t src = b * v_sb + h * v_sh + j;
+    const bool whole = t0 >= 0 && t0 + 8 <= n_t && ((uintptr_t)out % 16) == 0;
+    uint32_t w[8];  // dims j (low half) and j + 1 of the block's tokens
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int64_t t = min(max(t0 + i, (int64_t)0), n_t - 1);
+        const int64_t o = src + t * v_st;
+        if (OUT_BF || v_dtype == SS_F16) {
+            const uint16_t *p = static_cast<const uint16_t *>(v) + o;
+            w[i] = pairs ? *reinterpret_cast<const uint32_t *>(p) : *p;
+        } else {
+            const __half x0 = __float2half(load_as_f32(v, v_dtype, o));
+            const __half x1 = pairs ? __float2half(load_as_f32(v, v_dtype, o + 1)) : x0;
+            w[i] = (uint32_t)__half_as_ushort(x0) | ((uint32_t)__half_as_ushort(x1) << 16);
+        }
+    }
+    uint16_t *dst = reinterpret_cast<uint16_t *>(out) + ((bh * (cap / 8) + blk) * d + j) * 8;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        if (k == 1 && !pairs) break;
+        const int sh = 16 * k;
+        if (whole) {
+            uint32_t o4[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                o4[i] = ((w[2 * i] >> sh) & 0xffffu) | (((w[2 * i + 1] >> sh) & 0xffffu) << 16);
+            *reinterpret_cast<uint4 *>(dst + 8 * k) = make_uint4(o4[0], o4[1], o4[2], o4[3]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (t0 + i >= 0 && t0 + i < n_t) dst[8 * k + i] = (uint16_t)(w[i] >> sh);
+        }
+    }
 }
 
 // Whole keys for the hybrid prompt kernel: one wave per token.  Dim j of the
@@ -65,26 +103,46 @@ __global__ void __launch_bounds__(256)
 
 using namespace ss;
 
-extern "C" int ss_append_values_il8(const void *values, int v_dtype, int64_t n_b, int64_t n_h,
-                                    int64_t n_t, int64_t v_sb, int64_t v_sh, int64_t v_st,
-                                    int head_dim, void *out_il8, int64_t cap, int64_t offset,
-                                    void *stream) {
+template <bool OUT_BF>
+static int append_il8(const void *values, int v_dtype, int64_t n_b, int64_t n_h, int64_t n_t,
+                      int64_t v_sb, int64_t v_sh, int64_t v_st, int head_dim, void *out_il8,
+                      int64_t cap, int64_t offset, void *stream) {
     SS_REQUIRE(valid_dtype(v_dtype), "bad value dtype");
     SS_REQUIRE(n_b >= 0 && n_h >= 0 && n_t >= 0 && head_dim >= 1, "bad sizes");
     SS_REQUIRE(cap % 8 == 0, "cap must be a multiple of 8");
     SS_REQUIRE(offset >= 0 && offset + n_t <= cap, "tokens [%lld, %lld) exceed cap %lld",
                (long long)offset, (long long)(offset + n_t), (long long)cap);
-    const int64_t n_tok = n_b * n_h * n_t;
-    if (n_tok == 0) return SS_OK;
+    if (n_b * n_h * n_t == 0) return SS_OK;
     SS_REQUIRE(values && out_il8, "null pointer argument");
-    const int64_t total = n_tok * head_dim;
-    SS_UNSUPPORTED(total < (1LL << 32), "too many elements for one launch");
-    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(append_il8_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
-                       values, v_dtype, n_h, n_t, n_tok, v_sb, v_sh, v_st, head_dim,
-                       reinterpret_cast<__half *>(out_il8), cap, offset);
+    // two dims a thread where every row starts on a pair of elements
+    const int es = v_dtype == SS_F32 ? 4 : 2;
+    const bool pairs = head_dim % 2 == 0 && ((uintptr_t)values % (2 * es)) == 0 &&
+                       ((v_sb | v_sh | v_st) & 1) == 0;
+    const int64_t n_blk = (offset + n_t + 7) / 8 - offset / 8;
+    const int64_t total = n_b * n_h * n_blk * (pairs ? head_dim / 2 : head_dim);
+    SS_UNSUPPORTED(n_b * n_h * n_t * head_dim < (1LL << 32) && total < (1LL << 39),
+                   "too many elements for one launch");
+    hipLaunchKernelGGL(append_il8_kernel<OUT_BF>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+                       reinterpret_cast<hipStream_t>(stream), values, v_dtype, n_h, n_t, n_blk, total,
+                       v_sb, v_sh, v_st, head_dim, pairs ? 1 : 0, reinterpret_cast<__half *>(out_il8),
+                       cap, offset);
     SS_LAUNCH_CHECK("append_il8_kernel launch");
     return SS_OK;
+}
+
+extern "C" int ss_append_values_il8(const void *values, int v_dtype, int64_t n_b, int64_t n_h,
+                                    int64_t n_t, int64_t v_sb, int64_t v_sh, int64_t v_st,
+                                    int head_dim, void *out_il8, int64_t cap, int64_t offset,
+                                    void *stream) {
+    return append_il8<false>(values, v_dtype, n_b, n_h, n_t, v_sb, v_sh, v_st, head_dim, out_il8, cap,
+                             offset, stream);
+}
+
+extern "C" int ss_append_values_il8_bf16(const void *values, int64_t n_b, int64_t n_h, int64_t n_t,
+                                         int64_t v_sb, int64_t v_sh, int64_t v_st, int head_dim,
+                                         void *out_il8, int64_t cap, int64_t offset, void *stream) {
+    return append_il8<true>(values, SS_BF16, n_b, n_h, n_t, v_sb, v_sh, v_st, head_dim, out_il8, cap,
+                            offset, stream);
 }
 
 extern "C" int ss_raw_key_rows(const void *keys, int k_dtype, int64_t n_b, int64_t n_h,

@@ -166,3 +166,91 @@ def test_masked_decodes_equal_the_two_pass_path(backend, bits, dtype, d, hq, hkv
         assert torch.equal(torch.isnan(ref), torch.isnan(got)), name
         err = (got - ref).nan_to_num().abs().max() / ref.nan_to_num().abs().max().clamp(min=1e-30)
         assert float(err) <= REL_TOL, (name, float(err))
+
+
+@pytest.mark.parametrize("b,hq,hkv,d,t_q,past,causal,qdt,vdt,n_raw,nc,ws_heads", [
+    (1, 4, 1, 128, 1, 0, True, torch.float16, torch.float16, 0, 256, 0),       # one key, one row
+    (1, 8, 2, 128, 33, 0, True, torch.float16, torch.float16, 0, 256, 0),      # a sub-tile and a key
+    (2, 8, 2, 128, 64, 1, True, torch.bfloat16, torch.bfloat16, 0, 100, 0),    # 65 keys
+    (1, 14, 2, 128, 70, 300, True, torch.float16, torch.bfloat16, 0, 256, 1),  # groups of 7 heads
+    (1, 2, 2, 64, 129, 0, True, torch.float16, torch.float16, 0, 256, 0),      # one head a group
+    (1, 8, 2, 64, 40, 77, False, torch.bfloat16, torch.bfloat16, 0, 17, 1),    # no causal cut
+    (2, 8, 2, 128, 50, 200, True, torch.float16, torch.float16, 90, 256, 3),   # whole keys
+    (1, 8, 2, 64, 30, 64, True, torch.bfloat16, torch.bfloat16, 31, 256, 0),   # and bf16 values
+    (1, 64, 16, 128, 2080, 0, True, torch.float16, torch.float16, 0, 256, 0),  # 8 x 1 waves
+    (1, 64, 16, 64, 1040, 30, True, torch.float16, torch.float16, 0, 256, 0),  # 4 x 1 waves
+])
+def test_prompt_kernel_matches_the_definition(b, hq, hkv, d, t_q, past, causal, qdt, vdt, n_raw, nc,
+                                              ws_heads):
+    """ss_prefill_attn against attention over the reconstructed keys in
+    float64: tile edges, ragged rows, GQA groups, both value types, whole
+    (buffered) keys, and workspaces that hold a few heads at a time.  Key
+    and value slots past the last token hold NaN."""
+    g = torch.Generator(device="cuda").manual_seed(t_q * 7 + past)
+    nb, t_kv = d // 8, past + t_q
+    cap = (t_kv + 255) // 256 * 256
+    cents = torch.randn((nb, nc, 8), generator=g, device="cuda")
+    perm = torch.randperm(d, generator=g, device="cuda").int()
+    idx = torch.randint(0, nc, (b, hkv, cap, nb), generator=g, device="cuda").to(torch.uint8)
+    v = torch.randn((b, hkv, t_kv, d), generator=g, device="cuda").to(vdt)
+    v8 = torch.full((b, hkv, cap // 8, d, 8), float("nan"), dtype=vdt, device="cuda")
+    _hip.append_values_il8(v, v8, 0)
+    q = torch.randn((b, hq, t_q, d), generator=g, device="cuda").to(qdt)
+    scale, t_raw0 = 0.1, t_kv - n_raw
+    raw = torch.randn((b, hkv, max(n_raw, 1), d), generator=g, device="cuda").to(qdt)
+    kw = {}
+    if n_raw:
+        rows, fac = _hip.raw_key_rows(raw, perm)
+        kw = dict(kraw=rows, kfac=fac, t_raw0=t_raw0)
+    out = _hip.prefill_attn(q, scale, perm, _hip.codebook_f16x2(cents), nc, idx, v8, t_kv,
+                            causal=causal, q_offset=past if causal else 0,
+                            out_dtype=torch.float32, **kw)
+    if ws_heads:  # the same call with room for ws_heads heads
+        lib = _hip.load_library()
+        cb = _hip.codebook_f16x2(cents)
+        ws = torch.empty(lib.ss_prefill_workspace_bytes(1, 1, d, t_kv) * ws_heads,
+                         dtype=torch.uint8, device="cuda")
+        out2 = torch.empty_like(out)
+        _hip.check(lib.ss_prefill_attn(
+            q.data_ptr(), _hip.dtype_code(qdt), b, hq, hkv, t_q, d, scale, perm.data_ptr(),
+            cb.data_ptr(), nb, nc, idx.data_ptr(), cap, v8.data_ptr(), _hip.dtype_code(vdt), cap,
+            t_kv, _hip.ptr(kw.get("kraw")), _hip.ptr(kw.get("kfac")), t_raw0, int(causal),
+            past if causal else 0, out2.data_ptr(), _hip.SS_F32, ws.data_ptr(), ws.numel(),
+            _hip.stream_handle(q.device)))
+        assert torch.equal(out, out2)
+    k = cents.double()[torch.arange(nb, device="cuda"), idx[:, :, :t_kv].long()].flatten(-2)
+    if n_raw:
+        k[:, :, t_raw0:] = raw[:, :, :n_raw].double()[..., perm.long()]
+    qs = (q * scale).double()[..., perm.long()]
+    rep = hq // hkv
+    pos = torch.arange(t_kv, device="cuda")
+    hide = pos[None] > past + torch.arange(t_q, device="cuda")[:, None]
+    worst = 0.0
+    for bi in range(b):
+        for h in range(0, hq, 1 if t_q < 500 else 23):
+            s = qs[bi, h] @ k[bi, h // rep].t()
+            if causal:
+                s = s.masked_fill(hide, float("-inf"))
+            ref = torch.softmax(s, dim=-1) @ v[bi, h // rep].double()
+            worst = max(worst, float((out[bi, h] - ref).abs().max() / ref.abs().max()))
+    assert worst <= REL_TOL
+
+
+@pytest.mark.parametrize("n_t,offset,d,dtype,pad", [
+    (1, 0, 128, torch.float16, 0), (8, 0, 64, torch.float16, 0), (7, 5, 128, torch.float32, 0),
+    (30, 3, 128, torch.bfloat16, 0), (17, 8, 64, torch.float16, 1), (9, 7, 33, torch.float16, 0),
+])
+def test_append_il8_keeps_the_other_tokens(n_t, offset, d, dtype, pad):
+    """Blocks at the ends of an append keep the tokens outside it; odd head
+    dims, rows at odd addresses, float32 and bf16 values."""
+    b, h, cap = 2, 3, 48
+    g = torch.Generator(device="cuda").manual_seed(n_t)
+    for out_dtype in (torch.float16, torch.bfloat16):
+        if out_dtype == torch.bfloat16 and dtype != torch.bfloat16:
+            continue
+        v = torch.randn((b, h, n_t, d + pad), generator=g, device="cuda").to(dtype)[..., pad:]
+        out = torch.randn((b, h, cap // 8, d, 8), generator=g, device="cuda").to(out_dtype)
+        want = out.permute(0, 1, 2, 4, 3).reshape(b, h, cap, d).clone()
+        want[:, :, offset:offset + n_t] = v.to(out_dtype)
+        _hip.append_values_il8(v, out, offset)
+        assert torch.equal(out.permute(0, 1, 2, 4, 3).reshape(b, h, cap, d), want)
