@@ -254,3 +254,25 @@ def test_append_il8_keeps_the_other_tokens(n_t, offset, d, dtype, pad):
         want[:, :, offset:offset + n_t] = v.to(out_dtype)
         _hip.append_values_il8(v, out, offset)
         assert torch.equal(out.permute(0, 1, 2, 4, 3).reshape(b, h, cap, d), want)
+
+
+@pytest.mark.parametrize("nb,bd,n,dtype,use_perm,pad", [
+    (16, 8, 1, torch.float16, True, 0),       # one token
+    (16, 8, 31, torch.bfloat16, True, 0),     # one short of a workgroup's tokens
+    (32, 4, 33, torch.float32, True, 3),      # a workgroup and one, strided index rows
+    (8, 8, 100, torch.float16, False, 0),     # head_dim 64, no permutation
+    (16, 16, 65, torch.float16, True, 0),     # head_dim 256
+    (4, 16, 64, torch.bfloat16, True, 1),
+    (12, 8, 40, torch.float32, True, 0),      # 96 dims: the element kernel
+])
+def test_dequantised_rows_are_the_codebook_rows(nb, bd, n, dtype, use_perm, pad):
+    g = torch.Generator(device="cuda").manual_seed(nb * n)
+    d = nb * bd
+    cents = torch.randn((nb, 200, bd), generator=g, device="cuda")
+    store = torch.randint(0, 256, (n, nb + pad), generator=g, device="cuda", dtype=torch.uint8)
+    idx = store[:, :nb]
+    inv = torch.randperm(d, generator=g, device="cuda").to(torch.int32) if use_perm else None
+    got = _hip.dequantize_blockvq(idx, cents, inv, out_dtype=dtype)
+    rows = cents[torch.arange(nb, device="cuda"), idx.long().clamp(max=199)].flatten(1)
+    want = rows[:, inv.long()] if use_perm else rows
+    assert torch.equal(got, want.to(dtype))  # one rounding each
