@@ -185,20 +185,38 @@ __global__ void __launch_bounds__(256)
 // rounded separately in float32, as dequantize_grouped_kernel), and writes
 // each 8-token group it covers as one 16-byte store.  Tokens at or past n_t
 // inside the last group are written as zero; groups starting at or past n_t
-// are not written.
+// are not written.  LDS: the scales and zeros of the workgroup's tokens are
+// read once, coalesced, into LDS (kSzPairs pairs at most, checked by the host);
+// without it every word waits for 32 two-byte loads (16 heads, 8192 tokens of
+// 128 dims at 2 bits: 30.4 us, 13.7 now, 34 MB written).
+constexpr int kSzPairs = 2048;
+
+template <bool LDS>
 __global__ void __launch_bounds__(256)
     grouped_il_to_il8_kernel(const uint32_t *codes_il, int64_t cap, int d, int bits, int group,
                              const void *scales, const void *zeros, int sz_dtype, int64_t sz_cap,
                              int64_t n_t, int64_t n_blk, __half *out, int64_t cap_out) {
 #pragma clang fp contract(off)
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t e0 = blockIdx.x * blockDim.x, e = e0 + threadIdx.x;
     const int64_t bh = blockIdx.y;
-    if (e >= n_blk * d) return;
-    const int64_t blk = e / d;
-    const int dd = (int)(e - blk * d);
     const int vpw = vals_per_word(bits);
     const uint32_t mask = (1u << bits) - 1u;
     const int n_groups = d / group;
+    __shared__ float2 szl[LDS ? kSzPairs : 1];  // [token of the workgroup][group]
+    const int64_t tok0 = (int64_t)(e0 / (uint32_t)d) * vpw;
+    if constexpr (LDS) {
+        const int64_t tok1 = min(n_t, (int64_t)((e0 + 255) / (uint32_t)d + 1) * vpw);
+        const int n = (int)max(tok1 - tok0, (int64_t)0) * n_groups;
+        for (int i = threadIdx.x; i < n; i += 256) {
+            const int64_t gi = (bh * sz_cap + tok0) * n_groups + i;
+            szl[i] = make_float2(load_as_f32(scales, sz_dtype, gi), load_as_f32(zeros, sz_dtype, gi));
+        }
+        __syncthreads();
+    }
+    if (e >= n_blk * d) return;
+    const int64_t blk = e / (uint32_t)d;
+    const int dd = (int)(e - (uint32_t)blk * d);
+    const int grp = dd / group;
     const uint32_t word = codes_il[(bh * (cap / vpw) + blk) * d + dd];
     for (int h8 = 0; h8 < vpw / 8; ++h8) {
         const int64_t t0 = blk * vpw + h8 * 8;
@@ -210,9 +228,15 @@ __global__ void __launch_bounds__(256)
             float x = 0.f;
             if (t < n_t) {
                 const float q = (float)((word >> il_pos(bits, h8 * 8 + i)) & mask);
-                const int64_t gi = (bh * sz_cap + t) * n_groups + dd / group;
-                const float prod = q * load_as_f32(scales, sz_dtype, gi);
-                x = prod + load_as_f32(zeros, sz_dtype, gi);
+                float2 sz;
+                if constexpr (LDS) {
+                    sz = szl[(int)(t - tok0) * n_groups + grp];
+                } else {
+                    const int64_t gi = (bh * sz_cap + t) * n_groups + grp;
+                    sz = make_float2(load_as_f32(scales, sz_dtype, gi), load_as_f32(zeros, sz_dtype, gi));
+                }
+                const float prod = q * sz.x;
+                x = prod + sz.y;
             }
             v8[i] = __float2half(x);
         }
@@ -389,9 +413,12 @@ extern "C" int ss_grouped_il_to_il8(const uint32_t *codes_il, int64_t n_bh, int6
     const int64_t total = n_blk * head_dim;
     SS_UNSUPPORTED(total < (1LL << 32), "too many elements for one launch");
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(grouped_il_to_il8_kernel, dim3(blocks_for(total), (unsigned)n_bh), dim3(256),
-                       0, st, codes_il, cap, head_dim, bits, group_size, scales, zeros, sz_dtype,
-                       sz_cap, n_t, n_blk, reinterpret_cast<__half *>(out_il8), cap_out);
+    // words of a workgroup lie in at most 255 / head_dim + 2 token blocks
+    const bool lds = (int64_t)(255 / head_dim + 2) * vpw * (head_dim / group_size) <= kSzPairs;
+    const auto kern = lds ? grouped_il_to_il8_kernel<true> : grouped_il_to_il8_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3(blocks_for(total), (unsigned)n_bh), dim3(256), 0, st,
+                       codes_il, cap, head_dim, bits, group_size, scales, zeros, sz_dtype, sz_cap, n_t, n_blk,
+                       reinterpret_cast<__half *>(out_il8), cap_out);
     SS_LAUNCH_CHECK("grouped_il_to_il8_kernel launch");
     return SS_OK;
 }
