@@ -795,6 +795,20 @@ int ss_pack_grouped_il(const uint32_t *packed, int64_t n_b, int64_t n_h, int64_t
                        uint32_t *out_il, int64_t cap, int64_t offset, void *stream);
 
 /*
+ * Quantise values into a cache's interleaved codes, scales and zeros at
+ * positions offset .. offset+n_t-1 in one launch: what
+ * ss_quantize_values_grouped and ss_pack_grouped_il write (identical codes,
+ * scale and zero; other tokens sharing a word keep their codes).  codes_il
+ * [n_b][n_h][cap*bits/32][head_dim], scales and zeros
+ * [n_b][n_h][cap][head_dim/group_size].  head_dim 64 or 128, bits 2 or 4,
+ * group_size a power of two >= 8; else SS_ERR_UNSUPPORTED.
+ */
+int ss_append_values_grouped_il(const void *values, int v_dtype, int64_t n_b, int64_t n_h, int64_t n_t,
+                                int64_t v_sb, int64_t v_sh, int64_t v_st, int head_dim, int bits,
+                                int group_size, uint32_t *codes_il, void *scales, void *zeros,
+                                int sz_dtype, int64_t cap, int64_t offset, void *stream);
+
+/*
  * One decode step of an fp16-value cache in one launch: the cache holds
  * t_cache tokens (idx [batch][n_kv_heads][cap][n_blocks], values_il8 as
  * ss_decode_attn_il8), and the step's n_new (1..4) new tokens arrive as fp16

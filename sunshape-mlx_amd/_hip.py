@@ -197,6 +197,9 @@ _SIGNATURES = {
                                     _c_void_p, _int, _i64, _i64, _c_void_p, _i64, _c_void_p]),
     "ss_raw_key_rows": (_int, [_c_void_p, _int, _i64, _i64, _i64, _i64, _i64, _i64, _int,
                                _c_void_p, _c_void_p, _c_void_p, _c_void_p]),
+    "ss_append_values_grouped_il": (_int, [_c_void_p, _int, _i64, _i64, _i64, _i64, _i64, _i64,
+                                           _int, _int, _int, _c_void_p, _c_void_p, _c_void_p, _int,
+                                           _i64, _i64, _c_void_p]),
     "ss_quantize_values_grouped": (_int, [_c_void_p, _int, _i64, _i64, _i64, _i64, _i64, _i64,
                                           _int, _int, _int, _c_void_p, _c_void_p, _c_void_p, _int,
                                           _i64, _i64, _i64, _c_void_p]),
@@ -1901,6 +1904,29 @@ def quantize_values_grouped(values: torch.Tensor, bits: int, group_size: int,
         ptr(v4), dtype_code(v4.dtype), b_, h_, t_, v4.stride(0), v4.stride(1), v4.stride(2), d,
         int(bits), int(group_size), ptr(p4), ptr(s4), ptr(z4), dtype_code(s4.dtype), o_sb, o_sh,
         o_st, stream_handle(values.device)))
+
+
+def append_values_grouped_il(values: torch.Tensor, bits: int, group_size: int,
+                             codes_il: torch.Tensor, scales: torch.Tensor, zeros: torch.Tensor,
+                             offset: int) -> None:
+    """Quantise (B, H, T, D) values into cache positions [offset, offset + T)
+    of the interleaved codes (B, H, cap*bits/32, D) and of the scales and
+    zeros (B, H, cap, groups), one launch (``ss_append_values_grouped_il``):
+    :func:`quantize_values_grouped` and :func:`pack_grouped_il` together."""
+    require_gpu(values, codes_il, scales, zeros)
+    if values.dim() != 4 or values.stride(-1) != 1:
+        raise ValueError("values must be (B, H, T, D) with unit last stride")
+    b_, h_, t_, d = values.shape
+    if not (codes_il.is_contiguous() and scales.is_contiguous() and zeros.is_contiguous()):
+        raise ValueError("codes, scales and zeros must be contiguous")
+    cap = codes_il.shape[2] * (32 // bits)
+    if tuple(codes_il.shape) != (b_, h_, cap * bits // 32, d) or scales.dtype != zeros.dtype or \
+            tuple(scales.shape) != (b_, h_, cap, d // group_size) or scales.shape != zeros.shape:
+        raise ValueError("codes, scales and zeros do not match the values' shape")
+    _launched("sunshape_quantize_values_hip", load_library().ss_append_values_grouped_il(
+        ptr(values), dtype_code(values.dtype), b_, h_, t_, values.stride(0), values.stride(1),
+        values.stride(2), d, int(bits), int(group_size), ptr(codes_il), ptr(scales), ptr(zeros),
+        dtype_code(scales.dtype), cap, int(offset), stream_handle(values.device)))
 
 
 def dequantize_values_grouped(packed: torch.Tensor, scales: torch.Tensor, zeros: torch.Tensor,

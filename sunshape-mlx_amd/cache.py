@@ -541,15 +541,8 @@ class HybridSunShapeKVCache:
         if self.value_backend == "grouped":
             gc = self._value_codec_impl
             if self._grouped_il:
-                # quantise into contiguous rows, then interleave the codes
-                h_ = self.n_kv_heads
-                rows = torch.empty((b_, h_, n, gc.packed_dim), dtype=torch.int32, device=dev)
-                sc = torch.empty((b_, h_, n, gc.n_groups), dtype=self.value_scale_dtype, device=dev)
-                zr = torch.empty_like(sc)
-                _hip.quantize_values_grouped(vf, gc.bits, gc.group_size, rows, sc, zr)
-                self._value_scales[:, :, c0:c1] = sc
-                self._value_zeros[:, :, c0:c1] = zr
-                _hip.pack_grouped_il(rows, gc.bits, self._values_il, c0)
+                _hip.append_values_grouped_il(vf, gc.bits, gc.group_size, self._values_il,
+                                              self._value_scales, self._value_zeros, c0)
             else:
                 _hip.quantize_values_grouped(vf, gc.bits, gc.group_size,
                                              self._values_packed[:, :, c0:c1],

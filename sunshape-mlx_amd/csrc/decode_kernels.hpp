@@ -144,39 +144,6 @@ constexpr int pow2_ceil(int x) { return x <= 1 ? 1 : 2 * pow2_ceil((x + 1) / 2);
 // ---------------------------------------------------------------------------
 // Value formats.  Each lane of a token group holds DPL consecutive dims.
 // ---------------------------------------------------------------------------
-template <typename T>
-__device__ __forceinline__ void unpack16(const uint4 &u, float *x);
-
-template <>
-__device__ __forceinline__ void unpack16<__half>(const uint4 &u, float *x) {
-    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        __half2 h = *reinterpret_cast<const __half2 *>(&w[i]);
-        float2 f = __half22float2(h);
-        x[2 * i] = f.x;
-        x[2 * i + 1] = f.y;
-    }
-}
-
-template <>
-__device__ __forceinline__ void unpack16<__hip_bfloat16>(const uint4 &u, float *x) {
-    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        x[2 * i] = __uint_as_float(w[i] << 16);
-        x[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-    }
-}
-
-template <>
-__device__ __forceinline__ void unpack16<float>(const uint4 &u, float *x) {
-    x[0] = __uint_as_float(u.x);
-    x[1] = __uint_as_float(u.y);
-    x[2] = __uint_as_float(u.z);
-    x[3] = __uint_as_float(u.w);
-}
-
 template <int D, typename T>
 struct VDense {
     static constexpr int DPL = 16 / (int)sizeof(T);
@@ -4237,24 +4204,6 @@ struct MergeBuffer {
     int dtype, vec;
     int64_t sb, sh, st, n;
 };
-
-// Eight consecutive elements at p (element index i) as float32.
-__device__ __forceinline__ void load8_f32(const void *p, int dtype, int vec, int64_t i, float (&x)[8]) {
-    if (vec && dtype != SS_F32) {
-        const uint4 u = *reinterpret_cast<const uint4 *>(static_cast<const char *>(p) + i * 2);
-        if (dtype == SS_F16)
-            unpack16<__half>(u, x);
-        else
-            unpack16<__hip_bfloat16>(u, x);
-    } else if (vec) {
-        const uint4 *u = reinterpret_cast<const uint4 *>(static_cast<const char *>(p) + i * 4);
-        unpack16<float>(u[0], x);
-        unpack16<float>(u[1], x + 4);
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = load_as_f32(p, dtype, i + e);
-    }
-}
 
 // Merge of split-T partials: one workgroup per (group, row).  One wave turns
 // the splits' (m, l) into weights exp2(m_s - M) and the merged l; every thread

@@ -118,6 +118,59 @@ __device__ __forceinline__ void store4_from_f32(void *p, int dt, int64_t i, floa
     store_from_f32(p, dt, i + 3, x3);
 }
 
+// The elements of a 16-byte piece as float32.
+template <typename T>
+__device__ __forceinline__ void unpack16(const uint4 &u, float *x);
+
+template <>
+__device__ __forceinline__ void unpack16<__half>(const uint4 &u, float *x) {
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        __half2 h = *reinterpret_cast<const __half2 *>(&w[i]);
+        float2 f = __half22float2(h);
+        x[2 * i] = f.x;
+        x[2 * i + 1] = f.y;
+    }
+}
+
+template <>
+__device__ __forceinline__ void unpack16<__hip_bfloat16>(const uint4 &u, float *x) {
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        x[2 * i] = __uint_as_float(w[i] << 16);
+        x[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
+}
+
+template <>
+__device__ __forceinline__ void unpack16<float>(const uint4 &u, float *x) {
+    x[0] = __uint_as_float(u.x);
+    x[1] = __uint_as_float(u.y);
+    x[2] = __uint_as_float(u.z);
+    x[3] = __uint_as_float(u.w);
+}
+
+// Eight consecutive elements at p (element index i) as float32;
+// vec: 16-byte aligned.
+__device__ __forceinline__ void load8_f32(const void *p, int dtype, int vec, int64_t i, float (&x)[8]) {
+    if (vec && dtype != SS_F32) {
+        const uint4 u = *reinterpret_cast<const uint4 *>(static_cast<const char *>(p) + i * 2);
+        if (dtype == SS_F16)
+            unpack16<__half>(u, x);
+        else
+            unpack16<__hip_bfloat16>(u, x);
+    } else if (vec) {
+        const uint4 *u = reinterpret_cast<const uint4 *>(static_cast<const char *>(p) + i * 4);
+        unpack16<float>(u[0], x);
+        unpack16<float>(u[1], x + 4);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = load_as_f32(p, dtype, i + e);
+    }
+}
+
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));

@@ -159,6 +159,126 @@ __global__ void __launch_bounds__(256)
     *wp = word;
 }
 
+// Whole token rows of the grouped quantiser: 256 threads take 256 / (d/8)
+// tokens, eight values each in one 16-byte load; a group's lanes share its
+// minimum and maximum, the codes meet in LDS and leave as packed words.
+// Element for element the float32 steps of quantize_grouped_kernel (one thread
+// a token there, so 8192 tokens of 128 dims were 32 workgroups of serial
+// 2-byte loads: 54 us, 6.1 here).  IL: straight into the interleaved codes,
+// scales and zeros of a cache at positions offset .. offset + n_t - 1 (the
+// codes of other tokens sharing a word are kept); a workgroup owns whole words.
+struct GroupQuantArgs {
+    const void *values;
+    int v_dtype, vec;
+    int64_t n_h, n_t, n_tok, v_sb, v_sh, v_st;
+    int d, bits, group;
+    uint32_t *codes;
+    void *scales, *zeros;
+    int sz_dtype;
+    int64_t o_sb, o_sh, o_st;  // packed rows
+    int64_t cap, offset;       // interleaved
+};
+
+template <bool IL>
+__global__ void __launch_bounds__(256) quantize_rows_kernel(GroupQuantArgs a) {
+    const int tid = threadIdx.x;
+    const int cpr = a.d / 8, W = 256 / cpr;  // chunks of a token, tokens of a workgroup
+    const int tl = tid / cpr, ch = tid - tl * cpr;
+    const int lpg = a.group / 8;  // lanes of a group
+    const int n_groups = a.d / a.group;
+    const int vpw = vals_per_word(a.bits);
+    const float maxv = (float)((1 << a.bits) - 1);
+    __shared__ __align__(16) uint8_t codes[256 * 8];  // [token][dim]
+
+    // the thread's token: row of the values, row of the scales
+    const int64_t p0 = IL ? a.offset / W * W + (int64_t)blockIdx.x * W : (int64_t)blockIdx.x * W;
+    bool live;
+    int64_t vin, orow;
+    if constexpr (IL) {
+        const int64_t b = blockIdx.y / a.n_h, h = blockIdx.y - b * a.n_h, t = p0 + tl - a.offset;
+        live = t >= 0 && t < a.n_t;
+        vin = b * a.v_sb + h * a.v_sh + t * a.v_st;
+        orow = blockIdx.y * a.cap + p0 + tl;
+    } else {
+        const int64_t n = p0 + tl;
+        live = n < a.n_tok;
+        const int64_t b = n / (a.n_h * a.n_t), rem = n - b * a.n_h * a.n_t;
+        const int64_t h = rem / a.n_t, t = rem - h * a.n_t;
+        vin = b * a.v_sb + h * a.v_sh + t * a.v_st;
+        orow = b * a.o_sb + h * a.o_sh + t * a.o_st;
+    }
+    float x[8] = {};
+    if (live) load8_f32(a.values, a.v_dtype, a.vec, vin + ch * 8, x);
+    float mn = INFINITY, mx = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        mn = fminf(mn, x[e]);
+        mx = fmaxf(mx, x[e]);
+    }
+    for (int o = 1; o < lpg; o <<= 1) {
+        mn = fminf(mn, __shfl_xor(mn, o));
+        mx = fmaxf(mx, __shfl_xor(mx, o));
+    }
+    float sc = __fdiv_rn(__fsub_rn(mx, mn), maxv);
+    if (sc < 1e-8f) sc = 1e-8f;
+    if (live && (ch & (lpg - 1)) == 0) {
+        store_from_f32(a.scales, a.sz_dtype, orow * n_groups + ch / lpg, sc);
+        store_from_f32(a.zeros, a.sz_dtype, orow * n_groups + ch / lpg, mn);
+    }
+    uint32_t w[2] = {0u, 0u};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float qf = fminf(fmaxf(rintf(__fdiv_rn(__fsub_rn(x[e], mn), sc)), 0.f), maxv);
+        w[e / 4] |= (uint32_t)qf << (e % 4 * 8);
+    }
+    *reinterpret_cast<uint2 *>(codes + tid * 8) = make_uint2(w[0], w[1]);
+    __syncthreads();
+
+    const uint32_t mask = (1u << a.bits) - 1u;
+    if constexpr (IL) {
+        for (int i = tid; i < W / vpw * a.d; i += 256) {
+            const int blk = i / a.d, dd = i - blk * a.d;
+            uint32_t word = 0u, keep = 0u;
+            for (int k = 0; k < vpw; ++k) {
+                const int64_t t = p0 + blk * vpw + k - a.offset;
+                const int pos = il_pos(a.bits, k);
+                if (t >= 0 && t < a.n_t)
+                    word |= (uint32_t)codes[(blk * vpw + k) * a.d + dd] << pos;
+                else
+                    keep |= mask << pos;
+            }
+            uint32_t *wp = a.codes + (blockIdx.y * (a.cap / vpw) + p0 / vpw + blk) * a.d + dd;
+            if (p0 + blk * vpw >= a.offset + a.n_t || p0 + (blk + 1) * vpw <= a.offset) continue;
+            *wp = keep ? (*wp & keep) | word : word;
+        }
+    } else {
+        const int nw = packed_words(a.d, a.bits);
+        for (int i = tid; i < W * nw; i += 256) {
+            const int tk = i / nw, wi = i - tk * nw;
+            const int64_t n = p0 + tk;
+            if (n >= a.n_tok) break;
+            uint32_t word = 0u;
+            for (int k = 0; k < vpw; ++k)
+                if (wi * vpw + k < a.d) word |= (uint32_t)codes[tk * a.d + wi * vpw + k] << (k * a.bits);
+            const int64_t b = n / (a.n_h * a.n_t), rem = n - b * a.n_h * a.n_t;
+            const int64_t h = rem / a.n_t, t = rem - h * a.n_t;
+            a.codes[(b * a.o_sb + h * a.o_sh + t * a.o_st) * nw + wi] = word;
+        }
+    }
+}
+
+// Whether quantize_rows_kernel takes this row shape: its lanes split rows and
+// groups evenly.
+static bool quantize_rows_ok(int d, int group) {
+    auto pow2 = [](int x) { return (x & (x - 1)) == 0; };
+    return d >= 8 && d <= 512 && pow2(d) && group >= 8 && pow2(group);
+}
+
+static int rows_vec(const void *p, int dtype, int64_t sb, int64_t sh, int64_t st) {
+    const int64_t sz = dtype_bytes(dtype);
+    return (uintptr_t)p % 16 == 0 && sb * sz % 16 == 0 && sh * sz % 16 == 0 && st * sz % 16 == 0;
+}
+
 // The inverse of pack_grouped_il_kernel: one thread per output packed word
 // (row t of (B, H) row bh, word w) gathers its vpw dims' codes of token t.
 __global__ void __launch_bounds__(256)
@@ -270,6 +390,20 @@ extern "C" int ss_quantize_values_grouped(const void *values, int v_dtype, int64
     SS_REQUIRE(values && packed && scales && zeros, "null pointer argument");
     SS_UNSUPPORTED(n_tok < (1LL << 32), "too many tokens for one launch");
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    // (other shapes: one thread a token)
+    if (quantize_rows_ok(head_dim, group_size)) {
+        const int W = 256 / (head_dim / 8);
+        const GroupQuantArgs a{values,   v_dtype, rows_vec(values, v_dtype, v_sb, v_sh, v_st),
+                               n_h,      n_t,     n_tok,
+                               v_sb,     v_sh,    v_st,
+                               head_dim, bits,    group_size,
+                               packed,   scales,  zeros,
+                               sz_dtype, o_sb,    o_sh,
+                               o_st,     0,       0};
+        hipLaunchKernelGGL(quantize_rows_kernel<false>, dim3((unsigned)((n_tok + W - 1) / W)), dim3(256), 0, st, a);
+        SS_LAUNCH_CHECK("quantize_rows_kernel launch");
+        return SS_OK;
+    }
     hipLaunchKernelGGL(quantize_grouped_kernel, dim3(blocks_for(n_tok)), dim3(256), 0, st, values,
                        v_dtype, n_h, n_t, n_tok, v_sb, v_sh, v_st, head_dim, bits, group_size,
                        packed, scales, zeros, sz_dtype, o_sb, o_sh, o_st);
@@ -364,6 +498,41 @@ extern "C" int ss_pack_grouped_il(const uint32_t *packed, int64_t n_b, int64_t n
                        dim3(256), 0, st, packed, n_h, n_t, p_sb, p_sh, p_st, head_dim, bits, out_il,
                        cap, offset, b0, n_blk);
     SS_LAUNCH_CHECK("pack_grouped_il_kernel launch");
+    return SS_OK;
+}
+
+extern "C" int ss_append_values_grouped_il(const void *values, int v_dtype, int64_t n_b, int64_t n_h,
+                                           int64_t n_t, int64_t v_sb, int64_t v_sh, int64_t v_st,
+                                           int head_dim, int bits, int group_size, uint32_t *codes_il,
+                                           void *scales, void *zeros, int sz_dtype, int64_t cap,
+                                           int64_t offset, void *stream) {
+    SS_REQUIRE(valid_dtype(v_dtype), "bad value dtype");
+    SS_REQUIRE(sz_dtype == SS_F32 || sz_dtype == SS_F16, "scale/zero dtype must be f32 or f16");
+    SS_REQUIRE(bits == 2 || bits == 4, "interleaved codes need bits 2 or 4 (got %d)", bits);
+    SS_REQUIRE(head_dim >= 1 && group_size >= 1 && head_dim % group_size == 0,
+               "head_dim %d not divisible by group_size %d", head_dim, group_size);
+    SS_UNSUPPORTED((head_dim == 64 || head_dim == 128) && quantize_rows_ok(head_dim, group_size),
+                   "head_dim %d, group_size %d unsupported (64 or 128, a power of two >= 8)", head_dim,
+                   group_size);
+    SS_REQUIRE(n_b >= 0 && n_h >= 0 && n_t >= 0 && offset >= 0, "negative sizes");
+    SS_REQUIRE(cap % (32 / bits) == 0, "cap must be a multiple of %d", 32 / bits);
+    SS_REQUIRE(offset + n_t <= cap, "append range [%lld, %lld) past cap %lld", (long long)offset,
+               (long long)(offset + n_t), (long long)cap);
+    if (n_b * n_h * n_t == 0) return SS_OK;
+    SS_REQUIRE(values && codes_il && scales && zeros, "null pointer argument");
+    SS_UNSUPPORTED(n_b * n_h < 65536, "too many (batch, head) rows for one launch");
+    const int W = 256 / (head_dim / 8);  // tokens of a workgroup: a multiple of a word's
+    const int64_t n_wg = (offset + n_t - 1) / W - offset / W + 1;
+    const GroupQuantArgs a{values,   v_dtype, rows_vec(values, v_dtype, v_sb, v_sh, v_st),
+                           n_h,      n_t,     n_b * n_h * n_t,
+                           v_sb,     v_sh,    v_st,
+                           head_dim, bits,    group_size,
+                           codes_il, scales,  zeros,
+                           sz_dtype, 0,       0,
+                           0,        cap,     offset};
+    hipLaunchKernelGGL(quantize_rows_kernel<true>, dim3((unsigned)n_wg, (unsigned)(n_b * n_h)), dim3(256), 0,
+                       reinterpret_cast<hipStream_t>(stream), a);
+    SS_LAUNCH_CHECK("quantize_rows_kernel launch");
     return SS_OK;
 }
 

@@ -276,3 +276,37 @@ def test_dequantised_rows_are_the_codebook_rows(nb, bd, n, dtype, use_perm, pad)
     rows = cents[torch.arange(nb, device="cuda"), idx.long().clamp(max=199)].flatten(1)
     want = rows[:, inv.long()] if use_perm else rows
     assert torch.equal(got, want.to(dtype))  # one rounding each
+
+
+@pytest.mark.parametrize("bits,d,group,n_t,offset,cap,dtype,sz,pad", [
+    (2, 128, 64, 1, 5, 32, torch.float16, torch.float16, 0),       # one token inside a word
+    (2, 128, 128, 40, 30, 96, torch.bfloat16, torch.float32, 0),   # partial words at both ends
+    (4, 128, 64, 33, 8, 64, torch.float16, torch.float16, 1),      # rows at odd addresses
+    (4, 64, 32, 100, 29, 160, torch.float32, torch.float16, 0),    # head_dim 64
+    (2, 64, 64, 64, 32, 96, torch.float16, torch.float32, 0),      # whole workgroups
+])
+def test_append_grouped_il_is_quantise_then_interleave(bits, d, group, n_t, offset, cap, dtype, sz, pad):
+    """Codes, scales and zeros are the oracle's, and what other tokens hold
+    (also in shared words) is left alone."""
+    g = torch.Generator(device="cuda").manual_seed(n_t + d)
+    v = torch.randn((2, 3, n_t, d + pad), generator=g, device="cuda").to(dtype)[..., pad:]
+    il = torch.randint(-2**31, 2**31 - 1, (2, 3, cap * bits // 32, d), generator=g, device="cuda",
+                       dtype=torch.int32)
+    sc, ze = (torch.full((2, 3, cap, d // group), 7.0, device="cuda", dtype=sz) for _ in range(2))
+    old = _hip.grouped_il_to_packed(il, bits, cap)
+    _hip.append_values_grouped_il(v, bits, group, il, sc, ze, offset)
+    rows = torch.zeros((2, 3, n_t, d * bits // 32), dtype=torch.int32, device="cuda")
+    s1, z1 = (torch.zeros((2, 3, n_t, d // group), dtype=sz, device="cuda") for _ in range(2))
+    _hip.quantize_values_grouped(v, bits, group, rows, s1, z1)
+    packed, osc, oze, _ = O.quantize_values(v.float().cpu().numpy().reshape(-1, d), bits, group)
+    assert np.array_equal(rows.cpu().numpy().reshape(packed.shape).view(np.uint32), packed)
+    assert np.array_equal(s1.cpu().numpy().reshape(osc.shape), osc.astype(s1.cpu().numpy().dtype))
+    assert np.array_equal(z1.cpu().numpy().reshape(oze.shape), oze.astype(z1.cpu().numpy().dtype))
+    new = _hip.grouped_il_to_packed(il, bits, cap).view(torch.int32)
+    want = old.view(torch.int32).clone()
+    want[:, :, offset:offset + n_t] = rows
+    assert torch.equal(new, want)
+    for got, one in ((sc, s1), (ze, z1)):
+        full = torch.full_like(got, 7.0)
+        full[:, :, offset:offset + n_t] = one
+        assert torch.equal(got, full)
