@@ -328,6 +328,21 @@ class SunShapeBlockCodec:
         dims = (hb[:, None] * bd + torch.arange(bd, device=hb.device)[None]).flatten()
         return dims.to(torch.int32).to(self.device)
 
+    def _any_heavy(self) -> bool:
+        """Whether :meth:`heavy_dims` is not None.  Reading the mask waits for
+        the GPU, so the answer is kept with the mask and read again when it
+        changes (another tensor or an in-place update)."""
+        if self.mode != "profileperm_mixed_precision" or not self.heavy_fp16:
+            return False
+        hb = self.mixed_high_precision_blocks
+        if hb.is_inference():  # no version to tell an in-place update by
+            return bool(hb.any())
+        held = getattr(self, "_heavy_seen", None)
+        if held is None or held[0] is not hb or held[1] != hb._version:
+            held = (hb, hb._version, bool(hb.any()))
+            self._heavy_seen = held
+        return held[2]
+
     def kernel_value_transform(self) -> torch.Tensor:
         """(D, D) float32 matrix taking a codec-space row to the original
         basis, ``x_orig = x_codec @ M`` (the inverse permutation as a 0/1
@@ -366,7 +381,7 @@ class SunShapeBlockCodec:
         (codec.py:575-637).  Cached until the centroids or the heavy mask
         change."""
         c = self.centroids
-        if self.heavy_dims() is None:
+        if not self._any_heavy():
             return c
         hb = self.mixed_high_precision_blocks
         key = (c.data_ptr(), c._version, hb.data_ptr(), hb._version, str(c.device))
