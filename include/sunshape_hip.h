@@ -707,6 +707,22 @@ typedef struct {
 } ss_attn_mask;
 
 /*
+ * ss_decode_attn_turboquant's 3- and 4-bit values on the matrix cores: its
+ * arguments with the prepared codebook (ss_codebook_f16x2) for the centroids.
+ * SS_ERR_UNSUPPORTED for 2 bits, more than 32 heavy key dims, heavy dims with
+ * a mask, and level tables whose largest magnitude is not within 1e-30 .. 1e30.
+ */
+int ss_decode_attn_turboquant_mfma(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint32_t *packed, const float *norms,
+    const float *levels, const float *rotation, int bits, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims, int n_heavy_dims,
+    int causal, int64_t q_offset, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
+    int n_splits, void *stream);
+
+/*
  * The decodes above under a mask (the reference takes its two-pass path,
  * attention.py:236-246, 307-350): ss_decode_attn_il8_hybrid,
  * _dense_mfma, _grouped_il_hybrid, _turboquant_il, _turboquant,
@@ -751,6 +767,15 @@ int ss_decode_attn_turboquant_il_masked(
 int ss_decode_attn_turboquant_masked(
     const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
     int head_dim, float scale, const int32_t *perm, const float *centroids, int n_blocks,
+    int n_centroids, const uint8_t *idx, const uint32_t *packed, const float *norms,
+    const float *levels, const float *rotation, int bits, int64_t cap, int64_t t_kv,
+    const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,
+    int64_t buf_st, int64_t t_buf, const void *k_heavy, const int32_t *heavy_dims, int n_heavy_dims,
+    int causal, int64_t q_offset, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
+    int n_splits, const ss_attn_mask *mask, void *stream);
+int ss_decode_attn_turboquant_mfma_masked(
+    const void *q, int q_dtype, int64_t batch, int n_q_heads, int n_kv_heads, int64_t t_q,
+    int head_dim, float scale, const int32_t *perm, const void *codebook, int n_blocks,
     int n_centroids, const uint8_t *idx, const uint32_t *packed, const float *norms,
     const float *levels, const float *rotation, int bits, int64_t cap, int64_t t_kv,
     const void *k_buf, const void *v_buf, int buf_dtype, int64_t buf_sb, int64_t buf_sh,

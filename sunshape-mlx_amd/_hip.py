@@ -154,6 +154,11 @@ _SIGNATURES = {
         _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _int, _i64, _i64,
         _c_void_p, _c_void_p, _int, _i64, _i64, _i64, _i64, _c_void_p, _c_void_p, _int,
         _int, _i64, _c_void_p, _int, _c_void_p, _size, _int, _c_void_p]),
+    "ss_decode_attn_turboquant_mfma": (_int, [
+        _c_void_p, _int, _i64, _int, _int, _i64, _int, _f32, _c_void_p, _c_void_p, _int, _int,
+        _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _int, _i64, _i64,
+        _c_void_p, _c_void_p, _int, _i64, _i64, _i64, _i64, _c_void_p, _c_void_p, _int,
+        _int, _i64, _c_void_p, _int, _c_void_p, _size, _int, _c_void_p]),
     "ss_decode_turboquant_workspace_bytes": (_size, [_i64, _int, _int, _i64, _int, _i64, _i64,
                                                      _int]),
     "ss_decode_attn_turboquant_il": (_int, [
@@ -215,7 +220,7 @@ _SIGNATURES = {
 _MASKED = {"ss_decode_attn_il8_hybrid": "ss_decode_attn_il8_masked",
            "ss_decode_attn_grouped_il_hybrid": "ss_decode_attn_grouped_il_masked",
            **{f"ss_decode_attn_{n}": f"ss_decode_attn_{n}_masked"
-              for n in ("dense_mfma", "turboquant_il", "turboquant", "grouped_hybrid",
+              for n in ("dense_mfma", "turboquant_il", "turboquant", "turboquant_mfma", "grouped_hybrid",
                         "dense_hybrid", "sunshape_v")}}
 for _plain, _masked in _MASKED.items():
     _r, _a = _SIGNATURES[_plain]
@@ -1635,16 +1640,19 @@ def decode_attn_turboquant(q: torch.Tensor, scale: float, perm: torch.Tensor | N
                            buf_values: torch.Tensor | None = None,
                            buf_len: int = 0, k_heavy: torch.Tensor | None = None,
                            heavy_dims: torch.Tensor | None = None,
-                           mask: AttnMask | None = None) -> torch.Tensor:
+                           mask: AttnMask | None = None,
+                           codebook: torch.Tensor | None = None) -> torch.Tensor:
     """Fused decode over TurboQuant values: ``packed`` (B, Hkv, cap,
     packed_dim) codes, ``norms`` (B, Hkv, cap) float32, ``levels`` the 2^bits
     scaled Lloyd-Max levels (any float sequence; copied to the kernel
     arguments), ``rotation`` (D, D) float32 with ``value = norm * (levels[code]
     @ rotation)``.  A hybrid cache's recent tokens ``buf_keys``/``buf_values``
     (B, Hkv, >= buf_len, D, original basis) join the same softmax as
-    positions t_kv .. t_kv + buf_len - 1."""
+    positions t_kv .. t_kv + buf_len - 1.  With the prepared ``codebook``
+    (:func:`codebook_f16x2`) of the centroids, 3- and 4-bit values run on the
+    matrix cores where that kernel takes the call."""
     _check_decode_common(q, idx, centroids, perm)
-    require_gpu(packed, norms, rotation)
+    require_gpu(packed, norms, rotation, codebook)
     b_, hq, tq, d = q.shape
     _, hkv, cap, nb = idx.shape
     if packed.dim() != 4 or not packed.is_contiguous() or packed.shape[:3] != idx.shape[:3] or \
@@ -1670,12 +1678,30 @@ def decode_attn_turboquant(q: torch.Tensor, scale: float, perm: torch.Tensor | N
     ws_bytes = lib.ss_decode_turboquant_workspace_bytes(b_, hq, hkv, tq, d, int(t_kv), buf_len,
                                                         int(n_splits))
     ws = decode_workspace(q.device, ws_bytes)
-    _launched(_attn_stat("sunshape_fused_attention_turboquant", causal), _masked_call("ss_decode_attn_turboquant", (
-        ptr(q), dtype_code(q.dtype), b_, hq, hkv, tq, d, float(scale), ptr(perm), ptr(centroids),
-        nb, nc, ptr(idx), ptr(packed), ptr(norms), ctypes.cast(lv_host, ctypes.c_void_p).value,
-        ptr(rotation), int(bits), cap, int(t_kv), ptr(buf_keys), ptr(buf_values), bdt, bsb, bsh,
-        bst, buf_len, *_heavy_args(k_heavy, heavy_dims, b_, hkv, cap, 64), int(bool(causal)), int(q_offset), ptr(out), dtype_code(out.dtype), ptr(ws),
-        ws_bytes if ws is not None else 0, int(n_splits), stream_handle(q.device)), mask))
+    def call(name, cb):
+        return _masked_call(name, (
+            ptr(q), dtype_code(q.dtype), b_, hq, hkv, tq, d, float(scale), ptr(perm), ptr(cb),
+            nb, nc, ptr(idx), ptr(packed), ptr(norms), ctypes.addressof(lv_host),
+            ptr(rotation), int(bits), cap, int(t_kv), ptr(buf_keys), ptr(buf_values), bdt, bsb, bsh,
+            bst, buf_len, *_heavy_args(k_heavy, heavy_dims, b_, hkv, cap, 64), int(bool(causal)),
+            int(q_offset), ptr(out), dtype_code(out.dtype), ptr(ws),
+            ws_bytes if ws is not None else 0, int(n_splits), stream_handle(q.device)), mask)
+
+    stat = _attn_stat("sunshape_fused_attention_turboquant", causal)
+    # one query row a KV head leaves three of the matrix-core kernel's four rows
+    # empty: 4 x 16001 tokens of 16 heads 46 us there and 45 here at 128 dims,
+    # 33 and 28 at 64; two rows 46 and 62, 33 and 39
+    if codebook is not None and bits != 2 and hq // hkv * tq >= 2:
+        _poll_waits(q.device)
+        try:
+            _launched(stat, call("ss_decode_attn_turboquant_mfma", codebook))
+        except SunShapeUnsupported:
+            pass
+        else:
+            if _check_waits:
+                check_decode_waits(q.device)
+            return out
+    _launched(stat, call("ss_decode_attn_turboquant", centroids))
     return out
 
 

@@ -354,6 +354,7 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
             out = _hip.decode_attn_turboquant(q, kscale, perm, codec.centroids, ops["idx"],
                                               ops["packed"], ops["norms"], ops["levels"],
                                               ops["rotation"], ops["bits"],
+                                              codebook=codec.kernel_codebook(),
                                               buf_keys=ops["buf_keys"], buf_values=ops["buf_values"],
                                               buf_len=buffered, **hv, **kw)
             codec.last_score_backend = ("hip_fused_turboquant_buffer" if buffered

@@ -496,6 +496,10 @@ __device__ __forceinline__ void load_code_words(uint32_t (&cw)[2][NT], const uin
     }
 }
 template <class VF, class = void>
+struct VfTable : std::false_type {};  // the format reads a table in LDS (VF::stage_table)
+template <class VF>
+struct VfTable<VF, std::void_t<decltype(VF::kTable)>> : std::bool_constant<VF::kTable> {};
+template <class VF, class = void>
 struct VfArgsToLds : std::false_type {};  // the format's accumulator hand-off reads its Args
 template <class VF>
 struct VfArgsToLds<VF, std::void_t<decltype(&VF::to_lds_args)>> : std::true_type {};
@@ -1913,6 +1917,203 @@ struct VTq {
     }
 };
 
+// TurboQuant values of 3 or 4 bits on the matrix cores, from the packed rows
+// the cache keeps ([cap][NW] words per (b, h), one token a row).  The B
+// operand wants pairs of tokens of one dim: two rows' words interleave by bit
+// fields (token a's codes of the even dims beside token b's, and of the odd
+// dims), so one field is the pair's index into a table in LDS whose 8-byte
+// entry holds both levels as fp16 hi and lo parts (levels scaled to 2^14 ..:
+// 22 bits each) -- one LDS read per two values.  A holds w = p * norm as three
+// fp16 parts (rows 0-3, 4-7, 8-11: more than float32's 24 bits for weights
+// within 2^15 of the largest); norms enter relative to a power of two 2^e a
+// wave keeps at its largest norm so far, so any float32 norm fits.  Lane
+// (g, l16) takes the codes of dims NT*l16 .. and tokens 4j + g, whose slot in
+// the K order is 8g + j: a load of the wave covers whole rows.
+// Bound: the LDS reads (32 table reads beside the 16 LUT reads of a token's
+// scores a lane and 64 tokens).  B=4, T=16001, 32/8 heads of 128 dims, 4 bits
+// (43 MB), per dispatch under the profiler: 34.8 us on the vector ALUs, 23.4
+// here.
+template <int D, int BITS>
+struct VTqRows {
+    struct Args {
+        const uint32_t *packed;  // [rows][NW]
+        const float *norms;      // [rows]
+        float lv[16];            // the 2^BITS levels times the power of two 1 / linv
+        float linv;
+    };
+    static constexpr int NT = D / 16;
+    static constexpr int VPW = 32 / BITS;
+    static constexpr int NW = (D + VPW - 1) / VPW;
+    static constexpr bool kPrivateRing = true;
+    static constexpr int kSub = 1;
+    static constexpr bool kHybridBuffer = false;  // the buffer joins in the merge
+    static constexpr bool kHeavyCapable = true;
+    static constexpr int kTileV = D == 64 ? 1280 : 2048;  // (the ring holds the table, then the merges)
+    static constexpr int kLoadsV = 2;
+    static constexpr int kPRows = 12;
+    static constexpr int kMaxSlots = 16;
+    static constexpr int kComputeWaves = 8;
+    static constexpr bool kRegUnits = true;
+    static constexpr float kMaxLag = 4.f;    // fp16 weights: p <= 2^4
+    static constexpr float kWScale = 1024.f;  // ... times a norm below 2, staged times 2^10
+    static constexpr int kPairs = 1 << (2 * BITS);
+    static constexpr bool kTable = true;
+    struct Tile {
+        uint32_t w[2][8];  // [32-token half][j]: the lane's NT codes of token 4j + g, lowest first
+        float n;           // norm of token `lane`
+    };
+    struct Raw {
+        uint32_t w[2][8];
+        float n;
+    };
+    struct State {
+        uint32_t tab;  // LDS address of the table
+        int e;         // exponent the norms are taken relative to, and 2^-e
+        float ninv;
+    };
+    __device__ static void load(Raw &u, const Args &a, int64_t bh, int64_t cap, int64_t t0, int64_t t_last,
+                                int lane) {
+        const int g = lane >> 4, l16 = lane & 15;
+        const uint32_t last = (uint32_t)min(t_last - t0, (int64_t)kWave - 1);
+        const char *base = reinterpret_cast<const char *>(a.packed + (bh * cap + t0) * NW);
+        // the four bytes from the one that holds the lane's first code: its NT
+        // codes and, at 3 bits, the two unused bits of a word they straddle
+        // (30 bits at most; the last lane's codes end its row)
+        const uint32_t bit = first_bit(l16);
+        base += bit / 8;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t tk = min((uint32_t)(32 * ks + 4 * j + g), last);
+                __builtin_memcpy(&u.w[ks][j], base + tk * (NW * 4u), 4);
+            }
+        u.n = a.norms[bh * cap + min(t0 + lane, t_last)];
+    }
+    __device__ static void from_raw(Tile &tv, const Raw &u, int lane) {
+        const int l16 = lane & 15;
+        const uint32_t sh = first_bit(l16) % 8;
+        // 3 bits: the codes left in the first word, then (past its two unused
+        // bits) those of the next
+        const int n0 = min(VPW - NT * l16 % VPW, NT);
+        const uint32_t keep = n0 < NT ? (1u << (BITS * n0)) - 1u : 0xffffffffu;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t x = u.w[ks][j] >> sh;
+                tv.w[ks][j] = BITS == 3 ? (x & keep) | ((x >> 2) & ~keep) : x;
+            }
+        tv.n = u.n;
+    }
+    // bit of a row at which lane l16's codes start
+    __device__ static uint32_t first_bit(int l16) {
+        return (uint32_t)(NT * l16 / VPW * 32 + NT * l16 % VPW * BITS);
+    }
+    // the level pairs of code a | code b << BITS, at LDS address tab
+    __device__ static void stage_table(uint32_t tab, const Args &a, int tid, int nt) {
+        auto level = [&](int code) {
+            float v = a.lv[0];
+#pragma unroll
+            for (int i = 1; i < (1 << BITS); ++i) v = code == i ? a.lv[i] : v;
+            return v;
+        };
+        auto bits = [](_Float16 x) { return (uint32_t)__builtin_bit_cast(uint16_t, x); };
+        for (int i = tid; i < kPairs; i += nt) {
+            const float x = level(i & ((1 << BITS) - 1)), y = level(i >> BITS);
+            const _Float16 xh = (_Float16)x, yh = (_Float16)y;
+            const _Float16 xl = (_Float16)(x - (float)xh), yl = (_Float16)(y - (float)yh);
+            reinterpret_cast<lds_t<u32x2> *>(tab)[i] =
+                u32x2{bits(xh) | (bits(yh) << 16), bits(xl) | (bits(yl) << 16)};
+        }
+    }
+    __device__ static void issue(const Args &, int64_t, int64_t, int64_t, int64_t, uint32_t, int) {}
+    __device__ static void init(State &st) {
+        st.e = -126;
+        st.ninv = exp2i(126);
+    }
+    __device__ static void pv(Tile &tv, State &st, f32x4 (&acc)[NT], const float (&p)[kMfmaRows],
+                              const float (&corr)[kMfmaRows], bool rescale, int n_in, _Float16 *pw,
+                              int lane) {
+        const int g = lane >> 4, l16 = lane & 15;
+        float n = tv.n;
+        if (n_in < kWave) n = lane < n_in ? n : 0.f;  // past the split's end: p = 0
+        if (rescale) {
+            const f32x4 cv4 = f32x4{corr[0], corr[1], corr[2], corr[3]};
+#pragma unroll
+            for (int k = 0; k < NT; ++k) acc[k] *= cv4;
+        }
+        if (__builtin_amdgcn_ballot_w64(!(fabsf(n) * st.ninv < 2.f)) != 0) {
+            const float mx = wave_max(fabsf(n));
+            const int e = max(st.e, min((int)(__float_as_uint(mx) >> 23) - 127, 126));
+            const float f = exp2i(max(st.e - e, -126));
+#pragma unroll
+            for (int k = 0; k < NT; ++k) acc[k] *= f;
+            st.e = e;
+            st.ninv = exp2i(-e);
+        }
+        const float nw = n * st.ninv * kWScale;
+        const int slot = (lane & 32) + 8 * (lane & 3) + ((lane & 31) >> 2);
+#pragma unroll
+        for (int r = 0; r < kMfmaRows; ++r) {
+            float x = p[r] * nw;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {  // each part the rounded rest
+                const _Float16 h = (_Float16)x;
+                x -= (float)h;
+                pw[(4 * k + r) * kPStride + slot] = h;
+            }
+        }
+        wave_lds_sync();
+        constexpr uint32_t lowf = BITS == 4 ? 0x0f0f0f0fu : 0x071c71c7u;  // every other field
+        constexpr uint32_t idx_mask = (uint32_t)(kPairs - 1) * 8u;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            uint4 av = make_uint4(0u, 0u, 0u, 0u);
+            if (l16 < 12) av = *reinterpret_cast<const uint4 *>(pw + l16 * kPStride + 32 * ks + 8 * g);
+            const f16x8 a = __builtin_bit_cast(f16x8, av);
+            uint32_t pe[4], po[4];  // a pair's fields: even dims, odd dims
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t wa = tv.w[ks][2 * q], wb = tv.w[ks][2 * q + 1];
+                pe[q] = (wa & lowf) | ((wb << BITS) & ~lowf);
+                po[q] = ((wa >> BITS) & lowf) | (wb & ~lowf);
+            }
+#pragma unroll
+            for (int k = 0; k < NT; ++k) {
+                u32x2 t[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t f = k & 1 ? po[q] : pe[q];
+                    const int sh = 2 * BITS * (k / 2) - 3;  // the field, times the entry size
+                    const uint32_t off = (sh >= 0 ? f >> sh : f << -sh) & idx_mask;
+                    t[q] = *reinterpret_cast<const lds_t<u32x2> *>(st.tab + off);
+                }
+                acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    a, __builtin_bit_cast(f16x8, make_uint4(t[0].x, t[1].x, t[2].x, t[3].x)), acc[k], 0, 0, 0);
+                acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    a, __builtin_bit_cast(f16x8, make_uint4(t[0].y, t[1].y, t[2].y, t[3].y)), acc[k], 0, 0, 0);
+            }
+        }
+        wave_lds_sync();
+    }
+    // lanes 0-15 hold rows 0-3 (hi), 16-31 the mid and 32-47 the lo parts
+    __device__ static void to_lds_args(const f32x4 (&acc)[NT], const State &st, const Args &a, float *wa,
+                                       int lane) {
+        const int g = lane >> 4, l16 = lane & 15;
+        const float f = a.linv * (1.f / kWScale), fe = exp2i(st.e);
+#pragma unroll
+        for (int r = 0; r < kMfmaRows; ++r)
+#pragma unroll
+            for (int k = 0; k < NT; ++k) {
+                const float up = __shfl(acc[k][r], (lane + 16) & (kWave - 1));
+                if (g < 2)
+                    wa[(g * kMfmaRows + r) * D + NT * l16 + k] =
+                        (g == 0 ? acc[k][r] : acc[k][r] + up) * f * fe;
+            }
+    }
+};
+
 // ds_read_b64_tr_b16 at LDS byte address `addr`: in each 16-lane group, lane j
 // reads 4 halves; lane i receives column i of the 4 x 16 block they form (row
 // r from lane 4r + i/4, element i%4).
@@ -2286,6 +2487,11 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
     for (int n = 0; n < NT; ++n) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
     typename VF::State vst;
     VF::init(vst);
+    if constexpr (VfTable<VF>::value) {  // ordered by the prologue's barriers
+        static_assert(kRegs && K::kRingBytes >= VF::kPairs * 8, "table in the unused ring");
+        vst.tab = ring_l;
+        VF::stage_table(ring_l, va, tid, THREADS);
+    }
     // running maxima; a row past the last query row gets a maximum no score
     // reaches, so its probabilities are 0 and it never forces a reduction
     float m[R], lsum[R];

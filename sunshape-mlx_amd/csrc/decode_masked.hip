@@ -32,6 +32,10 @@ SS_MASKED(128, VBf16<128>)
 SS_MASKED(64, VBf16<64>)
 SS_MASKED(128, VTq<128>)
 SS_MASKED(64, VTq<64>)
+SS_MASKED(128, VTqRows<128, 3>)
+SS_MASKED(128, VTqRows<128, 4>)
+SS_MASKED(64, VTqRows<64, 3>)
+SS_MASKED(64, VTqRows<64, 4>)
 SS_MASKED_GIL(128, 2)
 SS_MASKED_GIL(128, 4)
 SS_MASKED_GIL(64, 2)

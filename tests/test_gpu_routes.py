@@ -310,3 +310,57 @@ def test_append_grouped_il_is_quantise_then_interleave(bits, d, group, n_t, offs
         full = torch.full_like(got, 7.0)
         full[:, :, offset:offset + n_t] = one
         assert torch.equal(got, full)
+
+
+@pytest.mark.parametrize("bits,d,hq,t_kv,t_buf,t_q,splits,spread,qdt", [
+    (4, 128, 8, 1, 0, 1, 0, 0, torch.float16),       # one token, the kernel rotates
+    (4, 128, 8, 64, 0, 1, 1, 0, torch.float16),      # one unit, one split
+    (3, 128, 8, 65, 5, 1, 0, 0, torch.bfloat16),     # a unit and one token, buffered tokens
+    (3, 64, 8, 700, 0, 1, 0, 0, torch.float32),      # head_dim 64: words straddled by dims
+    (4, 64, 6, 1500, 9, 1, 3, 20, torch.float16),    # norms over 40 powers of two
+    (3, 128, 8, 3000, 0, 3, 0, 20, torch.float32),   # ... causal rows
+    (4, 128, 14, 5001, 130, 1, 0, 0, torch.float32),  # seven heads a group
+])
+def test_turboquant_rows_on_the_matrix_cores(bits, d, hq, t_kv, t_buf, t_q, splits, spread, qdt):
+    """3/4-bit TurboQuant values read from their packed rows; no less exact
+    than the vector-ALU kernel of the same call (1e-6 of the largest output
+    for float32 rounding: ~16 roundings of 2^-24 in either)."""
+    b, hkv, cap = 2, 2, t_kv + 37
+    cents, perm, idx, _, q = decode_case(31 * t_kv + bits, b, hq, hkv, d, t_kv, t_q, cap)
+    rng = np.random.default_rng(t_kv)
+    codes = rng.integers(0, 1 << bits, (b, hkv, cap, d)).astype(np.uint8)
+    packed = O.pack_indices(codes, bits).astype(np.uint32)
+    norms = ((rng.random((b, hkv, cap)) + 0.1) *
+             np.exp2(rng.integers(-spread, spread + 1, (b, hkv, cap)))).astype(np.float32)
+    norms[:, :, t_kv:] = np.nan  # never read as a token
+    levels = (O.lloyd_max_gaussian(bits)[0] / np.sqrt(d)).astype(np.float32)
+    rot = O.rotation_matrix(d, 43)
+    vals = O.turboquant_decode(packed[:, :, :t_kv], norms[:, :, :t_kv], rot, levels, d, bits)
+    kb, vb = (rng.standard_normal((b, hkv, max(t_buf, 1), d)).astype(np.float32) for _ in range(2))
+    qd = torch.from_numpy(q).to(qdt)
+    scale = 1.0 / np.sqrt(d)
+    kw = dict(causal=t_q > 1, q_offset=t_kv + t_buf - t_q if t_q > 1 else 0, out_dtype=torch.float32,
+              n_splits=splits)
+    if t_buf:
+        kw.update(buf_keys=t(kb), buf_values=t(vb), buf_len=t_buf)
+    cb = _hip.codebook_f16x2(t(cents))
+    args = (qd.cuda(), scale, t(perm), t(cents), t(idx), t(packed.view(np.int32)), t(norms), levels,
+            t(rot), bits, t_kv)
+    outs = [_hip.decode_attn_turboquant(*args, codebook=c, **kw) for c in (cb, None)]
+    # the definition in float64
+    kc = np.stack([np.stack([O.dequantize_blockvq(idx[i, h, :t_kv], cents) for h in range(hkv)])
+                   for i in range(b)]).astype(np.float64)
+    qs = (qd * scale).double().numpy()
+    inv = np.argsort(perm)
+    kx = np.concatenate([kc[..., inv], kb[:, :, :t_buf].astype(np.float64)], 2)
+    vx = np.concatenate([vals.astype(np.float64), vb[:, :, :t_buf].astype(np.float64)], 2)
+    rep = hq // hkv
+    sc = qs @ np.repeat(kx, rep, 1).transpose(0, 1, 3, 2)
+    if t_q > 1:
+        hide = np.arange(t_kv + t_buf)[None] > kw["q_offset"] + np.arange(t_q)[:, None]
+        sc = np.where(hide, -np.inf, sc)
+    p = np.exp(sc - sc.max(-1, keepdims=True))
+    want = (p / p.sum(-1, keepdims=True)) @ np.repeat(vx, rep, 1)
+    err, ref = (rel_err(o.cpu().numpy(), want) for o in outs)
+    print("error", err, "vector-ALU kernel", ref)
+    assert err <= REL_TOL and err <= ref + 1e-6
