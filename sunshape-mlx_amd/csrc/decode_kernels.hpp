@@ -4428,7 +4428,9 @@ struct MergeBuffer {
 // One slot of the partials stays reserved for the buffer and is not read.
 // As a launch of its own, one workgroup per column with a token per thread
 // and element loads, the buffer took 85 us at 32 columns (B = 4, 128 tokens)
-// and 105 us at 128; the merge with it takes 14.8 and 18.4 us (5.5 without).
+// and 105 us at 128; the merge with it takes 12.5 and 15.6 us (5.5 without; 14.8
+// and 18.4 with loads under per-load tests of the type, which are waited for
+// one by one).
 template <int D, bool BUF>
 __global__ void __launch_bounds__(kDecodeThreads)
     decode_merge_kernel(DecodeCommon c, int R, const float *rot, void *rot_out, int rot_dtype,
@@ -4469,19 +4471,33 @@ __global__ void __launch_bounds__(kDecodeThreads)
         const int64_t n = min(mb.n, lim);
         const int64_t base = bb * mb.sb + kvh * mb.sh + dl * 8;
         const int64_t mrow = bb * c.m_sb + (kvh * c.rep + rr) * c.m_sh + tq * c.m_sq;
+        // (a load under its own test of the type is waited for by itself)
+        const bool raw16 = mb.vec && mb.dtype != SS_F32;
         for (int64_t j0 = 0; j0 < n; j0 += BT) {
-            float kx[PASSES][8], vx[PASSES][8];
+            uint4 kr[PASSES], vr[PASSES];  // 16-bit rows, aligned
+            if (raw16) {
 #pragma unroll
-            for (int i = 0; i < PASSES; ++i) {
-                const int64_t j = min(j0 + tg + i * TPG, n - 1);
-                load8_f32(mb.k, mb.dtype, mb.vec, base + j * mb.st, kx[i]);
-                load8_f32(mb.v, mb.dtype, mb.vec, base + j * mb.st, vx[i]);
+                for (int i = 0; i < PASSES; ++i) {
+                    const int64_t j = min(j0 + tg + i * TPG, n - 1);
+                    kr[i] = *reinterpret_cast<const uint4 *>(static_cast<const char *>(mb.k) + (base + j * mb.st) * 2);
+                    vr[i] = *reinterpret_cast<const uint4 *>(static_cast<const char *>(mb.v) + (base + j * mb.st) * 2);
+                }
             }
+            // eight elements of token tg + i * TPG
+            auto elems = [&](const uint4 &w, const void *p, int i, float (&x)[8]) {
+                if (!raw16)
+                    load8_f32(p, mb.dtype, mb.vec, base + min(j0 + tg + i * TPG, n - 1) * mb.st, x);
+                else if (mb.dtype == SS_F16)
+                    unpack16<__half>(w, x);
+                else
+                    unpack16<__hip_bfloat16>(w, x);
+            };
 #pragma unroll
             for (int i = 0; i < PASSES; ++i) {
-                float a = 0.f;
+                float a = 0.f, kx[8];
+                elems(kr[i], mb.k, i, kx);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) a = fmaf(qv[e], kx[i][e], a);
+                for (int e = 0; e < 8; ++e) a = fmaf(qv[e], kx[e], a);
 #pragma unroll
                 for (int o = LPT / 2; o > 0; o >>= 1) a += __shfl_xor(a, o);
                 const int tl = tg + i * TPG;
@@ -4504,8 +4520,10 @@ __global__ void __launch_bounds__(kDecodeThreads)
 #pragma unroll
             for (int i = 0; i < PASSES; ++i) {
                 const float p = prob(tg + i * TPG);
+                float vx[8];
+                elems(vr[i], mb.v, i, vx);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) ba[e] = fmaf(p, vx[i][e], ba[e]);
+                for (int e = 0; e < 8; ++e) ba[e] = fmaf(p, vx[e], ba[e]);
             }
             __syncthreads();  // bp is written again by the next chunk
         }
@@ -4518,15 +4536,48 @@ __global__ void __launch_bounds__(kDecodeThreads)
 #pragma unroll
             for (int e = 0; e < 8; ++e) bacc[wv][dl * 8 + e] = ba[e];
     }
+    // What does not depend on the weights is requested together, before them:
+    // the splits' (m, l) (wave 0), the first kAhead accumulator slices of each
+    // thread and its rows of the rotation.
+    constexpr int kAhead = 8;
     const float *ml = c.part_ml + ((int64_t)col * SS * R + r) * 2;
+    float2 mlv = make_float2(kLowest, 0.f);
+    if (wv == 0 && lane < S) mlv = *reinterpret_cast<const float2 *>(ml + (int64_t)lane * R * 2);
+    const int chunk = tid % CH, part = tid / CH;
+    const float4 *ap = reinterpret_cast<const float4 *>(c.part_acc + ((int64_t)col * SS * R + r) * D) + chunk;
+    float4 av[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+        const int s2 = part + i * NP;
+        av[i] = s2 < S ? ap[(int64_t)s2 * R * CH] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    // rotation: thread (part, chunk) takes dims 4 chunk .. of rows KP part ..
+    constexpr int KP = D / NP;
+    float4 rv[KP];
+    if (rot) {
+        const float *rp = rot + part * KP * D + 4 * chunk;
+        if (reinterpret_cast<uintptr_t>(rot) % 16 == 0) {
+#pragma unroll
+            for (int k = 0; k < KP; ++k) rv[k] = *reinterpret_cast<const float4 *>(rp + k * D);
+        } else {
+#pragma unroll
+            for (int k = 0; k < KP; ++k)
+                rv[k] = make_float4(rp[k * D], rp[k * D + 1], rp[k * D + 2], rp[k * D + 3]);
+        }
+    }
     float bw = 0.f;  // the buffer's weight (wave 0 sets it below)
     __shared__ float bwsh;
     if (wv == 0) {
-        float M = bm;
-        for (int s2 = lane; s2 < S; s2 += kWave) M = fmaxf(M, ml[(int64_t)s2 * R * 2]);
+        float M = fmaxf(bm, mlv.x);
+        for (int s2 = lane + kWave; s2 < S; s2 += kWave) M = fmaxf(M, ml[(int64_t)s2 * R * 2]);
         M = wave_max(M);
         float L = 0.f;
-        for (int s2 = lane; s2 < S; s2 += kWave) {
+        if (lane < S) {
+            const float w = fast_exp2(mlv.x - M);
+            wsh[lane] = w;
+            L = mlv.y * w;
+        }
+        for (int s2 = lane + kWave; s2 < S; s2 += kWave) {
             const float2 v = *reinterpret_cast<const float2 *>(ml + (int64_t)s2 * R * 2);
             const float w = fast_exp2(v.x - M);
             wsh[s2] = w;
@@ -4552,12 +4603,17 @@ __global__ void __launch_bounds__(kDecodeThreads)
         return a;
     };
     {
-        const int chunk = tid % CH, part = tid / CH;
-        const float4 *ap =
-            reinterpret_cast<const float4 *>(c.part_acc + ((int64_t)col * SS * R + r) * D) + chunk;
         float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            const float w = part + i * NP < S ? wsh[part + i * NP] : 0.f;
+            a.x = fmaf(av[i].x, w, a.x);
+            a.y = fmaf(av[i].y, w, a.y);
+            a.z = fmaf(av[i].z, w, a.z);
+            a.w = fmaf(av[i].w, w, a.w);
+        }
 #pragma unroll 8
-        for (int s2 = part; s2 < S; s2 += NP) {
+        for (int s2 = part + kAhead * NP; s2 < S; s2 += NP) {
             const float4 v = ap[(int64_t)s2 * R * CH];
             const float w = wsh[s2];
             a.x = fmaf(v.x, w, a.x);
@@ -4585,27 +4641,24 @@ __global__ void __launch_bounds__(kDecodeThreads)
     if (rot) {
         // the merged row is in a transformed basis (TurboQuant rotation, a
         // value codec's permutation or rotation): out = y @ M.  Every thread
-        // takes one output dim and a contiguous share of k (two interleaved
-        // accumulators), reading row k of M coalesced over the dims; the
-        // shares are added in LDS.
-        constexpr int PARTS = kDecodeThreads / D, KP = D / PARTS;
-        __shared__ float rsum[PARTS][D];
-        __syncthreads();
-        {
-            const int dd = tid % D, part = tid / D, k0 = part * KP;
-            float a0 = 0.f, a1 = 0.f;
-#pragma unroll 8
-            for (int k = k0; k < k0 + KP; k += 2) {
-                a0 = fmaf(yrow[k], rot[k * D + dd], a0);
-                a1 = fmaf(yrow[k + 1], rot[(k + 1) * D + dd], a1);
-            }
-            rsum[part][dd] = a0 + a1;
+        // takes four output dims and its share of k; the shares are added in
+        // LDS.
+        __syncthreads();  // yrow is written, red is free
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int k = 0; k < KP; ++k) {
+            const float y = yrow[part * KP + k];
+            a.x = fmaf(y, rv[k].x, a.x);
+            a.y = fmaf(y, rv[k].y, a.y);
+            a.z = fmaf(y, rv[k].z, a.z);
+            a.w = fmaf(y, rv[k].w, a.w);
         }
+        red[part * CH + chunk] = a;
         __syncthreads();
         if (tid < D) {
             float a = 0.f;
 #pragma unroll
-            for (int pp = 0; pp < PARTS; ++pp) a += rsum[pp][tid];
+            for (int pp = 0; pp < NP; ++pp) a += reinterpret_cast<const float *>(red)[pp * D + tid];
             store_from_f32(rot_out, rot_dtype, off + tid, a + buffered(tid));
         }
     }
