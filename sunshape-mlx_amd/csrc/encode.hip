@@ -647,13 +647,23 @@ __global__ void __launch_bounds__(kEmWaves * kWave)
                         Dv = __builtin_amdgcn_mfma_f32_32x32x16_f16(A3, B3, Dv, 0, 0, 0);
                         const int hk = t >> 2;
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            uint32_t p = (__float_as_uint(Dv[r]) & 0xffffff80u) | (uint32_t)((t & 3) * 16 + r);
-                            // centroid row of register r: 8*(r/4) + 4*h + r%4
-                            if (!FULL && t == nt - 1)
-                                p = (32 * t + 8 * (r >> 2) + 4 * h + (r & 3) < nc) ? p : 0xffffffffu;
-                            m2[hk] = umed3(m1[hk], m2[hk], p);
-                            m1[hk] = min(m1[hk], p);
+                        for (int r = 0; r < 16; r += 4) {
+                            uint32_t p[4];
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) {
+                                p[k] = (__float_as_uint(Dv[r + k]) & 0xffffff80u) | (uint32_t)((t & 3) * 16 + r + k);
+                                // centroid row of register r: 8*(r/4) + 4*h + r%4
+                                if (!FULL && t == nt - 1)
+                                    p[k] = (32 * t + 8 * (r >> 2) + 4 * h + k < nc) ? p[k] : 0xffffffffu;
+                            }
+                            // two at a time: m1 <= m2, so the second smallest of
+                            // (m1, m2, a, b) is min(m2, med3(m1, a, b)); five
+                            // operations for four values (eight one by one)
+                            const uint32_t da = umed3(m1[hk], p[0], p[1]);
+                            m1[hk] = min(m1[hk], min(p[0], p[1]));
+                            const uint32_t db = umed3(m1[hk], p[2], p[3]);
+                            m1[hk] = min(m1[hk], min(p[2], p[3]));
+                            m2[hk] = min(m2[hk], min(da, db));
                         }
                     }
                 }
