@@ -329,13 +329,15 @@ class SunShapeBlockCodec:
         return dims.to(torch.int32).to(self.device)
 
     def _any_heavy(self) -> bool:
-        """Whether :meth:`heavy_dims` is not None.  Reading the mask waits for
-        the GPU, so the answer is kept with the mask and read again when it
-        changes (another tensor or an in-place update)."""
+        """Whether :meth:`heavy_dims` is not None.  Reading a mask on the GPU
+        waits for it, so the answer is kept with the mask and read again when
+        it changes (another tensor or an in-place update).  A mask on the host
+        may share its memory with an array that changes unseen and costs
+        nothing to read: it is read each time."""
         if self.mode != "profileperm_mixed_precision" or not self.heavy_fp16:
             return False
         hb = self.mixed_high_precision_blocks
-        if hb.is_inference():  # no version to tell an in-place update by
+        if not hb.is_cuda or hb.is_inference():  # (no version there to tell an update by)
             return bool(hb.any())
         held = getattr(self, "_heavy_seen", None)
         if held is None or held[0] is not hb or held[1] != hb._version:
