@@ -241,6 +241,8 @@ static int turboquant_rows_decode(
     SS_UNSUPPORTED(mx >= 1e-30f && mx <= 1e30f, "level table out of the fp16 split's range");
     int e;
     frexpf(mx, &e);
+    static_assert(VTqRows<128, BITS>::reads_fit() && VTqRows<64, BITS>::reads_fit(),
+                  "row reads leave the packed rows");
     typename VTqRows<128, BITS>::Args va128{packed, norms, {}, ldexpf(1.f, e - 15)};
     typename VTqRows<64, BITS>::Args va64{packed, norms, {}, va128.linv};
     for (int i = 0; i < (1 << BITS); ++i) va128.lv[i] = va64.lv[i] = ldexpf(levels[i], 15 - e);

@@ -1977,10 +1977,9 @@ struct VTqRows {
         const uint32_t last = (uint32_t)min(t_last - t0, (int64_t)kWave - 1);
         const char *base = reinterpret_cast<const char *>(a.packed + (bh * cap + t0) * NW);
         // the four bytes from the one that holds the lane's first code: its NT
-        // codes and, at 3 bits, the two unused bits of a word they straddle
-        // (30 bits at most; the last lane's codes end its row)
-        const uint32_t bit = first_bit(l16);
-        base += bit / 8;
+        // codes and, at 3 bits, the two unused bits of a word they straddle;
+        // never past the row's end, which may be the buffer's
+        base += first_byte(l16);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
@@ -1992,7 +1991,7 @@ struct VTqRows {
     }
     __device__ static void from_raw(Tile &tv, const Raw &u, int lane) {
         const int l16 = lane & 15;
-        const uint32_t sh = first_bit(l16) % 8;
+        const uint32_t sh = first_bit(l16) - 8 * first_byte(l16);
         // 3 bits: the codes left in the first word, then (past its two unused
         // bits) those of the next
         const int n0 = min(VPW - NT * l16 % VPW, NT);
@@ -2007,8 +2006,22 @@ struct VTqRows {
         tv.n = u.n;
     }
     // bit of a row at which lane l16's codes start
-    __device__ static uint32_t first_bit(int l16) {
+    __host__ __device__ static constexpr uint32_t first_bit(int l16) {
         return (uint32_t)(NT * l16 / VPW * 32 + NT * l16 % VPW * BITS);
+    }
+    // byte of a row at which its four bytes start
+    __host__ __device__ static constexpr uint32_t first_byte(int l16) {
+        const uint32_t b = first_bit(l16) / 8, top = NW * 4 - 4;
+        return b < top ? b : top;
+    }
+    // every lane's codes lie in the four bytes it reads, and those in the row
+    static constexpr bool reads_fit() {
+        for (int l = 0; l < 16; ++l) {
+            const int c = NT * l + NT - 1;  // the lane's last code
+            const uint32_t end = c / VPW * 32 + c % VPW * BITS + BITS;
+            if (first_byte(l) + 4 > NW * 4u || end > 8 * first_byte(l) + 32) return false;
+        }
+        return true;
     }
     // the level pairs of code a | code b << BITS, at LDS address tab
     __device__ static void stage_table(uint32_t tab, const Args &a, int tid, int nt) {
