@@ -181,6 +181,18 @@ def _fused_hybrid_step(cache: HybridSunShapeKVCache, queries: torch.Tensor, scal
 _MASKED_ROWS = 64
 
 
+def _plain_mask(mask) -> bool:
+    """Whether ``mask`` is an array whose memory a kernel may read and through
+    which nothing is differentiated or batched: a learned bias, a dual number
+    and vmap's wrappers keep the two-pass path, whose torch operations carry
+    them."""
+    return (isinstance(mask, torch.Tensor)
+            and type(mask) in (torch.Tensor, torch.nn.Parameter)
+            and not (mask.requires_grad and torch.is_grad_enabled())
+            and torch.autograd.forward_ad._current_level < 0
+            and not torch._C._functorch.is_functorch_wrapped_tensor(mask))
+
+
 def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: int,
            out_dtype: torch.dtype, mask=None):
     """One fused launch over the whole cache, or None when no fused kernel
@@ -478,7 +490,7 @@ def sunshape_sdpa(queries: torch.Tensor, cache: SunShapeKVCache | HybridSunShape
     # and so does an array mask over few query rows
     can_fuse = (mask is None or use_causal) and compressed > 0
     array = None
-    if isinstance(mask, torch.Tensor) and compressed > 0 and hq // hkv * tq <= _MASKED_ROWS:
+    if compressed > 0 and hq // hkv * tq <= _MASKED_ROWS and _plain_mask(mask):
         array = _hip.attn_mask(mask.to(queries.device), (b_, hq, tq, t_kv))
     if can_fuse or array is not None:
         out = _fused(cache, queries, scale, use_causal, t_kv - tq if use_causal else 0,

@@ -168,6 +168,31 @@ def test_masked_decodes_equal_the_two_pass_path(backend, bits, dtype, d, hq, hkv
         assert float(err) <= REL_TOL, (name, float(err))
 
 
+def test_masks_that_carry_gradients_keep_the_two_pass_path():
+    """A learned bias gets its gradient, a dual bias its tangent and vmap its
+    batch: equal to the two-pass path's, and the same values as the fused
+    decode of the plain mask."""
+    cache = _masked_cache("fp16", 0, torch.float16, 128, 2, 1, 300, 128)
+    g = torch.Generator(device="cuda").manual_seed(4)
+    q = torch.randn((1, 8, 1, 128), generator=g, device="cuda").half()
+    bias, tangent = torch.randn((2, 8, 1, 300), generator=g, device="cuda")
+    plain = S.sunshape_sdpa(q, cache, 0.11, bias, out_dtype=torch.float32)
+    grads = []
+    for fn in (lambda m: S.sunshape_sdpa(q, cache, 0.11, m, out_dtype=torch.float32),
+               lambda m: attention._two_pass(cache, q, 0.11, m, torch.float32)):
+        m = bias.clone().requires_grad_()
+        out = fn(m)
+        assert rel_err(out.detach().cpu().numpy(), plain.cpu().numpy()) <= REL_TOL
+        out.square().sum().backward()
+        with torch.autograd.forward_ad.dual_level():
+            dual = torch.autograd.forward_ad.make_dual(bias, tangent)
+            jvp = torch.autograd.forward_ad.unpack_dual(fn(dual)).tangent.clone()
+        grads.append((m.grad, jvp, torch.vmap(fn)(torch.stack([bias, tangent]))))
+    for got, ref in zip(*grads):
+        assert torch.allclose(got, ref, rtol=1e-5, atol=1e-6 * float(ref.abs().max()))
+    assert torch.allclose(grads[0][2][0], plain, rtol=0, atol=REL_TOL * float(plain.abs().max()))
+
+
 @pytest.mark.parametrize("b,hq,hkv,d,t_q,past,causal,qdt,vdt,n_raw,nc,ws_heads", [
     (1, 4, 1, 128, 1, 0, True, torch.float16, torch.float16, 0, 256, 0),       # one key, one row
     (1, 8, 2, 128, 33, 0, True, torch.float16, torch.float16, 0, 256, 0),      # a sub-tile and a key
