@@ -66,8 +66,9 @@ def _prepared_decode(cache, ops: dict, codec: SunShapeBlockCodec, q: torch.Tenso
         tensors += (perm,)
     if buffered:  # the buffer stores (their windows move from call to call)
         tensors += (cache._key_buffer, cache._value_buffer)
+    # (a tensor may be given other memory in place, by set_ or .data)
     key = (kind, q.shape, q.dtype, q.device, kscale, ops.get("bits"), ops.get("group_size"),
-           buffered)
+           buffered, *[t.data_ptr() for t in tensors])
     held = getattr(cache, "_decode_prepared", None)
     if held is not None and held[0] == key and len(held[1]) == len(tensors) and \
             all(r() is t for r, t in zip(held[1], tensors)):

@@ -168,6 +168,20 @@ def test_masked_decodes_equal_the_two_pass_path(backend, bits, dtype, d, hq, hkv
         assert float(err) <= REL_TOL, (name, float(err))
 
 
+def test_kept_plan_follows_memory_given_in_place():
+    """A permutation given other memory through ``.data``: the next bf16
+    decode reads it there."""
+    cache = _masked_cache("fp16", 0, torch.bfloat16, 128, 2, 1, 300, 128)
+    q = torch.randn((1, 8, 1, 128), device="cuda").bfloat16()
+    first = S.sunshape_sdpa(q, cache, 0.11)
+    perm = cache.codec.permutation
+    old = perm.detach()  # the old memory stays allocated
+    perm.data = old.flip(0).clone()
+    got = S.sunshape_sdpa(q, cache, 0.11)
+    cache._decode_prepared = None
+    assert torch.equal(got, S.sunshape_sdpa(q, cache, 0.11)) and not torch.equal(got, first)
+
+
 def test_masks_that_carry_gradients_keep_the_two_pass_path():
     """A learned bias gets its gradient, a dual bias its tangent and vmap its
     batch: equal to the two-pass path's, and the same values as the fused
