@@ -1351,13 +1351,16 @@ def prefill_supported(n_q_heads: int, n_kv_heads: int, t_q: int, head_dim: int,
             and t_q >= rows // rep)
 
 
-def prompt_supported(q: torch.Tensor, n_kv_heads: int, n_blocks: int, t_kv: int) -> bool:
+def prompt_supported(q: torch.Tensor, n_kv_heads: int, n_blocks: int, t_kv: int,
+                     v_dtype: torch.dtype = torch.float16) -> bool:
     """Whether :func:`prefill_attn` takes queries ``q`` (B, Hq, T_q, D) against
     ``t_kv`` tokens and is the faster kernel for them.  It streams the keys
     once per 128 rows of a KV head, one tile of 64 tokens per 1.7 us (1.1 at
     head_dim 64) and chip-full of workgroups; the decodes stream them once
     per 4 rows.  Measured crossings (32/8 heads, past tokens: new tokens):
-    0: 128, 2048: 64-128, 32768: 64-128, 4 x 4096: 16-32."""
+    0: 128, 2048: 64-128, 32768: 64-128, 4 x 4096: 16-32.  Over bf16 values at
+    head_dim 64 the decode is the vector-ALU one, at less than half of that
+    per row and token (6000: 65 in 83 us, 1500: 101 in 47 against 76)."""
     b_, hq, tq, d = q.shape
     if q.dtype not in (torch.float16, torch.bfloat16) or d not in (64, 128) or n_blocks * 8 != d \
             or tq < 2:
@@ -1365,7 +1368,8 @@ def prompt_supported(q: torch.Tensor, n_kv_heads: int, n_blocks: int, t_kv: int)
     rows, heads = hq // n_kv_heads * tq, b_ * n_kv_heads
     fill = max(1.0, -(-rows // 128) * heads / 256)
     prompt_us = 25.0 + (1.7 if d == 128 else 1.1) * -(-t_kv // 64) * fill
-    return prompt_us < 15.0 + 9.2e-6 * rows * t_kv * heads
+    row_us = 4e-6 if d == 64 and v_dtype == torch.bfloat16 else 9.2e-6
+    return prompt_us < 15.0 + row_us * rows * t_kv * heads
 
 
 def decode_attn_il8_noalloc(q: torch.Tensor, scale: float, perm: torch.Tensor | None,

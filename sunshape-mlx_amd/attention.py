@@ -228,7 +228,8 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
     if mask is None and isinstance(cache, HybridSunShapeKVCache) and ops.get("k_heavy") is None and \
             (cache.dtype == torch.float16 or
              (cache.dtype == torch.bfloat16 and whole)) and \
-            _hip.prompt_supported(q, cache.n_kv_heads, codec.n_blocks, cache.offset) and \
+            _hip.prompt_supported(q, cache.n_kv_heads, codec.n_blocks, cache.offset,
+                                  cache.dtype) and \
             (whole or _hip.prefill_supported(hq, cache.n_kv_heads, tq, d, codec.n_blocks)):
         pf = cache.prefill_operands()
         if pf is not None:
@@ -271,7 +272,8 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
         out = None
         try:
             if (kind == "il8" or ops["values"].dtype == torch.bfloat16) and \
-                    _hip.prompt_supported(q, cache.n_kv_heads, codec.n_blocks, t_kv):
+                    _hip.prompt_supported(q, cache.n_kv_heads, codec.n_blocks, t_kv,
+                                          ops["values"].dtype):
                 v8 = ops["values"]
                 if kind == "dense":
                     v8 = torch.empty((b_, cache.n_kv_heads, (t_kv + 7) // 8, d, 8),
@@ -302,8 +304,12 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
         codec.last_score_backend = "hip_fused_mfma" if kind == "il8" else "hip_fused_mfma_dequant"
         return out
     # token-major bfloat16 values on the matrix cores, with or without
-    # buffered tokens
-    if kind == "dense" and ops["values"].dtype == torch.bfloat16:
+    # buffered tokens: one query position at head_dim 128 (4 x 8003 tokens 32
+    # against 38 us a step on the vector ALUs), and under a mask.  Elsewhere
+    # the vector-ALU decode below is ahead: 16 x 20000 tokens, four positions
+    # 565 against 431 us; 100000 tokens of 16 heads of 64 dims 79 against 50
+    if kind == "dense" and ops["values"].dtype == torch.bfloat16 and \
+            (mask is not None or (tq == 1 and d == 128)):
         try:
             if rounded:  # values of this call only: no plan to keep
                 plan = _hip.prepare_decode_dense(q, kscale, perm, codec.kernel_codebook(),
@@ -391,7 +397,8 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
             out = _hip.decode_attn_dense(q, kscale, perm, codec.centroids, ops["idx"],
                                          ops["values"], buf_keys=ops.get("buf_keys"),
                                          buf_values=ops.get("buf_values"), buf_len=buffered, **kw)
-            codec.last_score_backend = "hip_fused_buffer" if buffered else "hip_fused"
+            codec.last_score_backend = ("hip" if rounded else
+                                        "hip_fused_buffer" if buffered else "hip_fused")
     except _hip.SunShapeUnsupported:
         return None
     return out
