@@ -171,12 +171,12 @@ template <int NH8>
 int launch_sunv_masked(const DecodeCommon &c, const typename VSunV<128, 4>::Args &va,
                        const DecodeShape &s, hipStream_t st);
 
-template <int D, int R, class VF>
-static int launch(DecodeCommon c, const typename VF::Args &va, const DecodeShape &s,
+template <int D, int R, class VF, bool MK>
+static int launch_mk(DecodeCommon c, const typename VF::Args &va, const DecodeShape &s,
                   hipStream_t st, bool merge = true) {
     constexpr int TH = VfThreads<VF>::value;
     const size_t lds = decode_lds_bytes<D, R, TH / kWave>() + VfLds<VF>::value;
-    auto kern = decode_attn_kernel<D, R, VF>;
+    auto kern = decode_attn_kernel<D, R, VF, MK>;
     static bool attr_set = false;  // per instantiation
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
@@ -188,6 +188,13 @@ static int launch(DecodeCommon c, const typename VF::Args &va, const DecodeShape
     hipLaunchKernelGGL(kern, grid, dim3(TH), lds, st, c, va);
     SS_LAUNCH_CHECK("decode_attn_kernel launch");
     return merge ? launch_merge<D>(c, s, st) : SS_OK;
+}
+
+template <int D, int R, class VF>
+static int launch(DecodeCommon c, const typename VF::Args &va, const DecodeShape &s, hipStream_t st,
+                  bool merge = true) {
+    return c.mask_dt != kMaskNone ? launch_mk<D, R, VF, true>(c, va, s, st, merge)
+                                  : launch_mk<D, R, VF, false>(c, va, s, st, merge);
 }
 
 template <int D, class VF>

@@ -572,9 +572,12 @@ constexpr size_t decode_lds_bytes() {
 // 2^kValuLag).
 constexpr float kValuLag = 8.f;
 
-template <int D, int R, class VF>
+// MK: with a mask (an instantiation of its own: tested at run time inside the
+// loop, it cost every call, 101 bf16 tokens of 64-dim heads after 1500 52-55
+// us instead of 44-47).
+template <int D, int R, class VF, bool MK>
 __global__ void __launch_bounds__(VfThreads<VF>::value)
-    decode_attn_kernel(DecodeCommon c, typename VF::Args va) {
+    decode_attn_kernel(std::conditional_t<MK, DecodeCommon, DecodeCore> c, typename VF::Args va) {
     constexpr int TH = VfThreads<VF>::value, WV = TH / kWave;
     constexpr int NB = D / kBlockDim;
     constexpr int DPL = VF::DPL, LPT = VF::LPT, TPI = VF::TPI, ITERS = VF::ITERS;
@@ -688,7 +691,7 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int64_t gr = row_ok(r) ? (int64_t)rg * R + r : (int64_t)rg * R;
-        mrow[r] = bb * c.m_sb + (kvh * c.rep + gr / c.t_q) * c.m_sh + (gr % c.t_q) * c.m_sq;
+        if constexpr (MK) mrow[r] = bb * c.m_sb + (kvh * c.rep + gr / c.t_q) * c.m_sh + (gr % c.t_q) * c.m_sq;
     }
 
     float m[R], l[R], acc[R][DPL];
@@ -714,7 +717,7 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
         IdxRow<NB> ir;
         ir.load(idx_head + tk * NB, kok);
         uint32_t mk[R];
-        if (c.mask_dt != kMaskNone)
+        if constexpr (MK)
 #pragma unroll
             for (int r = 0; r < R; ++r) mk[r] = kok ? mask_load(c, mrow[r] + tk) : 0u;
 
@@ -748,7 +751,7 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
             }
         }
         float slo[R] = {};
-        if (c.mask_dt != kMaskNone)
+        if constexpr (MK)
 #pragma unroll
             for (int r = 0; r < R; ++r) s[r] = mask_score(c, mk[r], s[r], slo[r]);
 #pragma unroll
