@@ -1126,11 +1126,14 @@ def decode_plan(kind, batch, n_q_heads, n_kv_heads, t_q, head_dim, t_kv, n_split
 
 def codebook_f16x2(centroids: torch.Tensor) -> torch.Tensor:
     """Split-fp16 codebook (flat uint8 buffer) read by :func:`decode_attn_il8`
-    for float32 centroids (n_blocks, n_centroids, 8)."""
+    for float32 centroids (n_blocks, n_centroids, 8).  Other block dims are
+    refused before the launch, which reads 8 floats of every centroid."""
     require_gpu(centroids)
     if centroids.dim() != 3 or centroids.dtype != torch.float32 or not centroids.is_contiguous():
         raise ValueError("centroids must be contiguous float32 (n_blocks, n_centroids, 8)")
-    nb, nc, _ = centroids.shape
+    nb, nc, bd = centroids.shape
+    if bd != 8:
+        raise SunShapeUnsupported(-2, f"prepared codebooks hold blocks of 8 dims (got {bd})")
     lib = load_library()
     out = torch.empty(lib.ss_codebook_f16x2_bytes(nb, nc), dtype=torch.uint8,
                       device=centroids.device)

@@ -403,3 +403,31 @@ def test_turboquant_rows_on_the_matrix_cores(bits, d, hq, t_kv, t_buf, t_q, spli
     err, ref = (rel_err(o.cpu().numpy(), want) for o in outs)
     print("error", err, "vector-ALU kernel", ref)
     assert err <= REL_TOL and err <= ref + 1e-6
+
+
+def _other_codec_cache(d, block_dim, backend, dtype):
+    """A cache whose key codec no fused decode takes."""
+    rng = np.random.default_rng(d + block_dim)
+    codec = S.SunShapeBlockCodec(d, block_dim=block_dim, device="cuda")
+    codec.load_state_dict({"centroids": rng.standard_normal((d // block_dim, 256, block_dim))
+                           .astype(np.float32),
+                           "permutation": rng.permutation(d).astype(np.int32)})
+    cache = S.create_kv_cache(codec, n_kv_heads=2, dtype=dtype, value_backend=backend,
+                              value_bits=4 if backend != "fp16" else None, buffer_size=20)
+    g = torch.Generator(device="cuda").manual_seed(d)
+    k, v = torch.randn((2, 1, 2, 150, d), generator=g, device="cuda").to(dtype)
+    cache.update_and_fetch(k, v)
+    return cache, torch.randn((1, 8, 1, d), generator=g, device="cuda").to(dtype)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("d,block_dim,backend,dtype", [
+    (128, 4, "turboquant", torch.float16), (128, 4, "fp16", torch.bfloat16),
+    (128, 4, "grouped", torch.bfloat16), (128, 16, "turboquant", torch.bfloat16),
+    (64, 4, "fp16", torch.bfloat16),
+])
+def test_other_block_dims_take_the_two_pass_path(d, block_dim, backend, dtype, masked):
+    cache, q = _other_codec_cache(d, block_dim, backend, dtype)
+    mask = torch.arange(150, device="cuda") > 7 if masked else None
+    got = S.sunshape_sdpa(q, cache, 0.1, mask)
+    assert torch.equal(got, attention._two_pass(cache, q, 0.1, mask, dtype))
