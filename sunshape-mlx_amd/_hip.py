@@ -1134,6 +1134,8 @@ def codebook_f16x2(centroids: torch.Tensor) -> torch.Tensor:
     nb, nc, bd = centroids.shape
     if bd != 8:
         raise SunShapeUnsupported(-2, f"prepared codebooks hold blocks of 8 dims (got {bd})")
+    if nb % 4 or not 4 <= nb <= 64 or not 1 <= nc <= 256:  # as ss_codebook_f16x2 takes them
+        raise SunShapeUnsupported(-2, f"no prepared codebook of {nb} blocks and {nc} centroids")
     lib = load_library()
     out = torch.empty(lib.ss_codebook_f16x2_bytes(nb, nc), dtype=torch.uint8,
                       device=centroids.device)

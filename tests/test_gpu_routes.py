@@ -425,8 +425,10 @@ def _other_codec_cache(d, block_dim, backend, dtype):
     (128, 4, "turboquant", torch.float16), (128, 4, "fp16", torch.bfloat16),
     (128, 4, "grouped", torch.bfloat16), (128, 16, "turboquant", torch.bfloat16),
     (64, 4, "fp16", torch.bfloat16),
+    (80, 8, "turboquant", torch.float16), (112, 8, "fp16", torch.bfloat16),
+    (72, 8, "turboquant", torch.bfloat16),
 ])
-def test_other_block_dims_take_the_two_pass_path(d, block_dim, backend, dtype, masked):
+def test_other_codecs_take_the_two_pass_path(d, block_dim, backend, dtype, masked):
     cache, q = _other_codec_cache(d, block_dim, backend, dtype)
     mask = torch.arange(150, device="cuda") > 7 if masked else None
     got = S.sunshape_sdpa(q, cache, 0.1, mask)

@@ -29,3 +29,12 @@ def test_codebooks_of_other_block_dims_are_refused_before_a_launch(no_launch, sh
     tensor for smaller blocks."""
     with pytest.raises(_hip.SunShapeUnsupported):
         _hip.codebook_f16x2(torch.zeros(shape))
+
+
+@pytest.mark.parametrize("shape", [(10, 256, 8), (14, 256, 8), (9, 256, 8), (68, 256, 8),
+                                   (16, 257, 8), (2, 256, 8)])
+def test_codebooks_of_other_sizes_are_unsupported(no_launch, shape):
+    """A block count that is not a multiple of 4 (head dims 80, 112, 72) or
+    too many centroids: the error after which a call takes its other route."""
+    with pytest.raises(_hip.SunShapeUnsupported):
+        _hip.codebook_f16x2(torch.zeros(shape))
