@@ -99,26 +99,30 @@ __device__ __forceinline__ uint32_t mask_load(const DecodeCommon &c, int64_t off
     return static_cast<const uint16_t *>(c.mask)[off];
 }
 
-// A score in log2 units under mask element w (mask_load's bits), as hi + lo:
-// hidden or kept by a boolean, else the element added in natural units, where
-// the sum rounds as the reference's does (a mask of -1e9 absorbs the score in
-// float32, one of -65504 keeps its part above 2^-8).  hi is the sum in log2
-// units and lo what its rounding there left off, added back after the
-// running maximum is subtracted: a row hidden throughout by -65504 keeps the
-// reference's differences.  A finite sum stays finite, so float32's lowest
-// value hides as a boolean does; -inf and NaN keep their effect.
-__device__ __forceinline__ float mask_score(const DecodeCommon &c, uint32_t w, float s, float &lo) {
-    lo = 0.f;
+// A score in log2 units under mask element w (mask_load's bits): hidden or
+// kept by a boolean; under an additive mask in natural units, the element
+// added as the reference does (a mask of -1e9 absorbs the score in float32,
+// one of -65504 keeps its part above 2^-8, float32's lowest value hides as a
+// boolean does; -inf and NaN keep their effect).
+__device__ __forceinline__ float mask_score(const DecodeCommon &c, uint32_t w, float s) {
     if (c.mask_dt == kMaskBool) return w ? s : kLowest;
     const float x = c.mask_dt == kMaskF32   ? __uint_as_float(w)
                     : c.mask_dt == kMaskF16 ? __half2float(__ushort_as_half((unsigned short)w))
                                             : __uint_as_float(w << 16);
-    const float y = fmaf(s, 0.6931471805599453f, x);
-    const float hi = y * kLog2e;
-    if (fabsf(hi) == INFINITY) return fabsf(y) == INFINITY ? y : (y < 0.f ? kLowest : -kLowest);
-    lo = fmaf(y, kLog2e, -hi);
-    return hi;
+    return fmaf(s, 0.6931471805599453f, x);
 }
+
+// The factor that takes a difference of two of a call's scores (or running
+// maxima, as the split partials hold them) to log2 units.  Scores under an
+// additive mask stay in natural units until the maximum is subtracted: that
+// difference is exact near the maximum however large the mask, and never
+// above zero past it, so a probability is bounded by the maximum it is
+// relative to (a score rounded to log2 units first was off by up to 2^-25 of
+// the mask there, 18 units at -1e9).
+__device__ __forceinline__ float mask_unit(const DecodeCommon &c) {
+    return c.mask_dt == kMaskNone || c.mask_dt == kMaskBool ? 1.f : kLog2e;
+}
+__device__ __forceinline__ float mask_unit(const DecodeCore &) { return 1.f; }
 
 // What a row with no probability mass returns: zeros (an empty cache, a
 // causal row that sees no key), but under a mask NaN, as a softmax over
@@ -694,6 +698,7 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
         if constexpr (MK) mrow[r] = bb * c.m_sb + (kvh * c.rep + gr / c.t_q) * c.m_sh + (gr % c.t_q) * c.m_sq;
     }
 
+    const float mu = mask_unit(c);
     float m[R], l[R], acc[R][DPL];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -750,10 +755,9 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
                 for (int r = 0; r < R; ++r) s[r] += hs[r];
             }
         }
-        float slo[R] = {};
         if constexpr (MK)
 #pragma unroll
-            for (int r = 0; r < R; ++r) s[r] = mask_score(c, mk[r], s[r], slo[r]);
+            for (int r = 0; r < R; ++r) s[r] = mask_score(c, mk[r], s[r]);
 #pragma unroll
         for (int r = 0; r < R; ++r) s[r] = (kok && tk <= lim[r]) ? s[r] : -INFINITY;
         // a tile whose scores stay at most kValuLag log2 units above the
@@ -761,7 +765,8 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
         // no wave-wide reduction and no rescale of the accumulators
         uint64_t above = 0;
 #pragma unroll
-        for (int r = 0; r < R; ++r) above |= __builtin_amdgcn_ballot_w64(s[r] > m[r] + kValuLag);
+        for (int r = 0; r < R; ++r)
+            above |= __builtin_amdgcn_ballot_w64(MK ? (s[r] - m[r]) * mu > kValuLag : s[r] > m[r] + kValuLag);
         const bool moved = above != 0;
         float corr[R];
         if (moved) {
@@ -775,8 +780,8 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 const float mn = fmaxf(m[r], tmax[r]);
-                corr[r] = fast_exp2(m[r] - mn);
-                const float p = fast_exp2((s[r] - mn) + slo[r]);
+                corr[r] = fast_exp2((m[r] - mn) * mu);
+                const float p = fast_exp2((s[r] - mn) * mu);
                 l[r] = fmaf(l[r], corr[r], p);
                 m[r] = mn;
                 s[r] = p;
@@ -785,7 +790,7 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 corr[r] = 1.f;
-                s[r] = fast_exp2((s[r] - m[r]) + slo[r]);
+                s[r] = fast_exp2((s[r] - m[r]) * mu);
                 l[r] += s[r];
             }
         }
@@ -888,7 +893,7 @@ __global__ void __launch_bounds__(VfThreads<VF>::value)
         float L = 0.f, A = 0.f;
 #pragma unroll
         for (int w = 0; w < WV; ++w) {
-            const float f = fast_exp2(wm[w * R + r] - M);
+            const float f = fast_exp2((wm[w * R + r] - M) * mu);
             L = fmaf(wl[w * R + r], f, L);
             A = fmaf(wa[(w * R + r) * DS + d], f, A);
         }
@@ -2415,6 +2420,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
     constexpr bool HV = VfHeavyMfma<VF>::value;
     constexpr bool MK = VfMasked<VF>::value;  // an attention mask applies
     constexpr int MKN = MK ? R : 1;
+    const float mu = mask_unit(c);
     int64_t mrow[MKN];  // the rows' mask offsets (a row past the last takes row 0's)
     if constexpr (MK)
 #pragma unroll
@@ -2627,7 +2633,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                                 vc[j][k] = hv_raw[j][k];
                             }
                         }
-                    float sc[NSH][R], blo[NSH][MKN] = {};
+                    float sc[NSH][R];
 #pragma unroll
                     for (int j = 0; j < NSH; ++j) {
                         float part[R];
@@ -2645,7 +2651,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                             if constexpr (MK)
                                 sc[j][r] =
                                     mask_score(c, mask_load(c, mrow[r] + min(pos, c.t_kv + t_buf - 1)),
-                                               sc[j][r], blo[j][r]);
+                                               sc[j][r]);
                             sc[j][r] = (c0 + j < n_sh && pos <= lim[r]) ? sc[j][r] : -INFINITY;
                         }
                     }
@@ -2656,14 +2662,14 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                         for (int j = 1; j < NSH; ++j) mx = fmaxf(mx, sc[j][r]);
                         if (mx == -INFINITY) continue;  // nothing visible in this chunk
                         const float mn = fmaxf(bm[r], mx);
-                        const float corr = fast_exp2(bm[r] - mn);
+                        const float corr = fast_exp2((bm[r] - mn) * mu);
                         bm[r] = mn;
                         bl[r] *= corr;
 #pragma unroll
                         for (int k = 0; k < DLh; ++k) ba[r][k] *= corr;
 #pragma unroll
                         for (int j = 0; j < NSH; ++j) {
-                            const float pj = fast_exp2(MK ? (sc[j][r] - mn) + blo[j][r % MKN] : sc[j][r] - mn);
+                            const float pj = fast_exp2((sc[j][r] - mn) * mu);
                             bl[r] += pj;
 #pragma unroll
                             for (int k = 0; k < DLh; ++k) ba[r][k] = fmaf(pj, f32(vc[j][k]), ba[r][k]);
@@ -2706,12 +2712,10 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                 for (int r = 0; r < R; ++r) sc[r] *= kLog2e;
             }
             const int64_t pos = (kStepOnly ? c.t_kv : ex_pos0) + j;
-            float blo[MKN] = {};
             if constexpr (MK)
 #pragma unroll
                 for (int r = 0; r < R; ++r)
-                    sc[r] = mask_score(c, mask_load(c, mrow[r] + min(pos, c.t_kv + t_buf - 1)), sc[r],
-                                       blo[r]);
+                    sc[r] = mask_score(c, mask_load(c, mrow[r] + min(pos, c.t_kv + t_buf - 1)), sc[r]);
 #pragma unroll
             for (int r = 0; r < R; ++r) sc[r] = (ok && pos <= lim[r]) ? sc[r] : -INFINITY;
             float tmax[R], p[R], corr[R];
@@ -2719,8 +2723,8 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 const float mn = fmaxf(bm[r], tmax[r]);
-                corr[r] = fast_exp2(bm[r] - mn);
-                p[r] = fast_exp2(MK ? (sc[r] - mn) + blo[r % MKN] : sc[r] - mn);
+                corr[r] = fast_exp2((bm[r] - mn) * mu);
+                p[r] = fast_exp2((sc[r] - mn) * mu);
                 bm[r] = mn;
             }
             float ps[R];
@@ -3522,10 +3526,9 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                     for (int r = 0; r < R; ++r) sc[r] += hv[r];
                 }
             }
-            float mlo[MKN] = {};
             if constexpr (MK)
 #pragma unroll
-                for (int r = 0; r < R; ++r) sc[r] = mask_score(c, mk.w[r], sc[r], mlo[r]);
+                for (int r = 0; r < R; ++r) sc[r] = mask_score(c, mk.w[r], sc[r]);
             // A whole tile every row sees (no causal cut, no split end) whose
             // scores all stay at most kLag above the rows' running maxima
             // keeps the maxima: no reduction, no rescale (its probabilities
@@ -3537,7 +3540,8 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
             if (n_in == kWave && t0 + (kWave - 1) <= lim_min) {
                 uint64_t above = 0;
 #pragma unroll
-                for (int r = 0; r < R; ++r) above |= __builtin_amdgcn_ballot_w64(sc[r] > m[r] + kLag);
+                for (int r = 0; r < R; ++r)
+                    above |= __builtin_amdgcn_ballot_w64(MK ? (sc[r] - m[r]) * mu > kLag : sc[r] > m[r] + kLag);
                 moved = above != 0;
             } else {
                 const bool kok = lane < n_in;
@@ -3555,8 +3559,8 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     const float mn = fmaxf(m[r], tmax[r]);
-                    corr[r] = fast_exp2(m[r] - mn);
-                    p[r] = fast_exp2(MK ? (sc[r] - mn) + mlo[r % MKN] : sc[r] - mn);
+                    corr[r] = fast_exp2((m[r] - mn) * mu);
+                    p[r] = fast_exp2((sc[r] - mn) * mu);
                     lsum[r] = fmaf(lsum[r], corr[r], p[r]);
                     m[r] = mn;
                 }
@@ -3564,7 +3568,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     corr[r] = 1.f;
-                    p[r] = fast_exp2(MK ? (sc[r] - m[r]) + mlo[r % MKN] : sc[r] - m[r]);
+                    p[r] = fast_exp2((sc[r] - m[r]) * mu);
                     lsum[r] += p[r];
                 }
             }
@@ -3711,12 +3715,12 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
         A = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < NC; ++w) {
-            const float f = fast_exp2(mw[w] - M);
+            const float f = fast_exp2((mw[w] - M) * mu);
             L = fmaf(lw[w], f, L);
             A += (hi[w] + lo[w]) * f;
         }
         if (has_buf) {
-            const float f = fast_exp2(mb - M);
+            const float f = fast_exp2((mb - M) * mu);
             L = fmaf(lb, f, L);
             A += ab * f;
         }
@@ -3826,7 +3830,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                 Mr = part + kMergeParts * j < S ? fmaxf(Mr, __uint_as_float(mv[j][0])) : Mr;
 #pragma unroll
             for (int j = 0; j < kMergeLoads; ++j) {
-                const float w = part + kMergeParts * j < S ? fast_exp2(__uint_as_float(mv[j][0]) - Mr) : 0.f;
+                const float w = part + kMergeParts * j < S ? fast_exp2((__uint_as_float(mv[j][0]) - Mr) * mu) : 0.f;
                 Lr = fmaf(__uint_as_float(mv[j][1]), w, Lr);
                 Ar += av[j] * w;
             }
@@ -3850,7 +3854,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                 const f32x4 a2 = f32x4{q6[2 * CH + cidx], q6[3 * CH + cidx], q6[4 * CH + cidx],
                                        q6[5 * CH + cidx]};
                 const float Mn = fmaxf(Mr, m2);
-                const float fo = fast_exp2(Mr - Mn), fn = fast_exp2(m2 - Mn);
+                const float fo = fast_exp2((Mr - Mn) * mu), fn = fast_exp2((m2 - Mn) * mu);
                 Ar = Ar * fo + a2 * fn;
                 Lr = Lr * fo + l2 * fn;
                 Mr = Mn;
@@ -3914,7 +3918,7 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
         float L = 0.f;
         for (int s2 = lane; s2 < S; s2 += kWave) {
             const u32x2 v = mlb[s2 * R + r];
-            const float w = fast_exp2(__uint_as_float(v[0]) - M);
+            const float w = fast_exp2((__uint_as_float(v[0]) - M) * mu);
             wts[s2 * R + r] = w;
             L = fmaf(__uint_as_float(v[1]), w, L);
         }
@@ -4189,6 +4193,7 @@ __global__ void __launch_bounds__(kSvWaves * kWave)
     const char *kh_b = reinterpret_cast<const char *>(va.kheavy + (NH8 > 0 ? vrow0 * (NH8 * 8) : 0));
     const char *vi_b = reinterpret_cast<const char *>(va.idx + vrow0 * kSvNBV);
     const uint32_t t_last32 = (uint32_t)t_last;
+    const float mu = MK ? mask_unit(c) : 1.f;
     int64_t mrow[MK ? R : 1];  // the rows' mask offsets (a row past the last takes row 0's)
     if constexpr (MK)
 #pragma unroll
@@ -4266,15 +4271,15 @@ __global__ void __launch_bounds__(kSvWaves * kWave)
             s4 += (hs + hl * (1.f / kSplitScale)) * (qsc * kLog2e);
         }
         float sc[R] = {s4.x, s4.y, s4.z, s4.w};
-        float mlo[R] = {};
         if constexpr (MK)
 #pragma unroll
-            for (int r = 0; r < R; ++r) sc[r] = mask_score(c, cur.mk[r], sc[r], mlo[r]);
+            for (int r = 0; r < R; ++r) sc[r] = mask_score(c, cur.mk[r], sc[r]);
         bool moved = true;
         if (n_in == kWave && t0 + (kWave - 1) <= lim_min) {
             uint64_t above = 0;
 #pragma unroll
-            for (int r = 0; r < R; ++r) above |= __builtin_amdgcn_ballot_w64(sc[r] > m[r] + kPLag);
+            for (int r = 0; r < R; ++r)
+                above |= __builtin_amdgcn_ballot_w64(MK ? (sc[r] - m[r]) * mu > kPLag : sc[r] > m[r] + kPLag);
             moved = above != 0;
         } else {
             const bool kok = lane < n_in;
@@ -4291,8 +4296,8 @@ __global__ void __launch_bounds__(kSvWaves * kWave)
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 const float mn = fmaxf(m[r], tmax[r]);
-                corr[r] = fast_exp2(m[r] - mn);
-                p[r] = fast_exp2(MK ? (sc[r] - mn) + mlo[r] : sc[r] - mn);
+                corr[r] = fast_exp2((m[r] - mn) * mu);
+                p[r] = fast_exp2((sc[r] - mn) * mu);
                 lsum[r] = fmaf(lsum[r], corr[r], p[r]);
                 m[r] = mn;
             }
@@ -4300,7 +4305,7 @@ __global__ void __launch_bounds__(kSvWaves * kWave)
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 corr[r] = 1.f;
-                p[r] = fast_exp2(MK ? (sc[r] - m[r]) + mlo[r] : sc[r] - m[r]);
+                p[r] = fast_exp2((sc[r] - m[r]) * mu);
                 lsum[r] += p[r];
             }
         }
@@ -4406,7 +4411,7 @@ __global__ void __launch_bounds__(kSvWaves * kWave)
         float L = 0.f, A = 0.f;
 #pragma unroll
         for (int w = 0; w < NC; ++w) {
-            const float f = fast_exp2(wm[w * R + r] - M);
+            const float f = fast_exp2((wm[w * R + r] - M) * mu);
             L = fmaf(wl[w * R + r], f, L);
             A = fmaf(wa[((w * 2) * R + r) * D + d] + wa[((w * 2 + 1) * R + r) * D + d], f, A);
         }
@@ -4479,8 +4484,9 @@ __global__ void __launch_bounds__(kDecodeThreads)
     constexpr int LPT = D / 8;                    // lanes per token
     constexpr int TPG = kDecodeThreads / LPT;     // tokens per pass of the workgroup
     constexpr int BT = 128, PASSES = BT / TPG;    // tokens of a chunk
-    __shared__ float bp[BUF ? BT : 1], bplo[BUF ? BT : 1];  // scores, and what a mask left off
+    __shared__ float bp[BUF ? BT : 1];
     __shared__ float bacc[BUF ? kDecodeThreads / kWave : 1][BUF ? D : 1];
+    const float mu = mask_unit(c);
     float bm = kLowest, bl = 0.f;
     if constexpr (BUF) {
         const int dl = tid % LPT, tg = tid / LPT;  // dims 8*dl .. +7 of tokens tg + i*TPG
@@ -4526,18 +4532,16 @@ __global__ void __launch_bounds__(kDecodeThreads)
                 for (int o = LPT / 2; o > 0; o >>= 1) a += __shfl_xor(a, o);
                 const int tl = tg + i * TPG;
                 if (dl == 0) {
-                    float lo = 0.f;
                     if (c.mask_dt != kMaskNone && j0 + tl < n)
-                        a = mask_score(c, mask_load(c, mrow + c.t_kv + j0 + tl), a, lo);
+                        a = mask_score(c, mask_load(c, mrow + c.t_kv + j0 + tl), a);
                     bp[tl] = j0 + tl < n ? a : -INFINITY;
-                    bplo[tl] = lo;
                 }
             }
             __syncthreads();
             float mx = wave_max(fmaxf(bp[lane], bp[lane + kWave]));
-            const float mn = fmaxf(bm, mx), corr = fast_exp2(bm - mn);
+            const float mn = fmaxf(bm, mx), corr = fast_exp2((bm - mn) * mu);
             bm = mn;
-            auto prob = [&](int i) { return fast_exp2((bp[i] - mn) + bplo[i]); };
+            auto prob = [&](int i) { return fast_exp2((bp[i] - mn) * mu); };
             bl = fmaf(bl, corr, wave_sum(prob(lane) + prob(lane + kWave)));
 #pragma unroll
             for (int e = 0; e < 8; ++e) ba[e] *= corr;
@@ -4597,19 +4601,19 @@ __global__ void __launch_bounds__(kDecodeThreads)
         M = wave_max(M);
         float L = 0.f;
         if (lane < S) {
-            const float w = fast_exp2(mlv.x - M);
+            const float w = fast_exp2((mlv.x - M) * mu);
             wsh[lane] = w;
             L = mlv.y * w;
         }
         for (int s2 = lane + kWave; s2 < S; s2 += kWave) {
             const float2 v = *reinterpret_cast<const float2 *>(ml + (int64_t)s2 * R * 2);
-            const float w = fast_exp2(v.x - M);
+            const float w = fast_exp2((v.x - M) * mu);
             wsh[s2] = w;
             L = fmaf(v.y, w, L);
         }
         L = wave_sum(L);
         if constexpr (BUF) {
-            bw = fast_exp2(bm - M);
+            bw = fast_exp2((bm - M) * mu);
             L = fmaf(bl, bw, L);
             if (lane == 0) bwsh = bw;
         }

@@ -433,3 +433,39 @@ def test_other_codecs_take_the_two_pass_path(d, block_dim, backend, dtype, maske
     mask = torch.arange(150, device="cuda") > 7 if masked else None
     got = S.sunshape_sdpa(q, cache, 0.1, mask)
     assert torch.equal(got, attention._two_pass(cache, q, 0.1, mask, dtype))
+
+
+@pytest.mark.parametrize("backend,bits,dtype,d,hq,t_kv,t_q,buffer", [
+    ("fp16", 0, torch.float16, 128, 8, 1300, 1, 128),
+    ("fp16", 0, torch.float16, 64, 8, 400, 2, 16),
+    ("fp16", 0, torch.bfloat16, 128, 8, 700, 1, 40),
+    ("grouped", 2, torch.float16, 128, 8, 900, 1, 128),
+    ("grouped", 4, torch.float16, 128, 8, 900, 1, 20),
+    ("grouped", 3, torch.float16, 128, 8, 900, 1, 140),
+    ("turboquant", 2, torch.float16, 128, 8, 900, 1, 140),
+    ("turboquant", 4, torch.float16, 128, 8, 900, 1, 30),
+    ("turboquant", 4, torch.float16, 64, 2, 900, 1, 30),
+    ("sunshape", 8, torch.float16, 128, 8, 2500, 1, 140),
+    ("sunshape", 8, torch.float16, 64, 8, 900, 2, 10),
+])
+def test_masks_of_any_magnitude_equal_the_two_pass_path(backend, bits, dtype, d, hq, t_kv, t_q, buffer):
+    """Additive masks that hide by a large finite value: sequence 0 is padded
+    on the left by more than a unit of 64 keys (a hidden unit is attended
+    before a visible one), sequence 1 is hidden throughout."""
+    cache = _masked_cache(backend, bits, dtype, d, 2, 2, t_kv, buffer)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q = torch.randn((2, hq, t_q, d), generator=g, device="cuda").to(dtype)
+    keep = torch.rand((2, 1, t_q, t_kv), generator=g, device="cuda") > 0.1
+    keep[0, ..., :t_kv // 2 + 5] = False
+    keep[0, ..., -3:] = True
+    keep[1] = False
+    for low in (-1e4, -1e9, -1e10, -1e12, -1e30, -3e38):
+        for mdt in (torch.float32, torch.bfloat16):
+            if mdt == torch.bfloat16 and low not in (-1e9, -1e30):
+                continue
+            mask = torch.where(keep, 0.25, low).to(mdt)
+            ref = attention._two_pass(cache, q, 0.11, mask, torch.float32)
+            got = S.sunshape_sdpa(q, cache, 0.11, mask, out_dtype=torch.float32)
+            assert torch.isfinite(ref).all() and torch.isfinite(got).all(), (low, mdt)
+            err = (got - ref).abs().amax((1, 2, 3)) / ref.abs().amax((1, 2, 3))
+            assert float(err.max()) <= REL_TOL, (low, mdt, err)
