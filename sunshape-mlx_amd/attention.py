@@ -182,16 +182,23 @@ def _fused_hybrid_step(cache: HybridSunShapeKVCache, queries: torch.Tensor, scal
 _MASKED_ROWS = 64
 
 
-def _plain_mask(mask) -> bool:
-    """Whether ``mask`` is an array whose memory a kernel may read and through
+def _plain(t) -> bool:
+    """Whether ``t`` is an array whose memory a kernel may read and through
     which nothing is differentiated or batched: a learned bias, a dual number
     and vmap's wrappers keep the two-pass path, whose torch operations carry
     them."""
-    return (isinstance(mask, torch.Tensor)
-            and type(mask) in (torch.Tensor, torch.nn.Parameter)
-            and not (mask.requires_grad and torch.is_grad_enabled())
+    return (isinstance(t, torch.Tensor)
+            and type(t) in (torch.Tensor, torch.nn.Parameter)
+            and not (t.requires_grad and torch.is_grad_enabled())
             and torch.autograd.forward_ad._current_level < 0
-            and not torch._C._functorch.is_functorch_wrapped_tensor(mask))
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t))
+
+
+def _kernels_take(queries: torch.Tensor, out_dtype: torch.dtype) -> bool:
+    """Whether a call that the two-pass path takes in any type may go to a
+    kernel instead: queries and output of the kernels' types."""
+    types = (torch.float16, torch.bfloat16, torch.float32)
+    return queries.dtype in types and out_dtype in types
 
 
 def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: int,
@@ -220,6 +227,10 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
     # caches attend over the rounded values here too
     rounded = bool(buffered) and cache.dtype == torch.bfloat16 and \
         ops["kind"] in ("grouped_il", "grouped", "turboquant_il", "turboquant", "sunshape_v")
+    if rounded:  # two passes elsewhere, which take queries of any layout
+        if ops.get("k_heavy") is not None or not _kernels_take(queries, out_dtype):
+            return None
+        q = q.contiguous()
     # a prompt against a hybrid cache: compressed keys from the codebook,
     # buffered keys whole, values materialised once in the interleaved layout
     # (fp16 copies of quantised values only for the whole-group prompts at
@@ -245,8 +256,6 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
                 codec.last_score_backend = "hip" if rounded else "hip_prefill_mfma_hybrid"
                 return out
     if rounded:
-        if ops.get("k_heavy") is not None:
-            return None
         # the compressed values in bf16, token-major, for the bf16 decode
         tc = cache.compressed_offset
         ops = {"kind": "dense", "idx": ops["idx"][:, :, :tc].contiguous(),
@@ -498,11 +507,13 @@ def sunshape_sdpa(queries: torch.Tensor, cache: SunShapeKVCache | HybridSunShape
     # and so does an array mask over few query rows
     can_fuse = (mask is None or use_causal) and compressed > 0
     array = None
-    if compressed > 0 and hq // hkv * tq <= _MASKED_ROWS and _plain_mask(mask):
+    if compressed > 0 and hq // hkv * tq <= _MASKED_ROWS and _plain(mask) and \
+            _kernels_take(queries, out_dtype):
         array = _hip.attn_mask(mask.to(queries.device), (b_, hq, tq, t_kv))
     if can_fuse or array is not None:
-        out = _fused(cache, queries, scale, use_causal, t_kv - tq if use_causal else 0,
-                     out_dtype, array)
+        # (the two-pass path takes queries of any layout under a mask)
+        out = _fused(cache, queries if array is None else queries.contiguous(), scale, use_causal,
+                     t_kv - tq if use_causal else 0, out_dtype, array)
         if out is not None:
             if array is not None:  # the name the two-pass path reports for a mask
                 cache.codec.last_score_backend = "hip"

@@ -469,3 +469,28 @@ def test_masks_of_any_magnitude_equal_the_two_pass_path(backend, bits, dtype, d,
             assert torch.isfinite(ref).all() and torch.isfinite(got).all(), (low, mdt)
             err = (got - ref).abs().amax((1, 2, 3)) / ref.abs().amax((1, 2, 3))
             assert float(err.max()) <= REL_TOL, (low, mdt, err)
+
+
+@pytest.mark.parametrize("backend,bits,dtype,d,buffer,masked,t_q", [
+    ("fp16", 0, torch.float16, 128, 128, True, 3),
+    ("fp16", 0, torch.bfloat16, 64, 40, True, 2),
+    ("sunshape", 8, torch.float16, 128, 30, True, 2),
+    ("grouped", 2, torch.bfloat16, 128, 30, False, 3),      # bf16 hybrids of quantised values
+    ("turboquant", 4, torch.bfloat16, 64, 30, False, 200),  # ... and their prompts
+    ("turboquant", 3, torch.bfloat16, 128, 30, True, 2),
+])
+def test_query_layouts_and_types_of_the_two_pass_path(backend, bits, dtype, d, buffer, masked, t_q):
+    """Calls that the two-pass path takes in any layout and type: queries as
+    (B, T, H, D) seen through transpose(1, 2), float64 queries and outputs."""
+    cache = _masked_cache(backend, bits, dtype, d, 2, 2, 300, buffer)
+    g = torch.Generator(device="cuda").manual_seed(t_q)
+    q = torch.randn((2, t_q, 8, d), generator=g, device="cuda").to(dtype).transpose(1, 2)
+    mask = torch.arange(300, device="cuda") > 9 if masked else "causal"
+    ref = attention._two_pass(cache, q, 0.11, mask, torch.float32)
+    got = S.sunshape_sdpa(q, cache, 0.11, mask, out_dtype=torch.float32)
+    assert rel_err(got.cpu().numpy(), ref.cpu().numpy()) <= REL_TOL
+    same = S.sunshape_sdpa(q.contiguous(), cache, 0.11, mask, out_dtype=torch.float32)
+    assert torch.equal(got, same)
+    for queries, out_dtype in ((q.double(), None), (q, torch.float64)):
+        got = S.sunshape_sdpa(queries, cache, 0.11, mask, out_dtype=out_dtype)
+        assert torch.equal(got, attention._two_pass(cache, queries, 0.11, mask, torch.float64))
