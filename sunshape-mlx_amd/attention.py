@@ -194,11 +194,15 @@ def _plain(t) -> bool:
             and not torch._C._functorch.is_functorch_wrapped_tensor(t))
 
 
-def _kernels_take(queries: torch.Tensor, out_dtype: torch.dtype) -> bool:
+def _kernels_take(cache, queries: torch.Tensor, out_dtype: torch.dtype) -> bool:
     """Whether a call that the two-pass path takes in any type may go to a
-    kernel instead: queries and output of the kernels' types."""
+    kernel instead: queries and output of the kernels' types, and no gradient
+    through the queries or the stored tokens."""
     types = (torch.float16, torch.bfloat16, torch.float32)
-    return queries.dtype in types and out_dtype in types
+    stores = (getattr(cache, n, None) for n in ("_values", "_values_fp16", "_key_buffer",
+                                                "_value_buffer"))
+    return (queries.dtype in types and out_dtype in types and
+            all(_plain(t) for t in (queries, *stores) if t is not None))
 
 
 def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: int,
@@ -228,7 +232,7 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
     rounded = bool(buffered) and cache.dtype == torch.bfloat16 and \
         ops["kind"] in ("grouped_il", "grouped", "turboquant_il", "turboquant", "sunshape_v")
     if rounded:  # two passes elsewhere, which take queries of any layout
-        if ops.get("k_heavy") is not None or not _kernels_take(queries, out_dtype):
+        if ops.get("k_heavy") is not None or not _kernels_take(cache, queries, out_dtype):
             return None
         q = q.contiguous()
     # a prompt against a hybrid cache: compressed keys from the codebook,
@@ -508,7 +512,7 @@ def sunshape_sdpa(queries: torch.Tensor, cache: SunShapeKVCache | HybridSunShape
     can_fuse = (mask is None or use_causal) and compressed > 0
     array = None
     if compressed > 0 and hq // hkv * tq <= _MASKED_ROWS and _plain(mask) and \
-            _kernels_take(queries, out_dtype):
+            _kernels_take(cache, queries, out_dtype):
         array = _hip.attn_mask(mask.to(queries.device), (b_, hq, tq, t_kv))
     if can_fuse or array is not None:
         # (the two-pass path takes queries of any layout under a mask)

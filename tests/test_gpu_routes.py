@@ -481,7 +481,8 @@ def test_masks_of_any_magnitude_equal_the_two_pass_path(backend, bits, dtype, d,
 ])
 def test_query_layouts_and_types_of_the_two_pass_path(backend, bits, dtype, d, buffer, masked, t_q):
     """Calls that the two-pass path takes in any layout and type: queries as
-    (B, T, H, D) seen through transpose(1, 2), float64 queries and outputs."""
+    (B, T, H, D) seen through transpose(1, 2), float64 queries and outputs,
+    and gradients through the queries' scores of buffered keys."""
     cache = _masked_cache(backend, bits, dtype, d, 2, 2, 300, buffer)
     g = torch.Generator(device="cuda").manual_seed(t_q)
     q = torch.randn((2, t_q, 8, d), generator=g, device="cuda").to(dtype).transpose(1, 2)
@@ -494,3 +495,11 @@ def test_query_layouts_and_types_of_the_two_pass_path(backend, bits, dtype, d, b
     for queries, out_dtype in ((q.double(), None), (q, torch.float64)):
         got = S.sunshape_sdpa(queries, cache, 0.11, mask, out_dtype=out_dtype)
         assert torch.equal(got, attention._two_pass(cache, queries, 0.11, mask, torch.float64))
+    grads = []
+    for fn in (S.sunshape_sdpa, lambda x, c, s, m: attention._two_pass(c, x, s, m, x.dtype)):
+        x = q.float().requires_grad_()
+        out = fn(x, cache, 0.11, mask)
+        if out.requires_grad:  # (no buffered keys: the compressed scores carry none)
+            out.square().sum().backward()
+        grads.append(x.grad)
+    assert grads[0] is grads[1] is None or torch.equal(*grads)
