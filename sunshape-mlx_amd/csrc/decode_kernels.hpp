@@ -4550,8 +4550,11 @@ __global__ void __launch_bounds__(kDecodeThreads)
                 const float p = prob(tg + i * TPG);
                 float vx[8];
                 elems(vr[i], mb.v, i, vx);
+                // (past the last token its row again, with p = 0, which an
+                // infinite value would turn into NaN)
+                const bool ok = j0 + tg + i * TPG < n;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) ba[e] = fmaf(p, vx[e], ba[e]);
+                for (int e = 0; e < 8; ++e) ba[e] = fmaf(p, ok ? vx[e] : 0.f, ba[e]);
             }
             __syncthreads();  // bp is written again by the next chunk
         }

@@ -503,3 +503,22 @@ def test_query_layouts_and_types_of_the_two_pass_path(backend, bits, dtype, d, b
             out.square().sum().backward()
         grads.append(x.grad)
     assert grads[0] is grads[1] is None or torch.equal(*grads)
+
+
+@pytest.mark.parametrize("bdt,t_buf", [(torch.float16, 1), (torch.float32, 127), (torch.bfloat16, 131)])
+def test_merge_keeps_an_infinite_value_of_the_last_buffered_token(bdt, t_buf):
+    """One dim of the last token is infinite: infinite in the output, the
+    other dims as without it."""
+    d, t_kv = 128, 200
+    cents, perm, idx, vals, q = decode_case(t_buf, 1, 8, 2, d, t_kv, 1, t_kv, v_dtype=np.float32)
+    g = torch.Generator(device="cuda").manual_seed(t_buf)
+    kb, vb = torch.randn((2, 1, 2, t_buf, d), generator=g, device="cuda").to(bdt)
+    outs = []
+    for x in (1.0, float("inf")):
+        vb[..., -1, 5] = x
+        outs.append(_hip.decode_attn_dense(t(q), 0.1, t(perm), t(cents), t(idx), t(vals), t_kv,
+                                           buf_keys=kb, buf_values=vb, buf_len=t_buf,
+                                           out_dtype=torch.float32))
+    assert bool((outs[1][..., 5] == float("inf")).all())
+    outs[1][..., 5] = outs[0][..., 5]
+    assert torch.equal(*outs)
