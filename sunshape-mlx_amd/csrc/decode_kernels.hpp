@@ -510,6 +510,12 @@ template <class VF, class = void>
 struct VfTable : std::false_type {};  // the format reads a table in LDS (VF::stage_table)
 template <class VF>
 struct VfTable<VF, std::void_t<decltype(VF::kTable)>> : std::bool_constant<VF::kTable> {};
+// a dim whose hi part is infinite takes no lower parts: a probability's may be
+// zero or negative, and 0 * infinity and infinity - infinity are NaN
+template <class VF, class = void>
+struct VfKeepsInf : std::false_type {};
+template <class VF>
+struct VfKeepsInf<VF, std::void_t<decltype(VF::kKeepsInf)>> : std::bool_constant<VF::kKeepsInf> {};
 template <class VF, class = void>
 struct VfArgsToLds : std::false_type {};  // the format's accumulator hand-off reads its Args
 template <class VF>
@@ -2178,6 +2184,7 @@ struct VBf16 {
     static constexpr bool kHybridBuffer = true;
     static constexpr bool kHeavyCapable = false;
     static constexpr float kMaxLag = 8.f;  // bf16 probabilities (float32's exponent range)
+    static constexpr bool kKeepsInf = true;
     static constexpr bool kPrivateRing = false;
     static constexpr int kTileV = kWave * D * 2;
     static constexpr int kLoadsV = kTileV / 1024;
@@ -2223,7 +2230,7 @@ struct VBf16 {
     }
     __device__ static void init(State &) {}
     __device__ static void pv(Tile &tv, State &, f32x4 (&acc)[NT], const float (&p)[kMfmaRows],
-                              const float (&corr)[kMfmaRows], bool rescale, int, _Float16 *pw16,
+                              const float (&corr)[kMfmaRows], bool rescale, int n_in, _Float16 *pw16,
                               int lane) {
         const int g = lane >> 4, l16 = lane & 15;
         uint16_t *pw = reinterpret_cast<uint16_t *>(pw16);
@@ -2245,7 +2252,21 @@ struct VBf16 {
 #pragma unroll
             for (int n = 0; n < NT; ++n) acc[n] *= cv4;
         }
-        // (tokens past the split's end hold its last token's values, p = 0)
+        if (n_in < kWave) {  // last, partial tile: zero tokens >= t_end (p = 0 there)
+#pragma unroll
+            for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int n_ok = n_in - (32 * s2 + 8 * g + 4 * h);
+                    const uint32_t zx = n_ok >= 2 ? 0xffffffffu : n_ok == 1 ? 0x0000ffffu : 0u;
+                    const uint32_t zy = n_ok >= 4 ? 0xffffffffu : n_ok == 3 ? 0x0000ffffu : 0u;
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) {
+                        tv.v[s2][n][h].x &= zx;
+                        tv.v[s2][n][h].y &= zy;
+                    }
+                }
+        }
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
             uint4 a = make_uint4(0u, 0u, 0u, 0u);
@@ -3717,7 +3738,13 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
         for (int w = 0; w < NC; ++w) {
             const float f = fast_exp2((mw[w] - M) * mu);
             L = fmaf(lw[w], f, L);
-            A += (hi[w] + lo[w]) * f;
+            if constexpr (MK || VfKeepsInf<VF>::value) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    A[k] = fmaf(hi[w][k] + (fabsf(hi[w][k]) < INFINITY ? lo[w][k] : 0.f), f, A[k]);
+            } else {
+                A += (hi[w] + lo[w]) * f;
+            }
         }
         if (has_buf) {
             const float f = fast_exp2((mb - M) * mu);
@@ -3832,7 +3859,11 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
             for (int j = 0; j < kMergeLoads; ++j) {
                 const float w = part + kMergeParts * j < S ? fast_exp2((__uint_as_float(mv[j][0]) - Mr) * mu) : 0.f;
                 Lr = fmaf(__uint_as_float(mv[j][1]), w, Lr);
-                Ar += av[j] * w;
+                if constexpr (MK || VfKeepsInf<VF>::value) {  // (a slot past the last split: 0 * infinity)
+                    if (part + kMergeParts * j < S) Ar += av[j] * w;
+                } else {
+                    Ar += av[j] * w;
+                }
             }
         }
         // parts 1.. hand their (M, L, A) to part 0 through LDS (the ring)

@@ -522,3 +522,34 @@ def test_merge_keeps_an_infinite_value_of_the_last_buffered_token(bdt, t_buf):
     assert bool((outs[1][..., 5] == float("inf")).all())
     outs[1][..., 5] = outs[0][..., 5]
     assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("dtype,d,t_kv,masked", [
+    (torch.bfloat16, 128, 67, False), (torch.bfloat16, 128, 1500, False),
+    (torch.bfloat16, 64, 131, True), (torch.float16, 128, 1500, True),
+])
+def test_decodes_keep_infinite_values(dtype, d, t_kv, masked):
+    """Infinite values of a cache: infinite in their dims of the output, and
+    the other dims as without them.  (Of a key hidden by the mask: NaN, 0 *
+    infinity, as in the two-pass path.)"""
+    cache = _masked_cache("fp16", 0, dtype, d, 2, 1, t_kv, 128)
+    q = torch.randn((1, 8, 1, d), generator=torch.Generator(device="cuda").manual_seed(1),
+                    device="cuda").to(dtype)
+    mask = torch.arange(t_kv, device="cuda") != 1 if masked else None
+    plain = S.sunshape_sdpa(q, cache, 0.02, mask, out_dtype=torch.float32)
+    dims = {7: (t_kv - 1, torch.inf), 20: (t_kv // 2, -torch.inf), 40: (0, torch.inf)}
+    if masked:
+        dims[41] = (1, torch.inf)
+    v = cache._values  # (B, H, cap, D), or (B, H, cap/8, D, 8)
+    for dim, (tok, x) in dims.items():
+        if v.dim() == 5:
+            v[:, :, tok // 8, dim, tok % 8] = x
+        else:
+            v[:, :, tok, dim] = x
+    cache._version += 1
+    got = S.sunshape_sdpa(q, cache, 0.02, mask, out_dtype=torch.float32)
+    for dim, (_, x) in dims.items():
+        col = got[..., dim]
+        assert bool((torch.isnan(col) if dim == 41 else col == x).all()), dim
+        got[..., dim] = plain[..., dim]
+    assert torch.equal(got, plain)
