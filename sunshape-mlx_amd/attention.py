@@ -21,6 +21,7 @@ from __future__ import annotations
 import weakref
 
 import torch
+from torch.autograd import forward_ad as _forward_ad
 
 from . import _hip
 from .cache import HybridSunShapeKVCache, SunShapeKVCache
@@ -190,19 +191,30 @@ def _plain(t) -> bool:
     return (isinstance(t, torch.Tensor)
             and type(t) in (torch.Tensor, torch.nn.Parameter)
             and not (t.requires_grad and torch.is_grad_enabled())
-            and torch.autograd.forward_ad._current_level < 0
+            and _forward_ad._current_level < 0
             and not torch._C._functorch.is_functorch_wrapped_tensor(t))
+
+
+_KERNEL_TYPES = (torch.float16, torch.bfloat16, torch.float32)
 
 
 def _kernels_take(cache, queries: torch.Tensor, out_dtype: torch.dtype) -> bool:
     """Whether a call that the two-pass path takes in any type may go to a
     kernel instead: queries and output of the kernels' types, and no gradient
-    through the queries or the stored tokens."""
-    types = (torch.float16, torch.bfloat16, torch.float32)
-    stores = (getattr(cache, n, None) for n in ("_values", "_values_fp16", "_key_buffer",
-                                                "_value_buffer"))
-    return (queries.dtype in types and out_dtype in types and
-            all(_plain(t) for t in (queries, *stores) if t is not None))
+    or tangent through the queries or the stored tokens."""
+    if queries.dtype not in _KERNEL_TYPES or out_dtype not in _KERNEL_TYPES or \
+            _forward_ad._current_level >= 0:
+        return False
+    if not torch.is_grad_enabled():
+        return True
+    if isinstance(cache, HybridSunShapeKVCache):
+        stores = (queries, cache._values_fp16, cache._key_buffer, cache._value_buffer)
+    else:
+        stores = (queries, cache._values)
+    for t in stores:
+        if t is not None and t.requires_grad:
+            return False
+    return True
 
 
 def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: int,

@@ -2233,6 +2233,21 @@ struct VBf16 {
                               const float (&corr)[kMfmaRows], bool rescale, int n_in, _Float16 *pw16,
                               int lane) {
         const int g = lane >> 4, l16 = lane & 15;
+        if (n_in < kWave) {  // last, partial tile: zero tokens >= t_end (p = 0 there)
+#pragma unroll
+            for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int n_ok = n_in - (32 * s2 + 8 * g + 4 * h);
+                    const uint32_t zx = n_ok >= 2 ? 0xffffffffu : n_ok == 1 ? 0x0000ffffu : 0u;
+                    const uint32_t zy = n_ok >= 4 ? 0xffffffffu : n_ok == 3 ? 0x0000ffffu : 0u;
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) {
+                        tv.v[s2][n][h].x &= zx;
+                        tv.v[s2][n][h].y &= zy;
+                    }
+                }
+        }
         uint16_t *pw = reinterpret_cast<uint16_t *>(pw16);
 #pragma unroll
         for (int r = 0; r < kMfmaRows; r += 2) {
@@ -2251,21 +2266,6 @@ struct VBf16 {
             const f32x4 cv4 = f32x4{corr[0], corr[1], corr[2], corr[3]};
 #pragma unroll
             for (int n = 0; n < NT; ++n) acc[n] *= cv4;
-        }
-        if (n_in < kWave) {  // last, partial tile: zero tokens >= t_end (p = 0 there)
-#pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int n_ok = n_in - (32 * s2 + 8 * g + 4 * h);
-                    const uint32_t zx = n_ok >= 2 ? 0xffffffffu : n_ok == 1 ? 0x0000ffffu : 0u;
-                    const uint32_t zy = n_ok >= 4 ? 0xffffffffu : n_ok == 3 ? 0x0000ffffu : 0u;
-#pragma unroll
-                    for (int n = 0; n < NT; ++n) {
-                        tv.v[s2][n][h].x &= zx;
-                        tv.v[s2][n][h].y &= zy;
-                    }
-                }
         }
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
@@ -3859,11 +3859,9 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
             for (int j = 0; j < kMergeLoads; ++j) {
                 const float w = part + kMergeParts * j < S ? fast_exp2((__uint_as_float(mv[j][0]) - Mr) * mu) : 0.f;
                 Lr = fmaf(__uint_as_float(mv[j][1]), w, Lr);
-                if constexpr (MK || VfKeepsInf<VF>::value) {  // (a slot past the last split: 0 * infinity)
-                    if (part + kMergeParts * j < S) Ar += av[j] * w;
-                } else {
-                    Ar += av[j] * w;
-                }
+                if constexpr (MK || VfKeepsInf<VF>::value)  // (a slot past the last split: 0 * infinity)
+                    av[j] = part + kMergeParts * j < S ? av[j] : f32x4{0.f, 0.f, 0.f, 0.f};
+                Ar += av[j] * w;
             }
         }
         // parts 1.. hand their (M, L, A) to part 0 through LDS (the ring)
