@@ -100,7 +100,7 @@ def _fused_step(cache: SunShapeKVCache, queries: torch.Tensor, scale: float, cau
     tensors = (cache._key_indices, cache._values, codec.kernel_codebook(), codec.centroids)
     if perm is not None:
         tensors += (perm,)
-    key = ("step", q.shape, q.dtype, q.device, kscale)
+    key = ("step", q.shape, q.dtype, q.device, kscale, *[t.data_ptr() for t in tensors])
     held = getattr(cache, "_step_prepared", None)
     if held is not None and held[0] == key and len(held[1]) == len(tensors) and \
             all(r() is t for r, t in zip(held[1], tensors)):
@@ -140,7 +140,7 @@ def _fused_hybrid_step(cache: HybridSunShapeKVCache, queries: torch.Tensor, scal
                                                cache._key_buffer, cache._value_buffer)
     if perm is not None:
         tensors += (perm,)
-    key = ("hstep", q.shape, q.dtype, q.device, kscale)
+    key = ("hstep", q.shape, q.dtype, q.device, kscale, *[t.data_ptr() for t in tensors])
     held = getattr(cache, "_hstep_prepared", None)
     if held is not None and held[0] == key and len(held[1]) == len(tensors) and \
             all(r() is t for r, t in zip(held[1], tensors)):

@@ -249,8 +249,11 @@ class SunShapeKVCache:
         if not self.values_interleaved or c.mode != "profileperm_baseline" or c.n_centroids > 256:
             return None
         cb, pm, pre = c.centroids, c.permutation, c.encode_codebook()
+        # (addresses too: a tensor may be given other memory in place)
         key = (self._key_indices, self._values, cb, cb._version, pm,
-               pm._version if pm is not None else 0, pre)
+               pm._version if pm is not None else 0, pre,
+               self._key_indices.data_ptr(), self._values.data_ptr(), cb.data_ptr(),
+               pm.data_ptr() if pm is not None else 0)
         held = self._append_plan
         if held is None or len(held[0]) != len(key) or \
                 not all(a is b or (isinstance(a, int) and a == b) for a, b in zip(held[0], key)):
@@ -612,6 +615,8 @@ class HybridSunShapeKVCache:
         key = (self._key_buffer, self._value_buffer, self._key_indices, self._values_il,
                self._value_scales, self._value_zeros, cb, cb._version, pm,
                pm._version if pm is not None else 0)
+        # (addresses too: a tensor may be given other memory in place)
+        key += tuple([t.data_ptr() for t in key if isinstance(t, torch.Tensor)])
         held = self._step_plan
         if held is not None and len(held[0]) == len(key) and \
                 all(a is b or (isinstance(a, int) and a == b) for a, b in zip(held[0], key)):

@@ -56,6 +56,21 @@ def _compact_index_dtype(n_centroids: int) -> torch.dtype:
     return torch.int64
 
 
+def _seen(t: torch.Tensor | None):
+    """What a result derived from ``t`` is kept with: the tensor, its version,
+    and an alias that holds its memory (while held, no other memory has that
+    address)."""
+    return None if t is None else (t, t._version, t.detach())
+
+
+def _unchanged(seen, t: torch.Tensor | None) -> bool:
+    """Whether ``t`` is as :func:`_seen` saw it: not another tensor, updated
+    in place, or given other memory in place (by set_ or .data)."""
+    if seen is None or t is None:
+        return seen is t
+    return seen[0] is t and seen[1] == t._version and seen[2].data_ptr() == t.data_ptr()
+
+
 def _np(x) -> np.ndarray:
     if isinstance(x, torch.Tensor):
         return x.detach().float().cpu().numpy()
@@ -331,7 +346,7 @@ class SunShapeBlockCodec:
     def _any_heavy(self) -> bool:
         """Whether :meth:`heavy_dims` is not None.  Reading a mask on the GPU
         waits for it, so the answer is kept with the mask and read again when
-        it changes (another tensor or an in-place update).  A mask on the host
+        it changes (another tensor, other memory or an in-place update).  A mask on the host
         may share its memory with an array that changes unseen and costs
         nothing to read: it is read each time."""
         if self.mode != "profileperm_mixed_precision" or not self.heavy_fp16:
@@ -340,10 +355,10 @@ class SunShapeBlockCodec:
         if not hb.is_cuda or hb.is_inference():  # (no version there to tell an update by)
             return bool(hb.any())
         held = getattr(self, "_heavy_seen", None)
-        if held is None or held[0] is not hb or held[1] != hb._version:
-            held = (hb, hb._version, bool(hb.any()))
+        if held is None or not _unchanged(held[0], hb):
+            held = (_seen(hb), bool(hb.any()))
             self._heavy_seen = held
-        return held[2]
+        return held[1]
 
     def kernel_value_transform(self) -> torch.Tensor:
         """(D, D) float32 matrix taking a codec-space row to the original
@@ -357,9 +372,9 @@ class SunShapeBlockCodec:
             src = self.rotation
         else:
             src = None
-        key = (self.mode, None if src is None else (src.data_ptr(), src._version), str(self.device))
+        key = (self.mode, str(self.device))
         cached = getattr(self, "_kernel_value_transform", None)
-        if cached is None or cached[0] != key:
+        if cached is None or cached[0] != key or not _unchanged(cached[1], src):
             d = self.head_dim
             if self.mode in PERM_MODES:
                 m = torch.zeros((d, d), dtype=torch.float32, device=self.device)
@@ -368,9 +383,9 @@ class SunShapeBlockCodec:
                 m = self.rotation.float().contiguous()
             else:
                 m = torch.eye(d, dtype=torch.float32, device=self.device)
-            cached = (key, m)
+            cached = (key, _seen(src), m)
             self._kernel_value_transform = cached
-        return cached[1]
+        return cached[2]
 
     def scoring_centroids(self) -> torch.Tensor:
         """The centroids a cache's scores read.  With fp16 heavy blocks
@@ -386,25 +401,24 @@ class SunShapeBlockCodec:
         if not self._any_heavy():
             return c
         hb = self.mixed_high_precision_blocks
-        key = (c.data_ptr(), c._version, hb.data_ptr(), hb._version, str(c.device))
         cached = getattr(self, "_scoring_centroids", None)
-        if cached is None or cached[0] != key:
+        if cached is None or not (_unchanged(cached[0], c) and _unchanged(cached[1], hb)):
             z = c.clone()
             z[hb.to(torch.bool).to(z.device)] = 0.0
-            cached = (key, z.contiguous())
+            cached = (_seen(c), _seen(hb), z.contiguous())
             self._scoring_centroids = cached
-        return cached[1]
+        return cached[2]
 
     def kernel_codebook(self) -> torch.Tensor:
         """``scoring_centroids()`` as the split-fp16 buffer read by the
         matrix-core LUT build of the fused decodes, prepared once and rebuilt
-        when the centroids change (new tensor, device or in-place update)."""
+        when the centroids change (new tensor, memory or in-place update)."""
         c = self.scoring_centroids()
         cached = getattr(self, "_kernel_codebook", None)
-        if cached is None or cached[0] is not c or cached[1] != c._version:
-            cached = (c, c._version, _hip.codebook_f16x2(c))
+        if cached is None or not _unchanged(cached[0], c):
+            cached = (_seen(c), _hip.codebook_f16x2(c))
             self._kernel_codebook = cached
-        return cached[2]
+        return cached[1]
 
     def encode_codebook(self, centroids: torch.Tensor | None = None) -> torch.Tensor | None:
         """The prepared codebook of the matrix-core encoder for ``centroids``
@@ -414,10 +428,10 @@ class SunShapeBlockCodec:
         if not _hip.encode_codebook_supported(c):
             return None
         cached = getattr(self, "_encode_codebook", None)
-        if cached is None or cached[0] is not c or cached[1] != c._version:
-            cached = (c, c._version, _hip.encode_codebook(c))
+        if cached is None or not _unchanged(cached[0], c):
+            cached = (_seen(c), _hip.encode_codebook(c))
             self._encode_codebook = cached
-        return cached[2]
+        return cached[1]
 
     def _encode_centroids(self) -> torch.Tensor:
         if self.mode == "profileperm_localmetric_dsq":

@@ -8,7 +8,7 @@ import sunshape_mlx_amd as S
 
 
 @pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
-@pytest.mark.parametrize("how", ["replaced", "in_place", "inference"])
+@pytest.mark.parametrize("how", ["replaced", "in_place", "memory", "inference"])
 def test_scoring_centroids_follow_the_heavy_mask(how, device):
     rng = np.random.default_rng(3)
     codec = S.SunShapeBlockCodec(32, n_centroids=4, device=device,
@@ -26,6 +26,8 @@ def test_scoring_centroids_follow_the_heavy_mask(how, device):
         mask[heavy] = True
         if how == "replaced":
             codec.mixed_high_precision_blocks = mask
+        elif how == "memory":
+            codec.mixed_high_precision_blocks.data = mask
         else:
             codec.mixed_high_precision_blocks.copy_(mask)
         for _ in range(2):

@@ -182,6 +182,44 @@ def test_kept_plan_follows_memory_given_in_place():
     assert torch.equal(got, S.sunshape_sdpa(q, cache, 0.11)) and not torch.equal(got, first)
 
 
+@pytest.mark.parametrize("backend,bits,buffer,stores", [
+    ("fp16", 0, 128, ("_key_indices", "_values")),
+    ("fp16", 0, 20, ("_key_indices", "_values_il8", "_key_buffer", "_value_buffer")),
+    ("grouped", 2, 20, ("_key_indices", "_values_il", "_value_scales", "_key_buffer")),
+])
+@pytest.mark.parametrize("held", [True, False])
+def test_steps_follow_memory_given_in_place(backend, bits, buffer, stores, held):
+    """Codebook, permutation and stores given other memory through ``.data``:
+    the next step (one launch, or an append and a decode) reads and writes
+    there, as where they are replaced by other tensors."""
+    caches = [_masked_cache(backend, bits, torch.float16, 128, 2, 1, 300, buffer) for _ in range(2)]
+    g = torch.Generator(device="cuda").manual_seed(9)
+    k, v = torch.randn((2, 2, 1, 2, 1, 128), generator=g, device="cuda").half()
+    q = torch.randn((1, 8, 1, 128), generator=g, device="cuda").half()
+    outs, old = [], []
+    for i in range(2):
+        for cache in caches:
+            cache.fuse_steps = held
+            cache.update_and_fetch(k[i], v[i])
+            outs.append(S.sunshape_sdpa(q, cache, 0.11))
+            assert ("step" in cache.codec.last_score_backend) == held
+        for in_place, cache in enumerate(caches if i == 0 else ()):
+            c = cache.codec
+            for where, name, new in (
+                    [(c, "permutation", c.permutation.flip(0)), (c, "centroids", c.centroids * 0.5)] +
+                    [(cache, n, getattr(cache, n).clone()) for n in stores]):
+                if not in_place:
+                    setattr(where, name, new)
+                    continue
+                old.append(getattr(where, name).detach())  # stays allocated
+                getattr(where, name).data = new
+                old[-1].zero_()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[2], outs[3])
+    assert not torch.equal(outs[0], outs[2])
+    assert torch.equal(caches[0].key_indices, caches[1].key_indices)
+    assert not any(bool(t.any()) for t in old)
+
+
 def test_masks_that_carry_gradients_keep_the_two_pass_path():
     """A learned bias gets its gradient, a dual bias its tangent and vmap its
     batch: equal to the two-pass path's, and the same values as the fused
