@@ -247,17 +247,31 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
         if ops.get("k_heavy") is not None or not _kernels_take(cache, queries, out_dtype):
             return None
         q = q.contiguous()
+    # The two passes weigh a float32 cache's values in float32, the
+    # matrix-core decodes of these values with 16 or 22 bits: 7e-6 to 3.2e-5 of
+    # the result off 64 bits there, 8e-7 in two passes.  (Values that
+    # two passes round to 16 bits lose 1.6e-4 or more by that.)
+    if mask is not None and cache.dtype == torch.float32 and \
+            (ops["kind"] in ("grouped_il", "turboquant_il") or
+             (ops["kind"] == "sunshape_v" and d == 128)):
+        return None
     # a prompt against a hybrid cache: compressed keys from the codebook,
     # buffered keys whole, values materialised once in the interleaved layout
     # (fp16 copies of quantised values only for the whole-group prompts at
-    # head_dim 128: elsewhere the decodes' float32 values are the more exact)
+    # head_dim 128: elsewhere the decodes' float32 values are the more exact).
+    # Float32 results of those prompts alone, and of rounded values: the
+    # decodes' are 2.4e-7 to 3.8e-7 off 64 bits where the prompt kernel's are
+    # 3.6e-7 to 5.2e-7 (16-bit results do not show it)
     whole = ops["kind"] in ("il8", "dense") or rounded
+    full = out_dtype == torch.float32
     if mask is None and isinstance(cache, HybridSunShapeKVCache) and ops.get("k_heavy") is None and \
             (cache.dtype == torch.float16 or
              (cache.dtype == torch.bfloat16 and whole)) and \
             _hip.prompt_supported(q, cache.n_kv_heads, codec.n_blocks, cache.offset,
                                   cache.dtype) and \
-            (whole or _hip.prefill_supported(hq, cache.n_kv_heads, tq, d, codec.n_blocks)):
+            (rounded or (whole and not full) or
+             (cache.dtype == torch.float16 and
+              _hip.prefill_supported(hq, cache.n_kv_heads, tq, d, codec.n_blocks))):
         pf = cache.prefill_operands()
         if pf is not None:
             vil8, rows, fac, t_raw0 = pf
@@ -297,6 +311,8 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
         out = None
         try:
             if (kind == "il8" or ops["values"].dtype == torch.bfloat16) and \
+                    (not full or (kind == "il8" and _hip.prefill_supported(
+                        hq, cache.n_kv_heads, tq, d, codec.n_blocks))) and \
                     _hip.prompt_supported(q, cache.n_kv_heads, codec.n_blocks, t_kv,
                                           ops["values"].dtype):
                 v8 = ops["values"]

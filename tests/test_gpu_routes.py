@@ -211,7 +211,7 @@ def test_steps_follow_memory_given_in_place(backend, bits, buffer, stores, held)
                 if not in_place:
                     setattr(where, name, new)
                     continue
-                old.append(getattr(where, name).detach())  # stays allocated
+                old.append(getattr(where, name).data)  # stays allocated, versions of its own
                 getattr(where, name).data = new
                 old[-1].zero_()
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[2], outs[3])
@@ -311,6 +311,35 @@ def test_prompt_kernel_matches_the_definition(b, hq, hkv, d, t_q, past, causal, 
             ref = torch.softmax(s, dim=-1) @ v[bi, h // rep].double()
             worst = max(worst, float((out[bi, h] - ref).abs().max() / ref.abs().max()))
     assert worst <= REL_TOL
+
+
+@pytest.mark.parametrize("dtype,d,hq,hkv,buffer", [
+    (torch.float16, 64, 8, 2, 128), (torch.float16, 128, 14, 2, 128), (torch.bfloat16, 128, 8, 2, 128),
+    (torch.bfloat16, 64, 8, 2, 128), (torch.float16, 64, 8, 2, 40), (torch.bfloat16, 128, 8, 2, 40),
+])
+def test_float32_results_of_prompts_are_the_decodes(dtype, d, hq, hkv, buffer):
+    """Prompts of shapes that a decode takes as well: the prompt kernel for
+    results in the cache's type, the decode, which is nearer to 64 bits, for
+    float32 ones."""
+    cache = _masked_cache("fp16", 0, dtype, d, hkv, 1, 1400, buffer)
+    g = torch.Generator(device="cuda").manual_seed(d + hq)
+    q = torch.randn((1, hq, 900, d), generator=g, device="cuda").to(dtype)
+    got = S.sunshape_sdpa(q, cache, 0.11, "causal")
+    assert "prefill" in cache.codec.last_score_backend
+    exact = S.sunshape_sdpa(q, cache, 0.11, "causal", out_dtype=torch.float32)
+    assert "fused" in cache.codec.last_score_backend
+    assert rel_err(got.float().cpu().numpy(), exact.cpu().numpy()) <= REL_TOL + torch.finfo(dtype).eps
+
+
+@pytest.mark.parametrize("backend,bits,d,buffer", [("grouped", 2, 128, 20), ("grouped", 4, 64, 20),
+                                                   ("turboquant", 2, 128, 20),
+                                                   ("sunshape", 8, 128, 20)])
+def test_masked_float32_caches_keep_float32_weights(backend, bits, d, buffer):
+    cache = _masked_cache(backend, bits, torch.float32, d, 2, 1, 700, buffer)
+    q = torch.randn((1, 8, 1, d), device="cuda")
+    mask = torch.arange(700, device="cuda") > 9
+    assert torch.equal(S.sunshape_sdpa(q, cache, 0.11, mask),
+                       attention._two_pass(cache, q, 0.11, mask, torch.float32))
 
 
 @pytest.mark.parametrize("n_t,offset,d,dtype,pad", [
