@@ -29,7 +29,8 @@
 //
 // Values: fp16, P as one fp16 operand of p * 2^11 (as prefill32) or as its hi
 // and lo parts (22 bits, as the decode kernels; ss_prefill_attn chooses), or
-// bfloat16 with P as three bfloat16 parts (24 bits, float32's own).
+// bfloat16 with P as three bfloat16 parts (24 bits, float32's own; all above
+// zero, so that an infinite value stays infinite where it is seen).
 #include "ss_common.hpp"
 
 #include <algorithm>
@@ -42,7 +43,6 @@ namespace {
 typedef _Float16 pg_f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 pg_f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 pg_bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 pg_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float pg_f32x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 pg_f16x2 __attribute__((ext_vector_type(2)));
 typedef float pg_f32x16 __attribute__((ext_vector_type(16)));
@@ -56,6 +56,7 @@ using pg_lds = __attribute__((address_space(3))) T;
 // the fp16 maximum at 2^(kPgExp + kPgLag)).
 constexpr float kPgLag = 4.f;
 constexpr float kPgExp = 11.f;
+constexpr float kPgMore = 1.f + 0x1p-23f;
 
 struct FragArgs {
     const void *q;
@@ -86,6 +87,11 @@ struct FragArgs {
 
 __device__ __forceinline__ float pg_lane(float x, int src) {
     return __int_as_float(__builtin_amdgcn_ds_bpermute(src << 2, __float_as_int(x)));
+}
+
+// The high halves of two words as one, a's the lower.
+__device__ __forceinline__ uint32_t pg_high_halves(uint32_t a, uint32_t b) {
+    return __builtin_amdgcn_perm(b, a, 0x07060302u);
 }
 
 template <int N>
@@ -402,17 +408,19 @@ __global__ void __launch_bounds__(RW *KW *kWave, 2) prefill_frag_kernel(FragArgs
             ps += x0;
             ps += x1;
             if constexpr (BF) {
-                const pg_bf16x2 hi = __builtin_convertvector((pg_f32x2){x0, x1}, pg_bf16x2);
-                const uint32_t u = __builtin_bit_cast(uint32_t, hi);
-                ph[i / 2] = u;
-                const float r0 = x0 - __uint_as_float(u << 16), r1 = x1 - __uint_as_float(u & 0xffff0000u);
-                const uint32_t ul =
-                    __builtin_bit_cast(uint32_t, __builtin_convertvector((pg_f32x2){r0, r1}, pg_bf16x2));
-                pl[i / 2] = ul;
-                pm[i / 2] = __builtin_bit_cast(
-                    uint32_t, __builtin_convertvector((pg_f32x2){r0 - __uint_as_float(ul << 16),
-                                                                 r1 - __uint_as_float(ul & 0xffff0000u)},
-                                                      pg_bf16x2));
+                // truncated parts, all above zero where the probability is
+                // (the factor leaves each at least x * 2^-23 to take, an ulp of
+                // the probability at most): a part that is zero or negative,
+                // as rounded ones are, would make NaN of an infinite value
+                const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
+                ph[i / 2] = pg_high_halves(u0, u1);
+                const float r0 = fmaf(x0, kPgMore, -__uint_as_float(u0 & 0xffff0000u));
+                const float r1 = fmaf(x1, kPgMore, -__uint_as_float(u1 & 0xffff0000u));
+                const uint32_t w0 = __float_as_uint(r0), w1 = __float_as_uint(r1);
+                pl[i / 2] = pg_high_halves(w0, w1);
+                pm[i / 2] = pg_high_halves(
+                    __float_as_uint(fmaf(r0, kPgMore, -__uint_as_float(w0 & 0xffff0000u))),
+                    __float_as_uint(fmaf(r1, kPgMore, -__uint_as_float(w1 & 0xffff0000u))));
             } else {
                 const pg_f16x2 hi = __builtin_convertvector((pg_f32x2){x0, x1}, pg_f16x2);
                 ph[i / 2] = __builtin_bit_cast(uint32_t, hi);
@@ -522,7 +530,8 @@ __global__ void __launch_bounds__(RW *KW *kWave, 2) prefill_frag_kernel(FragArgs
             const int64_t op = orow / a.rep;
             const int oh = (int)(orow - op * a.rep);
             const int64_t off = ((bb * a.n_q_heads + (int64_t)kvh * a.rep + oh) * a.t_q + op) * D;
-            const float inv = Li > 0.f ? 1.f / Li : 0.f;  // acc and l both carry 2^11
+            // acc and l both carry 2^11 (bfloat16 parts: acc an ulp more)
+            const float inv = Li > 0.f ? (BF ? 2.f - kPgMore : 1.f) / Li : 0.f;
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
                 store_from_f32(a.out, a.out_dtype, off + 32 * nt + l32, acc[nt][i] * inv);

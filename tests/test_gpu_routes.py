@@ -620,3 +620,32 @@ def test_decodes_keep_infinite_values(dtype, d, t_kv, masked):
         assert bool((torch.isnan(col) if dim == 41 else col == x).all()), dim
         got[..., dim] = plain[..., dim]
     assert torch.equal(got, plain)
+
+
+@pytest.mark.parametrize("backend,d,t_q,buffer", [
+    ("fp16", 128, 1000, 128), ("fp16", 64, 1100, 128), ("fp16", 128, 2400, 128), ("fp16", 64, 1100, 40),
+    ("grouped", 128, 1000, 40)])
+def test_bf16_prompts_keep_infinite_values(backend, d, t_q, buffer):
+    """Infinite values of tokens that a row sees (of the first alone, with
+    probability 1, in row 0): infinite in their dims of the output, the other
+    dims as without them.  (Of tokens that it does not see: 0 * infinity, as
+    in the two-pass path.)"""
+    cache = _masked_cache(backend, 4, torch.bfloat16, d, 2, 1, t_q, buffer)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q = torch.randn((1, 8, t_q, d), generator=g, device="cuda").bfloat16()
+    before = S.get_kernel_stats()
+    plain = S.sunshape_sdpa(q, cache, 0.02, "causal")
+    assert any(n > before.get(k, 0) for k, n in S.get_kernel_stats().items() if "prefill" in k)
+    dims = {7: (t_q - 1, torch.inf)}  # (buffered, where there is a buffer)
+    store, base = (cache._values, 0) if buffer == 128 else \
+        (cache._value_buffer, cache.compressed_offset - cache._buf_start)
+    if buffer == 128:
+        dims.update({20: (t_q // 2, -torch.inf), 40: (0, torch.inf)})
+    for dim, (tok, x) in dims.items():
+        store[:, :, tok - base, dim] = x
+    cache._version += 1
+    got = S.sunshape_sdpa(q, cache, 0.02, "causal")
+    for dim, (tok, x) in dims.items():
+        assert bool((got[:, :, tok:, dim] == x).all()), dim
+        got[..., dim] = plain[..., dim]
+    assert torch.equal(got, plain)
