@@ -18,13 +18,14 @@ GPU (HIP LUT and score kernels, torch softmax and matmul), takes the rest.
 
 from __future__ import annotations
 
+import operator
 import weakref
 
 import torch
 from torch.autograd import forward_ad as _forward_ad
 
 from . import _hip
-from .cache import HybridSunShapeKVCache, SunShapeKVCache
+from .cache import HybridSunShapeKVCache, SunShapeKVCache, _plan_key
 from .codec import PERM_MODES, SunShapeBlockCodec
 
 
@@ -50,6 +51,12 @@ def _transform_grouped(codec: SunShapeBlockCodec, q_grouped: torch.Tensor) -> to
     return q_grouped
 
 
+def _alive(refs, tensors) -> bool:
+    """Whether the weak references are to ``tensors``, one by one."""
+    return len(refs) == len(tensors) and \
+        all(map(operator.is_, map(weakref.ref.__call__, refs), tensors))
+
+
 def _prepared_decode(cache, ops: dict, codec: SunShapeBlockCodec, q: torch.Tensor,
                      kscale: float, perm, buffered: bool = False):
     """The cache's prepared matrix-core decode (``_hip.PreparedDecode``, or
@@ -67,12 +74,10 @@ def _prepared_decode(cache, ops: dict, codec: SunShapeBlockCodec, q: torch.Tenso
         tensors += (perm,)
     if buffered:  # the buffer stores (their windows move from call to call)
         tensors += (cache._key_buffer, cache._value_buffer)
-    # (a tensor may be given other memory in place, by set_ or .data)
     key = (kind, q.shape, q.dtype, q.device, kscale, ops.get("bits"), ops.get("group_size"),
-           buffered, *[t.data_ptr() for t in tensors])
+           buffered, _plan_key(tensors))
     held = getattr(cache, "_decode_prepared", None)
-    if held is not None and held[0] == key and len(held[1]) == len(tensors) and \
-            all(r() is t for r, t in zip(held[1], tensors)):
+    if held is not None and held[0] == key and _alive(held[1], tensors):
         return held[2]
     nb, nc = codec.n_blocks, codec.n_centroids
     bk = ops["buf_keys"] if buffered else None
@@ -100,10 +105,9 @@ def _fused_step(cache: SunShapeKVCache, queries: torch.Tensor, scale: float, cau
     tensors = (cache._key_indices, cache._values, codec.kernel_codebook(), codec.centroids)
     if perm is not None:
         tensors += (perm,)
-    key = ("step", q.shape, q.dtype, q.device, kscale, *[t.data_ptr() for t in tensors])
+    key = ("step", q.shape, q.dtype, q.device, kscale, _plan_key(tensors))
     held = getattr(cache, "_step_prepared", None)
-    if held is not None and held[0] == key and len(held[1]) == len(tensors) and \
-            all(r() is t for r, t in zip(held[1], tensors)):
+    if held is not None and held[0] == key and _alive(held[1], tensors):
         plan = held[2]
     else:
         try:
@@ -140,10 +144,9 @@ def _fused_hybrid_step(cache: HybridSunShapeKVCache, queries: torch.Tensor, scal
                                                cache._key_buffer, cache._value_buffer)
     if perm is not None:
         tensors += (perm,)
-    key = ("hstep", q.shape, q.dtype, q.device, kscale, *[t.data_ptr() for t in tensors])
+    key = ("hstep", q.shape, q.dtype, q.device, kscale, _plan_key(tensors))
     held = getattr(cache, "_hstep_prepared", None)
-    if held is not None and held[0] == key and len(held[1]) == len(tensors) and \
-            all(r() is t for r, t in zip(held[1], tensors)):
+    if held is not None and held[0] == key and _alive(held[1], tensors):
         plan = held[2]
     else:
         cb = codec.kernel_codebook()
@@ -183,19 +186,22 @@ def _fused_hybrid_step(cache: HybridSunShapeKVCache, queries: torch.Tensor, scal
 _MASKED_ROWS = 64
 
 
+_PLAIN_TYPES = frozenset((torch.Tensor, torch.nn.Parameter))
+
+
 def _plain(t) -> bool:
     """Whether ``t`` is an array whose memory a kernel may read and through
     which nothing is differentiated or batched: a learned bias, a dual number
     and vmap's wrappers keep the two-pass path, whose torch operations carry
     them."""
     return (isinstance(t, torch.Tensor)
-            and type(t) in (torch.Tensor, torch.nn.Parameter)
+            and type(t) in _PLAIN_TYPES
             and not (t.requires_grad and torch.is_grad_enabled())
             and _forward_ad._current_level < 0
             and not torch._C._functorch.is_functorch_wrapped_tensor(t))
 
 
-_KERNEL_TYPES = (torch.float16, torch.bfloat16, torch.float32)
+_KERNEL_TYPES = frozenset((torch.float16, torch.bfloat16, torch.float32))
 
 
 def _kernels_take(cache, queries: torch.Tensor, out_dtype: torch.dtype) -> bool:

@@ -18,6 +18,8 @@ capacity up front so a long decode never regrows.
 
 from __future__ import annotations
 
+import operator
+
 import torch
 
 from . import _hip
@@ -132,6 +134,16 @@ def _grouped_il_ok(codec: SunShapeBlockCodec, head_dim: int, bits: int, group_si
             and codec.n_centroids <= 256)
 
 
+def _plan_key(tensors) -> list:
+    """The addresses behind ``tensors`` (a tensor may be given other memory in
+    place, by set_ or .data)."""
+    return list(map(torch.Tensor.data_ptr, tensors))
+
+
+def _same(held, tensors) -> bool:
+    return len(held) == len(tensors) and all(map(operator.is_, held, tensors))
+
+
 class SunShapeKVCache:
     """Block-VQ keys + fp16 values; drop-in for mlx-lm's KVCache protocol
     (reference cache.py:59-336)."""
@@ -197,8 +209,7 @@ class SunShapeKVCache:
         _hip.require_gpu(keys, values)
         self.flush()
         self._ensure_capacity(b_, t_, keys.device)
-        plan = self._append_kv_plan()
-        if plan is not None:  # encode + value store, one launch per decode step
+        if self._appends_kv():  # encode + value store, one launch per decode step
             k = keys if keys.stride(-1) == 1 else keys.contiguous()
             v = values if values.stride(-1) == 1 else values.contiguous()
             if self.fuse_steps and self.lazy_fetch and self.offset > 0 and \
@@ -208,7 +219,7 @@ class SunShapeKVCache:
                 # held for the next attention call's fused step
                 self._pending = (k, v, k._version, v._version, self.offset)
             else:
-                plan(k, v, self.offset)
+                self._append_kv_plan()(k, v, self.offset)
         else:
             sl = slice(self.offset, self.offset + t_)
             _encode_into(self.codec, keys, self._key_indices[:, :, sl])
@@ -241,25 +252,23 @@ class SunShapeKVCache:
         k, v, pos = self._take_pending()
         self._append_kv_plan()(k, v, pos)
 
-    def _append_kv_plan(self):
-        """The prepared ``ss_append_kv_il8`` for the current buffers and
-        codebook (None where that path does not apply: non-interleaved
-        values, or codecs whose keys the HIP encoder does not take)."""
+    def _appends_kv(self) -> bool:
+        """Whether ``ss_append_kv_il8`` applies (not to non-interleaved
+        values, nor to codecs whose keys the HIP encoder does not take)."""
         c = self.codec
-        if not self.values_interleaved or c.mode != "profileperm_baseline" or c.n_centroids > 256:
-            return None
+        return self.values_interleaved and c.mode == "profileperm_baseline" and c.n_centroids <= 256
+
+    def _append_kv_plan(self):
+        """The prepared ``ss_append_kv_il8`` for the current buffers and codebook."""
+        c = self.codec
         cb, pm, pre = c.centroids, c.permutation, c.encode_codebook()
-        # (addresses too: a tensor may be given other memory in place)
-        key = (self._key_indices, self._values, cb, cb._version, pm,
-               pm._version if pm is not None else 0, pre,
-               self._key_indices.data_ptr(), self._values.data_ptr(), cb.data_ptr(),
-               pm.data_ptr() if pm is not None else 0)
+        tensors = tuple([t for t in (self._key_indices, self._values, cb, pm, pre) if t is not None])
+        key = _plan_key(tensors)
         held = self._append_plan
-        if held is None or len(held[0]) != len(key) or \
-                not all(a is b or (isinstance(a, int) and a == b) for a, b in zip(held[0], key)):
-            held = (key, _hip.PreparedAppend(pm, cb, pre, self._key_indices, self._values))
+        if held is None or held[1] != key or not _same(held[0], tensors):
+            held = (tensors, key, _hip.PreparedAppend(pm, cb, pre, self._key_indices, self._values))
             self._append_plan = held
-        return held[1]
+        return held[2]
 
     # ----------------------------------------------------------- accessors
     @property
@@ -612,15 +621,14 @@ class HybridSunShapeKVCache:
                 c.mode != "profileperm_baseline" or c.n_centroids > 256:
             return None
         cb, pm = c.centroids, c.permutation
-        key = (self._key_buffer, self._value_buffer, self._key_indices, self._values_il,
-               self._value_scales, self._value_zeros, cb, cb._version, pm,
-               pm._version if pm is not None else 0)
-        # (addresses too: a tensor may be given other memory in place)
-        key += tuple([t.data_ptr() for t in key if isinstance(t, torch.Tensor)])
+        tensors = (self._key_buffer, self._value_buffer, self._key_indices, self._values_il,
+                   self._value_scales, self._value_zeros, cb)
+        if pm is not None:
+            tensors += (pm,)
+        key = _plan_key(tensors)
         held = self._step_plan
-        if held is not None and len(held[0]) == len(key) and \
-                all(a is b or (isinstance(a, int) and a == b) for a, b in zip(held[0], key)):
-            return held[1]
+        if held is not None and held[1] == key and _same(held[0], tensors):
+            return held[2]
         gc = self._value_codec_impl
         for t in (self._key_buffer, self._value_buffer, self._key_indices, self._values_il,
                   self._value_scales, self._value_zeros):
@@ -637,7 +645,7 @@ class HybridSunShapeKVCache:
                       self._compressed_capacity),
             "fn": _hip.load_library().ss_hybrid_append_grouped_il,
         }
-        self._step_plan = (key, args)
+        self._step_plan = (tensors, key, args)
         return args
 
     def _held_step_ok(self, k: torch.Tensor, v: torch.Tensor, t_: int, n_flush: int) -> bool:
@@ -681,14 +689,15 @@ class HybridSunShapeKVCache:
 
     def flush(self) -> None:
         """Do a held decode step's buffer store and flush now: one
-        ss_hybrid_append_grouped_il launch for grouped values; for fp16
-        values the buffer store, then the flush of the oldest tokens as an
-        unheld step does it."""
+        ss_hybrid_append_grouped_il launch for grouped values; else (fp16
+        values, stores that launch does not take) the buffer store, then the
+        flush of the oldest tokens as an unheld step does it."""
         if self._pending is None:
             return
         k, v, tc, s0, n, nf = self._take_pending()
-        if self._grouped_il:
-            self._run_grouped_step(self._grouped_step_plan(), k, v, tc, s0, n, nf)
+        plan = self._grouped_step_plan()
+        if plan is not None:
+            self._run_grouped_step(plan, k, v, tc, s0, n, nf)
             return
         after = (self._compressed_offset, self._buffer_offset, self._buf_start)
         t_ = k.shape[2]
@@ -717,11 +726,10 @@ class HybridSunShapeKVCache:
         v = values if values.stride(-1) == 1 else values.contiguous()
         hold = n_flush <= self._buffer_offset and self._held_step_ok(k, v, t_, n_flush)
         plan = None
-        if self._grouped_il and 0 <= n_flush <= self._buffer_offset and t_ <= 64 and \
-                (n_flush > 0 or hold):
+        if self._grouped_il and not hold and 0 < n_flush <= self._buffer_offset and t_ <= 64:
             self._grow_compressed(b_, self._compressed_offset + n_flush, dev)
             plan = self._grouped_step_plan()
-        if hold and (plan is not None or self._fp16_il8):
+        if hold:
             # held for the next attention call's fused step (the counters
             # include it already; flush() stores it)
             self._grow_compressed(b_, self._compressed_offset + n_flush, dev)
@@ -730,7 +738,7 @@ class HybridSunShapeKVCache:
             self._compressed_offset += n_flush
             self._buffer_offset += t_ - n_flush
             self._buf_start = s0 + n_flush if self._buffer_offset else 0
-            self.last_value_quant_backend = "hip" if plan is not None else "fp16"
+            self.last_value_quant_backend = "hip" if self._grouped_il else "fp16"
         elif plan is not None and k.dtype == v.dtype:
             s0, n, tc = self._buf_start, self._buffer_offset, self._compressed_offset
             self._run_grouped_step(plan, k, v, tc, s0, n, n_flush)

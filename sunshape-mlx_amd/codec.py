@@ -58,9 +58,9 @@ def _compact_index_dtype(n_centroids: int) -> torch.dtype:
 
 def _seen(t: torch.Tensor | None):
     """What a result derived from ``t`` is kept with: the tensor, its version,
-    and an alias that holds its memory (while held, no other memory has that
-    address)."""
-    return None if t is None else (t, t._version, t.detach())
+    its address, and an alias that holds the memory (while held, no other has
+    that address)."""
+    return None if t is None else (t, t._version, t.data_ptr(), t.detach())
 
 
 def _unchanged(seen, t: torch.Tensor | None) -> bool:
@@ -68,7 +68,7 @@ def _unchanged(seen, t: torch.Tensor | None) -> bool:
     in place, or given other memory in place (by set_ or .data)."""
     if seen is None or t is None:
         return seen is t
-    return seen[0] is t and seen[1] == t._version and seen[2].data_ptr() == t.data_ptr()
+    return seen[0] is t and seen[1] == t._version and seen[2] == t.data_ptr()
 
 
 def _np(x) -> np.ndarray:
@@ -415,10 +415,11 @@ class SunShapeBlockCodec:
         when the centroids change (new tensor, memory or in-place update)."""
         c = self.scoring_centroids()
         cached = getattr(self, "_kernel_codebook", None)
-        if cached is None or not _unchanged(cached[0], c):
-            cached = (_seen(c), _hip.codebook_f16x2(c))
+        if cached is None or cached[0] is not c or cached[1] != c._version or \
+                cached[2] != c.data_ptr():
+            cached = (*_seen(c), _hip.codebook_f16x2(c))
             self._kernel_codebook = cached
-        return cached[1]
+        return cached[4]
 
     def encode_codebook(self, centroids: torch.Tensor | None = None) -> torch.Tensor | None:
         """The prepared codebook of the matrix-core encoder for ``centroids``
@@ -428,10 +429,11 @@ class SunShapeBlockCodec:
         if not _hip.encode_codebook_supported(c):
             return None
         cached = getattr(self, "_encode_codebook", None)
-        if cached is None or not _unchanged(cached[0], c):
-            cached = (_seen(c), _hip.encode_codebook(c))
+        if cached is None or cached[0] is not c or cached[1] != c._version or \
+                cached[2] != c.data_ptr():
+            cached = (*_seen(c), _hip.encode_codebook(c))
             self._encode_codebook = cached
-        return cached[1]
+        return cached[4]
 
     def _encode_centroids(self) -> torch.Tensor:
         if self.mode == "profileperm_localmetric_dsq":
