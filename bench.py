@@ -328,8 +328,9 @@ def run_prefill(args) -> int:
     """Prefill: one prompt of T tokens (B=1, 32 query / 8 KV heads, D=128)
     attended causally against the cache that holds the same T tokens (u8
     key indices, fp16 values 8-token interleaved), as mlx-lm's prefill does
-    after update_and_fetch: sunshape_sdpa(q, cache, scale, mask="causal"),
-    whose fused path is one ss_prefill_attn_il8 launch.  Reported
+    after update_and_fetch.  The kernel timed is ss_prefill_attn_il8, the
+    entry point that needs no workspace; sunshape_sdpa(q, cache, scale,
+    mask="causal") takes ss_prefill_attn for a prompt of this length.  Reported
     as µs per prompt and attention TFLOP/s (QK^T and P.V over the causal
     half, 4 * B * Hq * D * T^2 / 2 flops); the decode-shaped kernel's time on
     the same prompt is reported beside it."""

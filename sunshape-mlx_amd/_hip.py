@@ -1252,7 +1252,8 @@ def prefill_attn_il8_hybrid(q: torch.Tensor, scale: float, perm: torch.Tensor | 
                             values_il8: torch.Tensor, t_kv: int, kraw: torch.Tensor,
                             kfac: torch.Tensor, t_raw0: int, causal: bool = True,
                             q_offset: int = 0, out_dtype: torch.dtype | None = None) -> torch.Tensor:
-    """:func:`prefill_attn_il8` over a hybrid cache (``ss_prefill_attn_il8_hybrid``):
+    """:func:`prefill_attn_il8` over a hybrid cache (``ss_prefill_attn_il8_hybrid``;
+    ``sunshape_sdpa`` takes :func:`prefill_attn` for these, this form is for direct callers):
     positions below ``t_raw0`` scored from ``idx``, the rest from the whole
     keys ``kraw`` (B, Hkv, t_kv - t_raw0, 2, 128) fp16 with factors ``kfac``
     (B, Hkv, t_kv - t_raw0) float32 (:func:`raw_key_rows`); ``values_il8``

@@ -330,7 +330,10 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
                                         codec.n_centroids, ops["idx"], v8, t_kv, causal=causal,
                                         q_offset=q_offset, out_dtype=out_dtype)
             elif kind == "il8" and _hip.prefill_supported(hq, cache.n_kv_heads, tq, d,
-                                                          codec.n_blocks):  # float32 queries
+                                                          codec.n_blocks):
+                # float32 queries, and 16-bit prompts below the rule's line, on
+                # the kernel they had before it (36 to 59 us for 32 to 200
+                # tokens; the rule weighs the other two: decode 13 to 22)
                 out = _hip.prefill_attn_il8(q, kscale, perm, codec.kernel_codebook(),
                                             codec.n_centroids, ops["idx"], ops["values"], t_kv,
                                             causal=causal, q_offset=q_offset,

@@ -146,8 +146,8 @@ static int turboquant_mfma_decode(
     const ss_attn_mask *mask, void *stream) {
     const float *cents = static_cast<const float *>(codebook);
     // fused: the kernel writes out itself, rotated (one split, or its
-    // in-kernel merge); else split partials that transformed_decode merges
-    // with the buffer's partial and rotates
+    // in-kernel merge); else split partials for transformed_decode's merge,
+    // which attends the buffered tokens, adds them and rotates
     auto launch_tq = [&](const DecodeCommon &c0, const DecodeShape &s, hipStream_t st,
                          bool fused) -> int {
         DecodeCommon c = c0;

@@ -273,8 +273,9 @@ static int grouped_checks(int head_dim, const uint32_t *packed, const void *scal
 }
 
 // Workspace of the TurboQuant decode: the split partials (as for the other
-// VALU decodes, plus one slot per column for buffered tokens), then the fp32
-// output rows of the rotated basis.
+// VALU decodes), then the fp32 output rows of the rotated basis.  A buffer
+// adds a slot per column: nothing is stored there, it makes a single split
+// write its partial for the merge, which attends the buffered tokens itself.
 static DecodeShape with_buffer_slot(DecodeShape s, int64_t t_buf) {
     if (t_buf > 0) s.S += 1;
     return s;

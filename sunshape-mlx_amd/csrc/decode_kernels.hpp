@@ -75,9 +75,9 @@ struct DecodeCore {
     const float *rot = nullptr;
 };
 // With the attention mask.  Matrix-core kernels that take no mask are passed
-// the core alone: with five more fields among their arguments the 2-bit
-// grouped step of 8 x 32768 tokens loaded them in smaller pieces and took
-// 41.1 us instead of 40.6.
+// the core alone: no argument that they do not read (the 2-bit grouped step of
+// 8 x 32768 tokens: 41.1 us with the mask's five fields, 41.0 without, which
+// is the runs' own difference).
 struct DecodeCommon : DecodeCore {
     // element (b, head, query position, key position t) at
     // mask[b*m_sb + head*m_sh + q*m_sq + t], kMask* type (kMaskNone: none)
@@ -1745,7 +1745,7 @@ struct VTq {
     static constexpr int kSub = 1;
     static constexpr int kCodeBytes = kCodeBytes1;
     static constexpr int kSzBytes = kSzBytes1;
-    static constexpr bool kHybridBuffer = false;  // the buffer joins as its own rotated partial
+    static constexpr bool kHybridBuffer = false;  // the buffer joins in the merge
     static constexpr bool kHeavyCapable = true;
     static constexpr int kTileV = kCodeBytes + 1024;
     static constexpr int kLoadsV = kCodeBytes / 1024 + 1;

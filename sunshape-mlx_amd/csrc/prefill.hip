@@ -29,7 +29,9 @@
 // (its own online softmax and accumulators), so there is no split, merge or
 // cross-wave combine.  Causal rows stop at q_offset + position.
 //
-// fp16 and bf16 queries take prefill32_il8_kernel instead: waves of 32 rows on
+// fp16 and bf16 queries take prefill32_il8_kernel instead (of the package's own
+// prompts only those too short for the kernel of prefill_frag.hip; longer
+// ones and those with whole keys come from direct callers): waves of 32 rows on
 // v_mfma_f32_32x32x16_f16 (S^T of 32 tokens x 32 rows: lane l holds token
 // l%32's block 2ks + l/32 as A, row l%32's dims 16ks + 8(l/32) .. as B) and
 // v_mfma_f32_32x32x16_f16 for P.V too (the S^T accumulator entries 8k2 ..

@@ -25,7 +25,7 @@
 // the exponentials taken out the rest takes 75, 89 and 93 % of the time.
 // 32/8 heads of 128 dims, prefill32 before: 4096 tokens 335 -> 258 us (533
 // TFLOP/s of attention), 2 x 512 tokens after 8192 367 -> 280 us; bf16 values,
-// 2041 tokens, 1146 us on the vector-ALU decode before, 119 now.
+// 2041 tokens, 1146 us on the vector-ALU decode before, 119 to 127 now.
 //
 // Values: fp16, P as one fp16 operand of p * 2^11 (as prefill32) or as its hi
 // and lo parts (22 bits, as the decode kernels; ss_prefill_attn chooses), or
