@@ -2169,7 +2169,8 @@ __device__ __forceinline__ f16x4 ds_read_tr16_at(uint32_t addr) {
 // over distinct banks (the permutation stays inside a row, so the copies stay
 // coalesced).  HBM bounds it, as VIl8.  B=4, T=8003, 32/8 heads of 128 dims,
 // per dispatch under the profiler: 26.9 us and a 3.9 us merge launch on the
-// vector ALUs, 24.3 us here (69.7 MB, 2.9 TB/s).
+// vector ALUs, 24.8 us here (69.7 MB, 2.8 TB/s; 24.3 before infinite values
+// were kept).
 template <int D>
 struct VBf16 {
     struct Args {
