@@ -301,12 +301,13 @@ def _fused(cache, queries: torch.Tensor, scale: float, causal: bool, q_offset: i
     if buffered and codec.mode not in PERM_MODES and codec.use_rotation:
         # the kernels score buffered keys against the query they are given,
         # here the rotated one: (q R^T) . (k R^T) = q . k for orthogonal R,
-        # so the buffer's keys go in rotated (float32, with float32 values
-        # to share their layout)
+        # so the buffer's keys go in rotated (float32, with float32 values in
+        # one tensor with them: contiguous() leaves the strides of a single
+        # sequence or head as they were, and the two have to agree)
         nb_ = buffered
-        ops = dict(ops, buf_keys=(ops["buf_keys"][:, :, :nb_].float()
-                                  @ codec.rotation.t()).contiguous(),
-                   buf_values=ops["buf_values"][:, :, :nb_].float().contiguous())
+        bk, bv = torch.stack((ops["buf_keys"][:, :, :nb_].float() @ codec.rotation.t(),
+                              ops["buf_values"][:, :, :nb_].float()))
+        ops = dict(ops, buf_keys=bk, buf_values=bv)
     t_kv = cache.compressed_offset if isinstance(cache, HybridSunShapeKVCache) else cache.offset
     kind = ops["kind"]
     # a prompt (many query rows per head) against an fp16 cache: keys

@@ -572,6 +572,31 @@ def test_query_layouts_and_types_of_the_two_pass_path(backend, bits, dtype, d, b
     assert grads[0] is grads[1] is None or torch.equal(*grads)
 
 
+@pytest.mark.parametrize("backend,bits,dtype,d,masked", [
+    ("fp16", 0, torch.float16, 128, True), ("grouped", 4, torch.float32, 64, True),
+    ("turboquant", 4, torch.float16, 96, True), ("turboquant", 2, torch.bfloat16, 128, False),
+    ("grouped", 2, torch.float16, 128, False)])
+@pytest.mark.parametrize("hkv", [1, 2])
+def test_rotated_hybrids_of_one_head(backend, bits, dtype, d, masked, hkv):
+    """Buffered tokens of a rotated codec's cache, of one sequence and one KV
+    head (size-1 dims, whose strides contiguous() leaves alone) or two."""
+    rng = np.random.default_rng(d)
+    codec = S.SunShapeBlockCodec(d, device="cuda", mode="rotated")
+    codec.load_state_dict({"centroids": rng.standard_normal((d // 8, 256, 8)).astype(np.float32),
+                           "rotation": np.linalg.qr(rng.standard_normal((d, d)))[0].astype(np.float32)})
+    cache = S.create_kv_cache(codec, n_kv_heads=hkv, dtype=dtype, value_backend=backend,
+                              value_bits=bits or None, buffer_size=50,
+                              value_group_size=32)
+    g = torch.Generator(device="cuda").manual_seed(d)
+    k, v = torch.randn((2, 1, hkv, 130, d), generator=g, device="cuda").to(dtype)
+    cache.update_and_fetch(k, v)
+    q = torch.randn((1, 4 * hkv, 3, d), generator=g, device="cuda").to(dtype)
+    mask = torch.arange(130, device="cuda") != 9 if masked else "causal"
+    ref = attention._two_pass(cache, q, 0.1, mask, torch.float32)
+    got = S.sunshape_sdpa(q, cache, 0.1, mask)
+    assert rel_err(got.float().cpu().numpy(), ref.cpu().numpy()) <= REL_TOL + torch.finfo(dtype).eps
+
+
 @pytest.mark.parametrize("bdt,t_buf", [(torch.float16, 1), (torch.float32, 127), (torch.bfloat16, 131)])
 def test_merge_keeps_an_infinite_value_of_the_last_buffered_token(bdt, t_buf):
     """One dim of the last token is infinite: infinite in the output, the
