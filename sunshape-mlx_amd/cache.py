@@ -134,6 +134,13 @@ def _grouped_il_ok(codec: SunShapeBlockCodec, head_dim: int, bits: int, group_si
             and codec.n_centroids <= 256)
 
 
+def _step_rows(k: torch.Tensor) -> bool:
+    """Whether the one-launch decode steps take new keys laid out as ``k``:
+    rows (and, sharing their strides, the values') that start on 16 bytes."""
+    s = k.stride()
+    return (s[0] | s[1] | s[2]) % 8 == 0 and s[2] >= k.shape[3] and k.data_ptr() % 16 == 0
+
+
 def _plan_key(tensors) -> list:
     """The addresses behind ``tensors`` (a tensor may be given other memory in
     place, by set_ or .data)."""
@@ -215,7 +222,7 @@ class SunShapeKVCache:
             if self.fuse_steps and self.lazy_fetch and self.offset > 0 and \
                     1 <= t_ <= _hip.MAX_STEP_TOKENS and k.dtype == torch.float16 and \
                     v.dtype == torch.float16 and k.stride()[:3] == v.stride()[:3] and \
-                    tuple(v.shape) == tuple(k.shape):
+                    tuple(v.shape) == tuple(k.shape) and _step_rows(k):
                 # held for the next attention call's fused step
                 self._pending = (k, v, k._version, v._version, self.offset)
             else:
@@ -662,7 +669,8 @@ class HybridSunShapeKVCache:
                 1 <= t_ <= _hip.MAX_STEP_TOKENS and n_flush <= _hip.MAX_STEP_TOKENS and
                 k.dtype == torch.float16 and v.dtype == torch.float16 and
                 k.stride(-1) == 1 and v.stride(-1) == 1 and
-                k.stride()[:3] == v.stride()[:3] and tuple(v.shape) == tuple(k.shape))
+                k.stride()[:3] == v.stride()[:3] and tuple(v.shape) == tuple(k.shape) and
+                _step_rows(k))
 
     def _run_grouped_step(self, plan, k, v, tc: int, s0: int, n: int, n_flush: int) -> None:
         """One ss_hybrid_append_grouped_il launch: the new tokens stored at

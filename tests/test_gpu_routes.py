@@ -220,6 +220,23 @@ def test_steps_follow_memory_given_in_place(backend, bits, buffer, stores, held)
     assert not any(bool(t.any()) for t in old)
 
 
+@pytest.mark.parametrize("backend,bits,d,buffer", [
+    ("fp16", 0, 64, 128), ("fp16", 0, 128, 20), ("grouped", 4, 128, 20)])
+def test_steps_of_unaligned_rows(backend, bits, d, buffer):
+    """New keys and values as slices of wider rows, at addresses and strides
+    the one-launch step does not take: as contiguous ones."""
+    g = torch.Generator(device="cuda").manual_seed(d)
+    wide = torch.randn((2, 1, 2, 1, d + 3), generator=g, device="cuda").half()
+    q = torch.randn((1, 8, 1, d), generator=g, device="cuda").half()
+    outs = []
+    for k, v in (wide[..., 1:d + 1], wide[..., 1:d + 1].contiguous()):
+        cache = _masked_cache(backend, bits, torch.float16, d, 2, 1, 300, buffer)
+        cache.update_and_fetch(k, v)
+        outs += [S.sunshape_sdpa(q, cache, 0.11), cache.key_indices, cache.values]
+    assert torch.equal(outs[1], outs[4]) and torch.equal(outs[2], outs[5])
+    assert rel_err(outs[0].float().cpu().numpy(), outs[3].float().cpu().numpy()) <= REL_TOL
+
+
 def test_masks_that_carry_gradients_keep_the_two_pass_path():
     """A learned bias gets its gradient, a dual bias its tangent and vmap its
     batch: equal to the two-pass path's, and the same values as the fused
