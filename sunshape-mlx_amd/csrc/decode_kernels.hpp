@@ -1235,6 +1235,7 @@ struct VIl8Hyb : VIl8<D> {
     };
     static constexpr bool kHybridBuffer = true;
     static constexpr bool kHeavyCapable = true;
+    static constexpr bool kKeepsInf = true;
 };
 
 // VIl8 for one decode step that also appends its tokens: the cache holds
@@ -1364,6 +1365,7 @@ struct VGil {
     static constexpr int kCodeBytes = kSub * kCodeBytes1;
     static constexpr int kSzBytes = kSub * kSzBytes1;
     static constexpr bool kHybridBuffer = true;  // hybrid caches: recent tokens join the pass
+    static constexpr bool kKeepsInf = true;      // (of buffered tokens)
     // fp16 heavy key dims: on the private-ring shapes (the loader-wave shape
     // has no registers to spare for them)
     static constexpr bool kHeavyCapable = kPrivateRing;
@@ -1662,6 +1664,7 @@ struct VGilStep : VGil<D, BITS, NG, SZT> {
     };
     static constexpr bool kStepShare = true;
     static constexpr bool kHybridStep = true;
+    static constexpr bool kKeepsInf = false;  // (8 x 32768 tokens: 41.4 us, 41.7 with the share's part)
     static constexpr bool kStepQuant = true;  // the flushed values are quantised
     static constexpr bool kHeavyCapable = false;
     static constexpr int kBits = BITS;
@@ -2654,6 +2657,10 @@ __global__ void __launch_bounds__((VF::kPrivateRing ? NC : NC + 1) * kWave)
                                 kc[j][k] = hk_raw[j][k];
                                 vc[j][k] = hv_raw[j][k];
                             }
+                            // (past the share's end its last row again, with
+                            // p = 0, which an infinite value would make NaN)
+                            if constexpr (MK || VfKeepsInf<VF>::value)
+                                vc[j][k] = c0 + j < n_sh ? vc[j][k] : (unsigned short)0;
                         }
                     float sc[NSH][R];
 #pragma unroll

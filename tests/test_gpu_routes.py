@@ -691,3 +691,34 @@ def test_bf16_prompts_keep_infinite_values(backend, d, t_q, buffer):
         assert bool((got[:, :, tok:, dim] == x).all()), dim
         got[..., dim] = plain[..., dim]
     assert torch.equal(got, plain)
+
+
+@pytest.mark.parametrize("backend,bits,dtype,d,t_q,masked", [
+    ("grouped", 2, torch.bfloat16, 64, 1, True), ("grouped", 4, torch.float16, 128, 3, True),
+    ("fp16", 0, torch.float16, 128, 1, True), ("fp16", 0, torch.float16, 128, 40, False),
+    ("grouped", 2, torch.float16, 128, 40, False)])
+def test_hybrids_keep_infinite_values(backend, bits, dtype, d, t_q, masked):
+    """An infinite value of a buffered token (the buffer's last, and one
+    inside) or, as fp16, of a stored one: infinite in its dim for the rows that
+    see it, the other dims as without it."""
+    t_kv, buffer = 777, 20
+    cache = _masked_cache(backend, bits, dtype, d, 2, 1, t_kv, buffer)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q = torch.randn((1, 8, t_q, d), generator=g, device="cuda").to(dtype)
+    mask = torch.arange(t_kv, device="cuda") != 9 if masked else "causal"
+    plain = S.sunshape_sdpa(q, cache, 0.02, mask)
+    first = t_kv if masked else t_kv - t_q  # the first key that row 0 does not see, less one
+    toks = {7: t_kv - 1, 20: t_kv - 9}
+    if backend == "fp16":
+        toks[40] = 400
+    for dim, tok in toks.items():
+        if tok >= cache.compressed_offset:
+            cache._value_buffer[:, :, cache._buf_start + tok - cache.compressed_offset, dim] = torch.inf
+        else:
+            cache._values_il8[:, :, tok // 8, dim, tok % 8] = torch.inf
+    cache._version += 1
+    got = S.sunshape_sdpa(q, cache, 0.02, mask)
+    for dim, tok in toks.items():
+        assert bool((got[:, :, max(tok - first, 0):, dim] == torch.inf).all()), dim
+        got[..., dim] = plain[..., dim]
+    assert torch.equal(got, plain)
